@@ -103,14 +103,18 @@ struct KParams {
 };
 
 // Stride of the population planes of a lattice of N nodes with rsz-byte
-// reals.  Planes whose byte size is a multiple of 64 KiB would start at the
+// reals.  Every plane starts on a multiple of 64 elements: the 64 consecutive
+// nodes a wave of the linear grid stores are then whole cache lines in all
+// planes (with stride N a plane of 78^3 floats starts 32 bytes into a line).
+// Planes whose byte size is a multiple of 64 KiB would start at the
 // same offset modulo large powers of two, and the 38 streams of a step then
 // collide on the same memory channels (a copy of 38 planes at 512^3: 4.72
 // TB/s with stride N, 5.34 TB/s padded).  The pad (4160 elements) keeps the
 // planes 256-byte aligned.
 inline int64_t plane_stride(int64_t N, int64_t rsz)
 {
-    return (N * rsz) % 65536 == 0 ? N + 4160 : N;
+    const int64_t S = (N + 63) / 64 * 64;
+    return (S * rsz) % 65536 == 0 ? S + 4160 : S;
 }
 
 inline void fill_float_params(KParams &P)
@@ -180,6 +184,58 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb)
     const uint32_t x = b % 8u, q = nb / 8u, r = nb % 8u;
     return x * q + (x < r ? x : r) + b / 8u;
 }
+
+// The same in groups of 64 blocks: each XCD takes 8 neighbouring blocks of a
+// group, and all XCDs stay within the same group (RUN_GROUP); RUN_ALL is the
+// order above, one contiguous range per XCD for the whole launch.
+enum { RUN_ALL = 0, RUN_GROUP = 8 };
+__device__ __forceinline__ uint32_t xcd_run(int run, uint32_t b, uint32_t nb)
+{
+    if (run == RUN_ALL) return xcd_block(b, nb);
+    const uint32_t base = b & ~63u, r = b & 63u, rem = nb - base;
+    return base + (rem >= 64u ? (r & 7u) * 8u + (r >> 3) : xcd_block(r, rem));
+}
+
+// linear index of the calling block, in dispatch order
+__device__ __forceinline__ uint32_t block_linear()
+{
+    return blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+}
+
+// Block order and kind of stores of a step over a state of `bytes` (both
+// buffers of every population set).
+//
+// Cached: the 256 MB last-level cache (and the L2s) hold the state from step
+// to step.  Plain loads and stores, and one contiguous range per XCD: a range
+// is then in the L2 of the XCD that wrote it, neighbouring tiles share halo
+// lines there, and lines that two waves write in part are merged there.
+// Rayleigh-Benard, float, us per step, round-robin order with non-temporal
+// loads (and, two steps per launch, stores) -> this: 256x128 4.65 -> 3.46,
+// 512x256 7.1 -> 5.3, 969x485 37.7 -> 15.8, 1024x512 22.5 -> 16.9; one step
+// per launch 64^3 18.4 -> 13.7, 78^3 35.4 -> 23.5; channel 78^3 18.1 -> 12.4,
+// 113^3 (219 MB) 43.6 -> 34.1, 128^3 (319 MB) 61.4 -> 56.0.
+//
+// Streamed: non-temporal stores where a wave's store is whole lines (linear
+// order, or rows of whole lines); 3-D row and linear grids in groups, so that
+// all XCDs work on the same planes of memory (256^3 988 -> 949 us; in eight
+// ranges 1000).  2-D tiles keep the eight ranges up to 1 GiB (2047x1021 102
+// -> 84, 2048x1024 85 -> 83; 4096x2048: 310 round-robin, 325 ranges, 301
+// groups).  FP64 (one step per launch): ranges up to 1.5 GiB, 2048x1024 280
+// -> 251, 128^3 265 -> 248; beyond in groups, 200^3 962 -> 947.
+constexpr int64_t CACHED_BYTES = (int64_t)320 << 20;
+struct StepOrder {
+    bool nts;  // non-temporal stores
+    int run;   // xcd_run
+};
+inline StepOrder step_order(int64_t bytes, bool whole_lines, int64_t range_bytes)
+{
+    return {bytes > CACHED_BYTES && whole_lines, bytes <= range_bytes ? RUN_ALL : RUN_GROUP};
+}
+inline int64_t state_bytes(const KParams &P, int64_t rsz)
+{
+    return 2 * (int64_t)Q * P.N * rsz * ((P.fluid ? 1 : 0) + (P.thermal ? 1 : 0));
+}
+constexpr int64_t RANGE_BYTES_2D = (int64_t)1 << 30, RANGE_BYTES_64 = (int64_t)3 << 29;
 
 // compile-time loop over q
 template <int q, int Q_, typename F>
@@ -361,13 +417,13 @@ inline int64_t batch2_tiles(int NX, int NY) { return (int64_t)((NX + 63) / 64) *
 enum { BATCH_FLUID = 1, BATCH_THERMAL = 2, BATCH_FLUID_THERMAL = 3 };
 // gen: some lattice of the launch uses the HIT / LES / two-way paths
 void launch_batch_fp32(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
-                       bool dense, bool gen, int arith64, bool ntl, hipStream_t s);
+                       bool dense, bool gen, int arith64, StepOrder order, hipStream_t s);
 void launch_batch_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
-                       bool dense, hipStream_t s);
+                       bool dense, StepOrder order, hipStream_t s);
 // two steps per launch for 2-D float-storage lattices (two_step_ok); nblocks
 // = 64 x 4 tiles of the launch
 void launch_batch2_fp32(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
-                        int arith64, bool ntl, hipStream_t s);
+                        int arith64, StepOrder order, hipStream_t s);
 
 // Kernel launchers (stream-ordered).
 void launch_step_fp64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,

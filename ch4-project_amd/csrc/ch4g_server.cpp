@@ -32,7 +32,7 @@ struct Batch {
         int dev32, arith64, kind;
         bool dense;                       // lanes decode their own rows (dense_rows)
         bool gen;                         // LES lattices (the kernel instance with those paths)
-        bool ntl;
+        StepOrder order;                  // block order and stores, by the group's state bytes
         bool two;                         // two steps per launch (k_step2_batch32)
         int first, count;                 // range in the entry table
         int nlaunch;                      // launches of the group per chunk
@@ -169,6 +169,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         G.first = (int)B.host.size();
         G.count = 0;
         int64_t bytes = 0;
+        bool whole_lines = true;
         // members of the group and their launches per chunk (two-step
         // groups: pairs, then the single step of an odd share)
         size_t i1 = i;
@@ -205,6 +206,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
             npair.push_back(G.two ? st / 2 : 0);
             ntile.push_back(G.two ? batch2_tiles(L->cfg.NX, L->cfg.NY) : batch_tiles(L->cfg.NX, L->cfg.NY, L->cfg.NZ));
             bytes += 2 * (int64_t)Q * L->N * (L->dev32 ? 4 : 8) * ((L->base.fluid ? 1 : 0) + (L->base.thermal ? 1 : 0));
+            whole_lines = whole_lines && (G.dense || L->cfg.NX * (L->dev32 ? 4 : 8) % 128 == 0);
             G.count++;
         }
         G.off.assign((size_t)KG, 0);
@@ -229,8 +231,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
             G.nblk[(size_t)k] = t0;
             B.slots.push_back({0u, (uint32_t)t0}); // sentinel
         }
-        // non-temporal loads when the group's lattices fit the last-level cache
-        G.ntl = bytes <= ((int64_t)192 << 20);
+        G.order = step_order(bytes, whole_lines, G.two ? RANGE_BYTES_2D : G.dev32 ? CACHED_BYTES : RANGE_BYTES_64);
         B.groups.push_back(G);
     }
     if (!B.stream) HIPCHK(hipStreamCreateWithFlags(&B.stream, hipStreamNonBlocking));
@@ -321,11 +322,11 @@ int launch_steps(Batch &B)
             const BatchSlot *sl = B.dev_slots + G.off[(size_t)k];
             const int ns = G.nslot[(size_t)k];
             if (G.two)
-                launch_batch2_fp32(tab, sl, ns, nt, G.kind, G.arith64, G.ntl, st);
+                launch_batch2_fp32(tab, sl, ns, nt, G.kind, G.arith64, G.order, st);
             else if (G.dev32)
-                launch_batch_fp32(tab, sl, ns, nb, G.kind, G.dense, G.gen, G.arith64, G.ntl, st);
+                launch_batch_fp32(tab, sl, ns, nb, G.kind, G.dense, G.gen, G.arith64, G.order, st);
             else
-                launch_batch_fp64(tab, sl, ns, nb, G.kind, G.dense, st);
+                launch_batch_fp64(tab, sl, ns, nb, G.kind, G.dense, G.order, st);
         }
     }
     for (size_t g = 1; g < ng; g++) {

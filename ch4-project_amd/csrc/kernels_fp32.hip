@@ -20,25 +20,10 @@ namespace ch4g {
 
 namespace {
 
-// Population planes are streamed: every value is read once and written once
-// per step.  Stores are always non-temporal; loads are non-temporal when the
-// two lattices fit the last-level cache (measured faster there), plain
-// otherwise (x-shifted reads of neighbouring wavefronts share L2 lines).
-template <bool NTL>
-__device__ __forceinline__ float ldp(const float *p)
-{
-    if constexpr (NTL)
-        return __builtin_nontemporal_load(p);
-    else
-        return *p;
-}
-
-// Stores are non-temporal except where the single-step kernels update a
-// lattice resident in the last-level cache (NT = false there: the next
-// step's reads then find the state in the cache; channel 78^3 21.6 -> 18.8
-// us per step, while the two-step kernel and streamed lattices are faster
-// with non-temporal stores: 512x256 7.24 vs 7.45 us, 256^3 957 vs 999 us).
-template <bool NT = true>
+// Every population value is read once and written once per step.  Stores are
+// non-temporal (NT) where step_order says so; loads are plain: x-shifted
+// reads of neighbouring waves share cache lines.
+template <bool NT>
 __device__ __forceinline__ void stp(float *p, float v)
 {
     if constexpr (NT)
@@ -114,7 +99,7 @@ __device__ __forceinline__ void force_at32(const KParams &P, const HitTable &tab
 // Streaming of the previous step (pull) with halfway bounce-back at y walls.
 // Branch-free: every load address is computed first (wall crossings are a
 // wave-uniform select), so all 19 loads are in flight together.
-template <bool FIRST, bool NTL>
+template <bool FIRST>
 __device__ __forceinline__ void gather_f32(const KParams &P, const Row &R, const Nbr &b, const float *__restrict__ in,
                                            uint32_t n, float f[Q])
 {
@@ -122,12 +107,12 @@ __device__ __forceinline__ void gather_f32(const KParams &P, const Row &R, const
     static_for<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         if constexpr (FIRST) {
-            f[q] = ldp<NTL>(in + (size_t)q * N + n);
+            f[q] = in[(size_t)q * N + n];
         } else {
             const bool cross = P.wall_f && crosses_wall<q>(b);
             const float *base = in + (size_t)(cross ? invq(q) : q) * N;
             const uint32_t off = cross ? n : src_index<q>(b, P.NX, P.NY);
-            float v = ldp<NTL>(base + off);
+            float v = base[off];
             if constexpr (cyq(q) > 0) v = fmaf(wf(q), cross ? 0.f : R.dr_up, v);
             if constexpr (cyq(q) < 0) v = fmaf(wf(q), cross ? 0.f : R.dr_dn, v);
             f[q] = v;
@@ -136,7 +121,7 @@ __device__ __forceinline__ void gather_f32(const KParams &P, const Row &R, const
 }
 
 // Fixed-T y walls: same-direction population + w 2((T_w - T_ref) - T_lag).
-template <bool FIRST, bool NTL>
+template <bool FIRST>
 __device__ __forceinline__ void gather_g32(const KParams &P, const Row &R, const Nbr &b, const float *__restrict__ in,
                                            uint32_t n, float dTlag, float g[Q])
 {
@@ -146,11 +131,11 @@ __device__ __forceinline__ void gather_g32(const KParams &P, const Row &R, const
     static_for<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         if constexpr (FIRST) {
-            g[q] = ldp<NTL>(in + (size_t)q * N + n);
+            g[q] = in[(size_t)q * N + n];
         } else {
             const bool cross = P.wall_t && crosses_wall<q>(b);
             const uint32_t off = cross ? n : src_index<q>(b, P.NX, P.NY);
-            float v = ldp<NTL>(in + (size_t)q * N + off);
+            float v = in[(size_t)q * N + off];
             if constexpr (cyq(q) > 0) v = fmaf(wf(q), cross ? fac_bot : R.dt_up, v);
             if constexpr (cyq(q) < 0) v = fmaf(wf(q), cross ? fac_top : R.dt_dn, v);
             g[q] = v;
@@ -161,13 +146,11 @@ __device__ __forceinline__ void gather_g32(const KParams &P, const Row &R, const
 // The same gathers with 32-bit byte offsets from the array base (arrays of
 // less than 4 GiB): a load is the array's scalar base plus one 32-bit vector
 // offset instead of a 64-bit address per lane and population.
-template <bool NTL>
 __device__ __forceinline__ float ldo(const float *base, uint32_t byteoff)
 {
-    return ldp<NTL>((const float *)((const char *)base + byteoff));
+    return *(const float *)((const char *)base + byteoff);
 }
 
-template <bool NTL>
 __device__ __forceinline__ void gather_f32_o32(const KParams &P, const Row &R, const Nbr &b,
                                                const float *__restrict__ in, uint32_t n, float f[Q])
 {
@@ -176,14 +159,13 @@ __device__ __forceinline__ void gather_f32_o32(const KParams &P, const Row &R, c
         constexpr int q = decltype(qc)::value;
         const bool cross = P.wall_f && crosses_wall<q>(b);
         const uint32_t off = cross ? (uint32_t)invq(q) * S4 + n * 4u : (uint32_t)q * S4 + src_index<q>(b, P.NX, P.NY) * 4u;
-        float v = ldo<NTL>(in, off);
+        float v = ldo(in, off);
         if constexpr (cyq(q) > 0) v = fmaf(wf(q), cross ? 0.f : R.dr_up, v);
         if constexpr (cyq(q) < 0) v = fmaf(wf(q), cross ? 0.f : R.dr_dn, v);
         f[q] = v;
     });
 }
 
-template <bool NTL>
 __device__ __forceinline__ void gather_g32_o32(const KParams &P, const Row &R, const Nbr &b,
                                                const float *__restrict__ in, uint32_t n, float dTlag, float g[Q])
 {
@@ -194,7 +176,7 @@ __device__ __forceinline__ void gather_g32_o32(const KParams &P, const Row &R, c
         constexpr int q = decltype(qc)::value;
         const bool cross = P.wall_t && crosses_wall<q>(b);
         const uint32_t off = (uint32_t)q * S4 + (cross ? n : src_index<q>(b, P.NX, P.NY)) * 4u;
-        float v = ldo<NTL>(in, off);
+        float v = ldo(in, off);
         if constexpr (cyq(q) > 0) v = fmaf(wf(q), cross ? fac_bot : R.dt_up, v);
         if constexpr (cyq(q) < 0) v = fmaf(wf(q), cross ? fac_top : R.dt_dn, v);
         g[q] = v;
@@ -280,13 +262,14 @@ struct NodeOut {
 };
 
 // NodeOut with 32-bit byte offsets (arrays of less than 4 GiB)
+template <bool NT>
 struct NodeOut32 {
     float *__restrict__ f;
     float *__restrict__ g;
     float *__restrict__ tlag;
     uint32_t n4, S4;  // byte offset of the node, plane stride in bytes
-    __device__ void put_f(int q, float v) const { stp((float *)((char *)f + ((uint32_t)q * S4 + n4)), v); }
-    __device__ void put_g(int q, float v) const { stp((float *)((char *)g + ((uint32_t)q * S4 + n4)), v); }
+    __device__ void put_f(int q, float v) const { stp<NT>((float *)((char *)f + ((uint32_t)q * S4 + n4)), v); }
+    __device__ void put_g(int q, float v) const { stp<NT>((float *)((char *)g + ((uint32_t)q * S4 + n4)), v); }
     __device__ void put_tlag(float v) const { *(float *)((char *)tlag + n4) = v; }
     __device__ float get_tau() const { return 0.f; }  // no LES on the two-step path
     __device__ void put_tau(float) const {}
@@ -540,7 +523,7 @@ __device__ __forceinline__ void collide_thermal(const KParams &P, const Row &R, 
 // batched kernel, so a lattice advances bit-identically in either.
 // A = arithmetic type of the collision (float for CH4G_FP32_DEV, double for
 // CH4G_FP32_STORE); storage is float in both.
-template <bool FIRST, bool FLUID, bool THERMAL, typename A, bool NTL, bool GEN>
+template <bool FIRST, bool FLUID, bool THERMAL, typename A, bool NTS, bool GEN>
 __device__ __forceinline__ void step_node32(const KParams &P, const float *__restrict__ fin,
                                             const float *__restrict__ gin, float *__restrict__ fout,
                                             float *__restrict__ gout, float *__restrict__ tlag,
@@ -553,10 +536,10 @@ __device__ __forceinline__ void step_node32(const KParams &P, const float *__res
     float g[Q];
     if constexpr (THERMAL) {
         dTlag = tlag[n];
-        gather_g32<FIRST, NTL>(P, R, b, gin, n, dTlag, g);
+        gather_g32<FIRST>(P, R, b, gin, n, dTlag, g);
     }
     float f[Q];
-    if constexpr (FLUID) gather_f32<FIRST, NTL>(P, R, b, fin, n, f);
+    if constexpr (FLUID) gather_f32<FIRST>(P, R, b, fin, n, f);
     A dT = A(0);
     if constexpr (THERMAL) {
         if constexpr (sizeof(A) == 4) {
@@ -566,7 +549,7 @@ __device__ __forceinline__ void step_node32(const KParams &P, const float *__res
         }
     }
     A ux = 0, uy = 0, uz = 0, tau_les = A(0);
-    const NodeOut<!NTL> out{fout, gout, tlag, taules, taules, n, n, (size_t)P.S};
+    const NodeOut<NTS> out{fout, gout, tlag, taules, taules, n, n, (size_t)P.S};
     if constexpr (FLUID) collide_fluid<A, GEN>(P, R, x, y, z, n, f, dTlag, dT, out, ux, uy, uz, tau_les);
     if constexpr (THERMAL) collide_thermal<A, GEN>(P, R, y, g, dT, ux, uy, uz, tau_les, out);
     if constexpr (GEN && !FIRST) {
@@ -587,30 +570,33 @@ __device__ __forceinline__ void step_node32(const KParams &P, const float *__res
 }
 
 // Row grid (blocks along x of one (y, z) row: row quantities block-uniform)
-// or, DENSE, a linear grid with one node per lane (see dense_rows).
-template <bool FIRST, bool FLUID, bool THERMAL, typename A, bool NTL, bool DENSE, bool GEN>
+// or, DENSE, a linear grid with one node per lane (see dense_rows), in the
+// block order of step_order.
+template <bool FIRST, bool FLUID, bool THERMAL, typename A, bool NTS, bool DENSE, bool GEN>
 __global__ void __launch_bounds__(256) k_step_fp32(KParams P, const float *__restrict__ fin,
                                                    const float *__restrict__ gin, float *__restrict__ fout,
                                                    float *__restrict__ gout, float *__restrict__ tlag,
-                                                   float *__restrict__ taules)
+                                                   float *__restrict__ taules, int run)
 {
     int x, y, z;
     uint32_t n;
+    const uint32_t lb = xcd_run(run, block_linear(), gridDim.x * gridDim.y * gridDim.z);
     if constexpr (DENSE) {
-        n = blockIdx.x * blockDim.x + threadIdx.x;
+        n = lb * blockDim.x + threadIdx.x;
         if (n >= (uint32_t)P.N) return;
         const uint32_t row = n / (uint32_t)P.NX;
         x = (int)(n - row * (uint32_t)P.NX);
         y = (int)(row % (uint32_t)P.NY);
         z = (int)(row / (uint32_t)P.NY);
     } else {
-        x = blockIdx.x * blockDim.x + threadIdx.x;
+        const uint32_t row = lb / gridDim.x;
+        x = (lb - row * gridDim.x) * blockDim.x + threadIdx.x;
         if (x >= P.NX) return;
-        y = blockIdx.y;
-        z = blockIdx.z;
-        n = ((uint32_t)z * P.NY + y) * P.NX + x;
+        y = (int)(row % (uint32_t)P.NY);
+        z = (int)(row / (uint32_t)P.NY);
+        n = row * (uint32_t)P.NX + x;
     }
-    step_node32<FIRST, FLUID, THERMAL, A, NTL, GEN>(P, fin, gin, fout, gout, tlag, taules, x, y, z, n);
+    step_node32<FIRST, FLUID, THERMAL, A, NTS, GEN>(P, fin, gin, fout, gout, tlag, taules, x, y, z, n);
 }
 
 // ---------------------------------------------------------------------------
@@ -674,7 +660,7 @@ constexpr int tile2_planes()
 
 // The two steps of one 64 x TY tile whose first node is (x0, y0), through
 // the block's LDS array t (shared by the single-lattice and batched kernels).
-template <bool FLUID, bool THERMAL, typename A, bool NTL, int TY>
+template <bool FLUID, bool THERMAL, typename A, bool NTS, int TY>
 __device__ __forceinline__ void step2_tile(const KParams &P, const float *__restrict__ fin,
                                            const float *__restrict__ gin, float *__restrict__ fout,
                                            float *__restrict__ gout, const float *__restrict__ tl_in,
@@ -701,9 +687,9 @@ __device__ __forceinline__ void step2_tile(const KParams &P, const float *__rest
         float g[Q], f[Q];
         if constexpr (THERMAL) {
             dTlag = tl_in[n];
-            gather_g32_o32<NTL>(P, R, b, gin, n, dTlag, g);
+            gather_g32_o32(P, R, b, gin, n, dTlag, g);
         }
-        if constexpr (FLUID) gather_f32_o32<NTL>(P, R, b, fin, n, f);
+        if constexpr (FLUID) gather_f32_o32(P, R, b, fin, n, f);
         A dT = A(0);
         if constexpr (THERMAL) {
             if constexpr (sizeof(A) == 4) {
@@ -742,21 +728,22 @@ __device__ __forceinline__ void step2_tile(const KParams &P, const float *__rest
         }
     }
     A ux = 0, uy = 0, uz = 0, tau_les = A(0);
-    const NodeOut32 out{fout, gout, tl_out, n * 4u, (uint32_t)P.S * 4u};
+    const NodeOut32<NTS> out{fout, gout, tl_out, n * 4u, (uint32_t)P.S * 4u};
     if constexpr (FLUID) collide_fluid<A, false>(P, R, x, y, 0, n, f, dTlag, dT, out, ux, uy, uz, tau_les);
     if constexpr (THERMAL) collide_thermal<A, false>(P, R, y, g, dT, ux, uy, uz, tau_les, out);
 }
 
-template <bool FLUID, bool THERMAL, typename A, bool NTL, int TY>
+template <bool FLUID, bool THERMAL, typename A, bool NTS, int TY>
 __global__ void __launch_bounds__(Tile2<TY>::THREADS) k_step2_fp32(KParams P, const float *__restrict__ fin,
                                                                    const float *__restrict__ gin,
                                                                    float *__restrict__ fout, float *__restrict__ gout,
                                                                    const float *__restrict__ tl_in,
-                                                                   float *__restrict__ tl_out)
+                                                                   float *__restrict__ tl_out, int run)
 {
     __shared__ float t[tile2_planes<FLUID, THERMAL>() * Tile2<TY>::M];
-    step2_tile<FLUID, THERMAL, A, NTL, TY>(P, fin, gin, fout, gout, tl_in, tl_out, blockIdx.x * T2_TX,
-                                           blockIdx.y * TY, t);
+    const uint32_t lb = xcd_run(run, block_linear(), gridDim.x * gridDim.y), row = lb / gridDim.x;
+    step2_tile<FLUID, THERMAL, A, NTS, TY>(P, fin, gin, fout, gout, tl_in, tl_out,
+                                           (int)(lb - row * gridDim.x) * T2_TX, (int)row * TY, t);
 }
 
 // ---------------------------------------------------------------------------
@@ -916,14 +903,13 @@ __device__ __forceinline__ Planes make_planes(const float *base, int64_t S)
 // cache-policy bits of buffer instructions: non-temporal
 constexpr int CPOL_NT = 2;
 
-template <int q, bool NT>
+template <int q>
 __device__ __forceinline__ float bload(const Planes &p, uint32_t soff, uint32_t voff)
 {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(p.r[q / 7], (int)voff, (int)soff,
-                                                                          NT ? CPOL_NT : 0));
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(p.r[q / 7], (int)voff, (int)soff, 0));
 }
 
-template <bool FLUID, bool THERMAL, bool NTL>
+template <bool FLUID, bool THERMAL>
 __device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, const Planes &pf, const Planes &pg,
                                              const float *__restrict__ tl_in, uint32_t n, RawNode &r)
 {
@@ -933,14 +919,14 @@ __device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, con
         static_for<0, Q>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             const bool cross = P.wall_t && crosses_wall<q>(b);
-            r.g[q] = bload<q, NTL>(pg, (uint32_t)(q % 7) * pg.pb, cross ? n4 : src_index<q>(b, P.NX, P.NY) * 4u);
+            r.g[q] = bload<q>(pg, (uint32_t)(q % 7) * pg.pb, cross ? n4 : src_index<q>(b, P.NX, P.NY) * 4u);
         });
     }
     if constexpr (FLUID) {
         static_for<0, Q>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             if constexpr (cyq(q) == 0) {
-                r.f[q] = bload<q, NTL>(pf, (uint32_t)(q % 7) * pf.pb, src_index<q>(b, P.NX, P.NY) * 4u);
+                r.f[q] = bload<q>(pf, (uint32_t)(q % 7) * pf.pb, src_index<q>(b, P.NX, P.NY) * 4u);
             } else {
                 // bounce-back reads the opposite plane (same group of seven)
                 constexpr int iq = q % 7, ii = invq(q) % 7, mn = iq < ii ? iq : ii;
@@ -948,7 +934,7 @@ __device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, con
                 const bool cross = P.wall_f && crosses_wall<q>(b);
                 const uint32_t voff = cross ? n4 + (uint32_t)(ii - mn) * pf.pb
                                             : src_index<q>(b, P.NX, P.NY) * 4u + (uint32_t)(iq - mn) * pf.pb;
-                r.f[q] = bload<q, NTL>(pf, (uint32_t)mn * pf.pb, voff);
+                r.f[q] = bload<q>(pf, (uint32_t)mn * pf.pb, voff);
             }
         });
     }
@@ -1068,22 +1054,21 @@ __device__ __forceinline__ void ring_put(float *t, int m, int it, const float rf
 // not written.  Per two steps the state is read (1 + 2/zc) x M/T times and
 // written once; the temperature lag is read from tl_in and written to tl_out
 // (halo nodes of one block are tile nodes of another).
-template <bool FLUID, bool THERMAL, typename A, bool NTL, class TZ>
+template <bool FLUID, bool THERMAL, typename A, class TZ>
 __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp32(KParams P, const float *__restrict__ fin,
                                                              const float *__restrict__ gin, float *__restrict__ fout,
                                                              float *__restrict__ gout,
                                                              const float *__restrict__ tl_in,
-                                                             float *__restrict__ tl_out, int zc, int remap)
+                                                             float *__restrict__ tl_out, int zc)
 {
     constexpr int M = TZ::M, W = TZ::W, TX = TZ::TX, TY = TZ::TY;
     __shared__ float t[TZ::FLOATS];
     const int NX = P.NX, NY = P.NY, NZ = P.NZ;
-    // block -> (x tile, y tile, z range); with remap, the blocks that one XCD
-    // receives (every 8th in dispatch order) cover consecutive tiles, so
-    // neighbouring tiles share their halo rows in that XCD's L2
-    const uint32_t nbx = gridDim.x, nby = gridDim.y, total = nbx * nby * gridDim.z;
-    uint32_t bid = blockIdx.x + nbx * (blockIdx.y + nby * blockIdx.z);
-    if (remap) bid = xcd_block(bid, total);
+    // block -> (x tile, y tile, z range); the blocks that one XCD receives
+    // cover consecutive tiles, so neighbouring tiles share their halo rows in
+    // that XCD's L2
+    const uint32_t nbx = gridDim.x, nby = gridDim.y;
+    const uint32_t bid = xcd_block(block_linear(), nbx * nby * gridDim.z);
     const int x0 = (int)(bid % nbx) * TX, y0 = (int)((bid / nbx) % nby) * TY;
     const int zb = (int)(bid / (nbx * nby)) * zc, ze = min(zb + zc, NZ);
     const int w = NX - x0 < TX ? NX - x0 : TX;
@@ -1129,7 +1114,7 @@ __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp32(KParams P, const fl
             node_a(it, n, b);
             const Row R = row_of(P, ya);
             RawNode cur;
-            load_raw_buf<FLUID, THERMAL, NTL>(P, b, pin_f, pin_g, tl_in, n, cur);
+            load_raw_buf<FLUID, THERMAL>(P, b, pin_f, pin_g, tl_in, n, cur);
             finish_raw<FLUID, THERMAL>(P, R, b, cur);
             const float dTlag = THERMAL ? cur.tl : 0.f;
             A dT = A(0);
@@ -1220,13 +1205,14 @@ __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp32(KParams P, const fl
 // of the lattice's share of a chunk; the lag stays in place).  Population
 // buffers alternate with every launch of a lattice, its lag arrays with
 // every two-step launch (parities in the slot).
-template <bool FLUID, bool THERMAL, typename A, bool NTL>
+template <bool FLUID, bool THERMAL, typename A, bool NTS>
 __global__ void __launch_bounds__(Tile2<4>::THREADS) k_step2_batch32(const BatchEntry *__restrict__ tab,
-                                                                     const BatchSlot *__restrict__ slots, int nslots)
+                                                                     const BatchSlot *__restrict__ slots, int nslots,
+                                                                     int run)
 {
     constexpr int TY = 4;
     __shared__ float t[tile2_planes<FLUID, THERMAL>() * Tile2<TY>::M];
-    const uint32_t bt = blockIdx.x;
+    const uint32_t bt = xcd_run(run, blockIdx.x, gridDim.x);
     if (bt >= slots[nslots].tile0) return;
     int lo = 0, hi = nslots - 1;
     while (lo < hi) {
@@ -1250,11 +1236,11 @@ __global__ void __launch_bounds__(Tile2<4>::THREADS) k_step2_batch32(const Batch
     if (single) {
         const int x = x0 + (int)threadIdx.x % T2_TX, y = y0 + (int)threadIdx.x / T2_TX;
         if ((int)threadIdx.x >= T2_TX * TY || x >= P.NX || y >= P.NY) return;
-        step_node32<false, FLUID, THERMAL, A, NTL, false>(P, fin, gin, fout, gout, tl_a, (float *)E.taules, x, y, 0,
+        step_node32<false, FLUID, THERMAL, A, NTS, false>(P, fin, gin, fout, gout, tl_a, (float *)E.taules, x, y, 0,
                                                            (uint32_t)y * (uint32_t)P.NX + (uint32_t)x);
         return;
     }
-    step2_tile<FLUID, THERMAL, A, NTL, TY>(P, fin, gin, fout, gout, tl_a, tl_b, x0, y0, t);
+    step2_tile<FLUID, THERMAL, A, NTS, TY>(P, fin, gin, fout, gout, tl_a, tl_b, x0, y0, t);
 }
 
 // Velocity of the step at every node (the u[] that add_collision reads,
@@ -1271,7 +1257,7 @@ __global__ void __launch_bounds__(256) k_velocity32(KParams P, const float *__re
     const Row R = row_of(P, y);
     const Nbr b = make_nbr(x, y, z, P.NX, P.NY, P.NZ);
     float f[Q];
-    gather_f32<FIRST, false>(P, R, b, fin, n, f);
+    gather_f32<FIRST>(P, R, b, fin, n, f);
     const float dTlag = P.thermal ? tlag[n] : 0.f;
     Moments<A> m;
     fluid_moments<A, true>(P, R, x, y, z, n, f, dTlag, m);
@@ -1286,11 +1272,12 @@ __global__ void __launch_bounds__(256) k_velocity32(KParams P, const float *__re
 // holds it (wave-uniform binary search over the launch's few slots), with
 // that lattice's step parity; the state buffer of each lattice alternates
 // with the step parity.  One instance per population-set kind.
-template <bool FLUID, bool THERMAL, typename A, bool NTL, bool DENSE, bool GEN>
+template <bool FLUID, bool THERMAL, typename A, bool NTS, bool DENSE, bool GEN>
 __global__ void __launch_bounds__(256) k_step_batch32(const BatchEntry *__restrict__ tab,
-                                                      const BatchSlot *__restrict__ slots, int nslots)
+                                                      const BatchSlot *__restrict__ slots, int nslots, int run)
 {
-    const uint32_t wt = __builtin_amdgcn_readfirstlane(blockIdx.x * BATCH_WAVES_PER_BLOCK + threadIdx.x / BATCH_WAVE);
+    const uint32_t wt = __builtin_amdgcn_readfirstlane(xcd_run(run, blockIdx.x, gridDim.x) * BATCH_WAVES_PER_BLOCK +
+                                                       threadIdx.x / BATCH_WAVE);
     if (wt >= slots[nslots].tile0) return;
     int lo = 0, hi = nslots - 1;
     while (lo < hi) {
@@ -1327,7 +1314,7 @@ __global__ void __launch_bounds__(256) k_step_batch32(const BatchEntry *__restri
         z = row / (uint32_t)P.NY;
         n = row * (uint32_t)P.NX + x;
     }
-    step_node32<false, FLUID, THERMAL, A, NTL, GEN>(P, fin, gin, fout, gout, tl, tau, (int)x, (int)y, (int)z, n);
+    step_node32<false, FLUID, THERMAL, A, NTS, GEN>(P, fin, gin, fout, gout, tl, tau, (int)x, (int)y, (int)z, n);
 }
 
 __global__ void __launch_bounds__(256) k_gather_fp32(KParams P, const float *__restrict__ fin,
@@ -1351,9 +1338,9 @@ __global__ void __launch_bounds__(256) k_gather_fp32(KParams P, const float *__r
         float g[Q];
         dTlag = tlag[n];
         if (P.first)
-            gather_g32<true, false>(P, R, b, gin, n, dTlag, g);
+            gather_g32<true>(P, R, b, gin, n, dTlag, g);
         else
-            gather_g32<false, false>(P, R, b, gin, n, dTlag, g);
+            gather_g32<false>(P, R, b, gin, n, dTlag, g);
         double s = 0.0;
         for (int q = 0; q < Q; q++) {
             s += (double)g[q];
@@ -1365,9 +1352,9 @@ __global__ void __launch_bounds__(256) k_gather_fp32(KParams P, const float *__r
     if (P.fluid) {
         float f[Q];
         if (P.first)
-            gather_f32<true, false>(P, R, b, fin, n, f);
+            gather_f32<true>(P, R, b, fin, n, f);
         else
-            gather_f32<false, false>(P, R, b, fin, n, f);
+            gather_f32<false>(P, R, b, fin, n, f);
         double drho = 0.0, jx = 0.0, jy = 0.0, jz = 0.0;
         for (int q = 0; q < Q; q++) {
             double d = (double)f[q];
@@ -1415,22 +1402,20 @@ void launch_step_fp32(const KParams &P, const float *fin, const float *gin, floa
         grid = dim3((unsigned)((P.N + 255) / 256));
         block = dim3(256);
     }
-    // both lattices resident in the 256 MB last-level cache?
-    const int64_t lattice_bytes = 2 * (int64_t)Q * P.N * 4 * ((P.fluid ? 1 : 0) + (P.thermal ? 1 : 0));
-    const bool ntl = lattice_bytes <= ((int64_t)192 << 20);
+    const StepOrder o = step_order(state_bytes(P, 4), dense || P.NX % 32 == 0, CACHED_BYTES);
     const bool gen = P.hit || P.les || P.twoway || P.part || P.f0p || P.f0n;
 #define CH4G_LAUNCH32G_(F_, FL_, TH_, A_, N_, D_)                                                                     \
     do {                                                                                                              \
         if (gen)                                                                                                      \
             hipLaunchKernelGGL((k_step_fp32<F_, FL_, TH_, A_, N_, D_, true>), grid, block, 0, s, P, fin, gin, fout,  \
-                               gout, tlag, taules);                                                                   \
+                               gout, tlag, taules, o.run);                                                            \
         else                                                                                                          \
             hipLaunchKernelGGL((k_step_fp32<F_, FL_, TH_, A_, N_, D_, false>), grid, block, 0, s, P, fin, gin, fout, \
-                               gout, tlag, taules);                                                                   \
+                               gout, tlag, taules, o.run);                                                            \
     } while (0)
 #define CH4G_LAUNCH32D_(F_, FL_, TH_, A_, D_)                                                                          \
     do {                                                                                                              \
-        if (ntl)                                                                                                      \
+        if (o.nts)                                                                                                    \
             CH4G_LAUNCH32G_(F_, FL_, TH_, A_, true, D_);                                                              \
         else                                                                                                          \
             CH4G_LAUNCH32G_(F_, FL_, TH_, A_, false, D_);                                                             \
@@ -1491,27 +1476,19 @@ namespace {
 // planes.
 template <class TZ>
 void launch_z2(const KParams &P, const float *fin, const float *gin, float *fout, float *gout, const float *tl_in,
-               float *tl_out, int zc, int remap, bool ntl, hipStream_t s)
+               float *tl_out, int zc, hipStream_t s)
 {
     const unsigned bx = (unsigned)((P.NX + TZ::TX - 1) / TZ::TX), by = (unsigned)((P.NY + TZ::TY - 1) / TZ::TY);
     const dim3 grid(bx, by, (unsigned)((P.NZ + zc - 1) / zc));
-#define CH4G_Z2N_(FL_, TH_, A_, N_)                                                                                   \
-    hipLaunchKernelGGL((k_step2z_fp32<FL_, TH_, A_, N_, TZ>), grid, dim3(TZ::THREADS), 0, s, P, fin, gin, fout,     \
-                       gout, tl_in, tl_out, zc, remap)
 #define CH4G_Z2_(FL_, TH_, A_)                                                                                        \
-    do {                                                                                                              \
-        if (ntl)                                                                                                      \
-            CH4G_Z2N_(FL_, TH_, A_, true);                                                                            \
-        else                                                                                                          \
-            CH4G_Z2N_(FL_, TH_, A_, false);                                                                           \
-    } while (0)
+    hipLaunchKernelGGL((k_step2z_fp32<FL_, TH_, A_, TZ>), grid, dim3(TZ::THREADS), 0, s, P, fin, gin, fout, gout,   \
+                       tl_in, tl_out, zc)
     constexpr bool FL = TZ::F == 1, TH = TZ::H == 1;
     if (P.arith64)
         CH4G_Z2_(FL, TH, double);
     else
         CH4G_Z2_(FL, TH, float);
 #undef CH4G_Z2_
-#undef CH4G_Z2N_
 }
 
 template <bool FL, bool TH, int TX, int TY, bool HOLD>
@@ -1528,16 +1505,14 @@ using TZ_ = TileZ<FL, TH, TX, TY, HOLD>;
 void launch_two_steps_3d(const KParams &P, const float *fin, const float *gin, float *fout, float *gout,
                          const float *tl_in, float *tl_out, hipStream_t s)
 {
-    const int64_t lattice_bytes = 2 * (int64_t)Q * P.N * 4 * ((P.fluid ? 1 : 0) + (P.thermal ? 1 : 0));
-    const bool ntl = lattice_bytes <= ((int64_t)192 << 20);
     const bool tall = P.fluid && !(P.thermal && P.arith64);
     const int TY = tall ? 8 : 4;
     const int64_t columns = (int64_t)((P.NX + 63) / 64) * ((P.NY + TY - 1) / TY);
     int64_t zc = (int64_t)P.NZ * columns / 1024;
     zc = zc < 8 ? 8 : (zc > 128 ? 128 : zc);
     zc = zc > P.NZ ? P.NZ : zc;
-    const int z = (int)zc, remap = 1;
-#define Z2(...) launch_z2<TZ_<__VA_ARGS__>>(P, fin, gin, fout, gout, tl_in, tl_out, z, remap, ntl, s)
+    const int z = (int)zc;
+#define Z2(...) launch_z2<TZ_<__VA_ARGS__>>(P, fin, gin, fout, gout, tl_in, tl_out, z, s)
     if (P.fluid && P.thermal) {
         if (P.arith64)
             Z2(true, true, 64, 4, true);
@@ -1560,13 +1535,11 @@ void launch_two_steps_fp32(const KParams &P, const float *fin, const float *gin,
         launch_two_steps_3d(P, fin, gin, fout, gout, tl_in, tl_out, s);
         return;
     }
-    // non-temporal loads while both lattices fit the last-level cache (as the
-    // single-step kernel); 64x5 tiles (fewer halo nodes) once there are at
+    // 64x5 tiles (fewer halo nodes) once there are at
     // least two rounds of blocks (two blocks per CU by LDS), else 64x4 tiles
     // (more, smaller blocks fill the CUs evenly; 64x3 tiles, three blocks per
     // CU, were slower at 512x256: 9.6 against 7.3 us per step)
-    const int64_t lattice_bytes = 2 * (int64_t)Q * P.N * 4 * ((P.fluid ? 1 : 0) + (P.thermal ? 1 : 0));
-    const bool ntl = lattice_bytes <= ((int64_t)192 << 20);
+    const StepOrder o = step_order(state_bytes(P, 4), P.NX % 32 == 0, RANGE_BYTES_2D);
     const unsigned bx = (unsigned)((P.NX + T2_TX - 1) / T2_TX);
     const bool ty5 = (int64_t)bx * ((P.NY + 4) / 5) >= 1024;
     const dim3 g4(bx, (unsigned)((P.NY + 3) / 4)), g5(bx, (unsigned)((P.NY + 4) / 5));
@@ -1574,14 +1547,14 @@ void launch_two_steps_fp32(const KParams &P, const float *fin, const float *gin,
     do {                                                                                                              \
         if (ty5)                                                                                                      \
             hipLaunchKernelGGL((k_step2_fp32<FL_, TH_, A_, N_, 5>), g5, dim3(Tile2<5>::THREADS), 0, s, P, fin, gin,  \
-                               fout, gout, tl_in, tl_out);                                                            \
+                               fout, gout, tl_in, tl_out, o.run);                                                            \
         else                                                                                                          \
             hipLaunchKernelGGL((k_step2_fp32<FL_, TH_, A_, N_, 4>), g4, dim3(Tile2<4>::THREADS), 0, s, P, fin, gin,  \
-                               fout, gout, tl_in, tl_out);                                                            \
+                               fout, gout, tl_in, tl_out, o.run);                                                            \
     } while (0)
 #define CH4G_T2_(FL_, TH_, A_)                                                                                        \
     do {                                                                                                              \
-        if (ntl)                                                                                                      \
+        if (o.nts)                                                                                                    \
             CH4G_T2N_(FL_, TH_, A_, true);                                                                            \
         else                                                                                                          \
             CH4G_T2N_(FL_, TH_, A_, false);                                                                           \
@@ -1622,20 +1595,21 @@ void launch_velocity_fp32(const KParams &P, const float *fin, const float *tlag,
 }
 
 void launch_batch_fp32(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
-                       bool dense, bool gen, int arith64, bool ntl, hipStream_t s)
+                       bool dense, bool gen, int arith64, StepOrder o, hipStream_t s)
 {
     dim3 grid((unsigned)nblocks), block(256);
 #define CH4G_BATCH32G_(FL_, TH_, A_, N_, D_)                                                                          \
     do {                                                                                                              \
         if (gen)                                                                                                      \
-            hipLaunchKernelGGL((k_step_batch32<FL_, TH_, A_, N_, D_, true>), grid, block, 0, s, tab, slots, nslots); \
+            hipLaunchKernelGGL((k_step_batch32<FL_, TH_, A_, N_, D_, true>), grid, block, 0, s, tab, slots, nslots,   \
+                               o.run);                                                                                \
         else                                                                                                          \
             hipLaunchKernelGGL((k_step_batch32<FL_, TH_, A_, N_, D_, false>), grid, block, 0, s, tab, slots,         \
-                               nslots);                                                                               \
+                               nslots, o.run);                                                                               \
     } while (0)
 #define CH4G_BATCH32D_(FL_, TH_, A_, D_)                                                                              \
     do {                                                                                                              \
-        if (ntl)                                                                                                      \
+        if (o.nts)                                                                                                    \
             CH4G_BATCH32G_(FL_, TH_, A_, true, D_);                                                                   \
         else                                                                                                          \
             CH4G_BATCH32G_(FL_, TH_, A_, false, D_);                                                                  \
@@ -1667,15 +1641,15 @@ void launch_batch_fp32(const BatchEntry *tab, const BatchSlot *slots, int nslots
 }
 
 void launch_batch2_fp32(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
-                        int arith64, bool ntl, hipStream_t s)
+                        int arith64, StepOrder o, hipStream_t s)
 {
     dim3 grid((unsigned)nblocks), block(Tile2<4>::THREADS);
 #define CH4G_B2_(FL_, TH_, A_)                                                                                        \
     do {                                                                                                              \
-        if (ntl)                                                                                                      \
-            hipLaunchKernelGGL((k_step2_batch32<FL_, TH_, A_, true>), grid, block, 0, s, tab, slots, nslots);         \
+        if (o.nts)                                                                                                    \
+            hipLaunchKernelGGL((k_step2_batch32<FL_, TH_, A_, true>), grid, block, 0, s, tab, slots, nslots, o.run);         \
         else                                                                                                          \
-            hipLaunchKernelGGL((k_step2_batch32<FL_, TH_, A_, false>), grid, block, 0, s, tab, slots, nslots);        \
+            hipLaunchKernelGGL((k_step2_batch32<FL_, TH_, A_, false>), grid, block, 0, s, tab, slots, nslots, o.run);        \
     } while (0)
 #define CH4G_B2(FL_, TH_)                                                                                             \
     do {                                                                                                              \
@@ -1723,7 +1697,7 @@ __global__ void __launch_bounds__(FM32_THREADS) k_force_sum32(KParams P, const f
             float dT = 0.f;
             if (P.thermal && P.buoy) {
                 float g[Q];
-                gather_g32<FIRST, false>(P, R, make_nbr(x, y, z, P.NX, P.NY, P.NZ), gin, n, dTlag, g);
+                gather_g32<FIRST>(P, R, make_nbr(x, y, z, P.NX, P.NY, P.NZ), gin, n, dTlag, g);
                 if (P.arith64) {
                     double s = 0.0;
                     for (int q = 0; q < Q; q++) s += (double)g[q];

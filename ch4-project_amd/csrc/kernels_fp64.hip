@@ -128,6 +128,16 @@ __device__ __forceinline__ void gather_thermal(const KParams &P, const Nbr &b, c
     });
 }
 
+// population stores: non-temporal (NT) where step_order says so
+template <bool NT>
+__device__ __forceinline__ void stp64(double *p, double v)
+{
+    if constexpr (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
 // equilibrium (lb.c:382-415)
 __device__ __forceinline__ double feq_q(const KParams &P, int q, double rho, double ux, double uy, double uz,
                                         double u2)
@@ -227,7 +237,7 @@ __device__ __forceinline__ void fluid_velocity64(const KParams &P, const double 
 
 // One node of the fused step (shared by the single-lattice and the batched
 // kernels, so a lattice advances bit-identically in either).
-template <bool FIRST, bool FLUID, bool THERMAL>
+template <bool FIRST, bool FLUID, bool THERMAL, bool NT>
 __device__ __forceinline__ void step_node64(const KParams &P, const double *__restrict__ fin,
                                             const double *__restrict__ gin, double *__restrict__ fout,
                                             double *__restrict__ gout, double *__restrict__ tlag,
@@ -279,7 +289,7 @@ __device__ __forceinline__ void step_node64(const KParams &P, const double *__re
                 r += P.guo_fac * wq(q) * rho * Fn[1] * dy;
                 r += P.guo_fac * wq(q) * rho * Fn[2] * dz;
             }
-            fout[(size_t)q * N + n] = r;
+            stp64<NT>(fout + (size_t)q * N + n, r);
         }
     }
 
@@ -292,36 +302,39 @@ __device__ __forceinline__ void step_node64(const KParams &P, const double *__re
         for (int q = 0; q < Q; q++) {
             double r = g[q];
             r += -invtau_t * (g[q] - feq_q(P, q, T, ux, uy, uz, u2));
-            gout[(size_t)q * N + n] = r;
+            stp64<NT>(gout + (size_t)q * N + n, r);
         }
         tlag[n] = T;
     }
 }
 
-// Row grid or, DENSE, a linear grid with one node per lane (see dense_rows).
-template <bool FIRST, bool FLUID, bool THERMAL, bool DENSE>
+// Row grid or, DENSE, a linear grid with one node per lane (see dense_rows),
+// in the block order of step_order.
+template <bool FIRST, bool FLUID, bool THERMAL, bool DENSE, bool NT>
 __global__ void __launch_bounds__(256) k_step_fp64(KParams P, const double *__restrict__ fin,
                                                    const double *__restrict__ gin, double *__restrict__ fout,
                                                    double *__restrict__ gout, double *__restrict__ tlag,
-                                                   double *__restrict__ taules)
+                                                   double *__restrict__ taules, int run)
 {
     int x, y, z;
     uint32_t n;
+    const uint32_t lb = xcd_run(run, block_linear(), gridDim.x * gridDim.y * gridDim.z);
     if constexpr (DENSE) {
-        n = blockIdx.x * blockDim.x + threadIdx.x;
+        n = lb * blockDim.x + threadIdx.x;
         if (n >= (uint32_t)P.N) return;
         const uint32_t row = n / (uint32_t)P.NX;
         x = (int)(n - row * (uint32_t)P.NX);
         y = (int)(row % (uint32_t)P.NY);
         z = (int)(row / (uint32_t)P.NY);
     } else {
-        x = blockIdx.x * blockDim.x + threadIdx.x;
+        const uint32_t row = lb / gridDim.x;
+        x = (lb - row * gridDim.x) * blockDim.x + threadIdx.x;
         if (x >= P.NX) return;
-        y = blockIdx.y;
-        z = blockIdx.z;
-        n = ((uint32_t)z * P.NY + y) * P.NX + x;
+        y = (int)(row % (uint32_t)P.NY);
+        z = (int)(row / (uint32_t)P.NY);
+        n = row * (uint32_t)P.NX + x;
     }
-    step_node64<FIRST, FLUID, THERMAL>(P, fin, gin, fout, gout, tlag, taules, x, y, z, n);
+    step_node64<FIRST, FLUID, THERMAL, NT>(P, fin, gin, fout, gout, tlag, taules, x, y, z, n);
 }
 
 // Velocity of the step at every node (the u[] that add_collision reads,
@@ -348,11 +361,12 @@ __global__ void __launch_bounds__(256) k_velocity64(KParams P, const double *__r
 }
 
 // Many lattices in one launch (see k_step_batch32).
-template <bool FLUID, bool THERMAL, bool DENSE>
+template <bool FLUID, bool THERMAL, bool DENSE, bool NT>
 __global__ void __launch_bounds__(256) k_step_batch64(const BatchEntry *__restrict__ tab,
-                                                      const BatchSlot *__restrict__ slots, int nslots)
+                                                      const BatchSlot *__restrict__ slots, int nslots, int run)
 {
-    const uint32_t wt = __builtin_amdgcn_readfirstlane(blockIdx.x * BATCH_WAVES_PER_BLOCK + threadIdx.x / BATCH_WAVE);
+    const uint32_t wt = __builtin_amdgcn_readfirstlane(xcd_run(run, blockIdx.x, gridDim.x) * BATCH_WAVES_PER_BLOCK +
+                                                       threadIdx.x / BATCH_WAVE);
     if (wt >= slots[nslots].tile0) return;
     int lo = 0, hi = nslots - 1;
     while (lo < hi) {
@@ -389,7 +403,7 @@ __global__ void __launch_bounds__(256) k_step_batch64(const BatchEntry *__restri
         z = row / (uint32_t)P.NY;
         n = row * (uint32_t)P.NX + x;
     }
-    step_node64<false, FLUID, THERMAL>(P, fin, gin, fout, gout, tl, tau, (int)x, (int)y, (int)z, n);
+    step_node64<false, FLUID, THERMAL, NT>(P, fin, gin, fout, gout, tl, tau, (int)x, (int)y, (int)z, n);
 }
 
 // Streaming of the last step + hydro_fields, without a new collision:
@@ -462,14 +476,24 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
         grid = dim3((unsigned)((P.N + 255) / 256));
         block = dim3(256);
     }
+    const StepOrder o = step_order(state_bytes(P, 8), dense || P.NX % 16 == 0, RANGE_BYTES_64);
+    // ranges and plain stores go together (see step_order)
+    const bool nt = o.nts && o.run == RUN_GROUP;
+#define CH4G_LAUNCH64N_(F_, FL_, TH_, D_)                                                                             \
+    do {                                                                                                              \
+        if (nt)                                                                                                       \
+            hipLaunchKernelGGL((k_step_fp64<F_, FL_, TH_, D_, true>), grid, block, 0, s, P, fin, gin, fout, gout,    \
+                               tlag, taules, o.run);                                                                  \
+        else                                                                                                          \
+            hipLaunchKernelGGL((k_step_fp64<F_, FL_, TH_, D_, false>), grid, block, 0, s, P, fin, gin, fout, gout,   \
+                               tlag, taules, o.run);                                                                  \
+    } while (0)
 #define CH4G_LAUNCH64(F_, FL_, TH_)                                                                                   \
     do {                                                                                                              \
         if (!(F_) && dense)                                                                                           \
-            hipLaunchKernelGGL((k_step_fp64<false, FL_, TH_, true>), grid, block, 0, s, P, fin, gin, fout, gout,     \
-                               tlag, taules);                                                                         \
+            CH4G_LAUNCH64N_(false, FL_, TH_, true);                                                                   \
         else                                                                                                          \
-            hipLaunchKernelGGL((k_step_fp64<F_, FL_, TH_, false>), grid, block, 0, s, P, fin, gin, fout, gout, tlag, \
-                               taules);                                                                               \
+            CH4G_LAUNCH64N_(F_, FL_, TH_, false);                                                                     \
     } while (0)
     if (P.fluid && P.thermal) {
         if (P.first) CH4G_LAUNCH64(true, true, true); else CH4G_LAUNCH64(false, true, true);
@@ -479,6 +503,7 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
         if (P.first) CH4G_LAUNCH64(true, false, true); else CH4G_LAUNCH64(false, false, true);
     }
 #undef CH4G_LAUNCH64
+#undef CH4G_LAUNCH64N_
 }
 
 void launch_velocity_fp64(const KParams &P, const double *fin, const double *tlag, hipStream_t s)
@@ -492,15 +517,23 @@ void launch_velocity_fp64(const KParams &P, const double *fin, const double *tla
 }
 
 void launch_batch_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
-                       bool dense, hipStream_t s)
+                       bool dense, StepOrder o, hipStream_t s)
 {
     dim3 grid((unsigned)nblocks), block(256);
+    const bool nt = o.nts && o.run == RUN_GROUP;
+#define CH4G_BATCH64N_(FL_, TH_, D_)                                                                                  \
+    do {                                                                                                              \
+        if (nt)                                                                                                       \
+            hipLaunchKernelGGL((k_step_batch64<FL_, TH_, D_, true>), grid, block, 0, s, tab, slots, nslots, o.run);  \
+        else                                                                                                          \
+            hipLaunchKernelGGL((k_step_batch64<FL_, TH_, D_, false>), grid, block, 0, s, tab, slots, nslots, o.run); \
+    } while (0)
 #define CH4G_BATCH64(FL_, TH_)                                                                                        \
     do {                                                                                                              \
         if (dense)                                                                                                    \
-            hipLaunchKernelGGL((k_step_batch64<FL_, TH_, true>), grid, block, 0, s, tab, slots, nslots);            \
+            CH4G_BATCH64N_(FL_, TH_, true);                                                                           \
         else                                                                                                          \
-            hipLaunchKernelGGL((k_step_batch64<FL_, TH_, false>), grid, block, 0, s, tab, slots, nslots);           \
+            CH4G_BATCH64N_(FL_, TH_, false);                                                                          \
     } while (0)
     if (kind == BATCH_FLUID_THERMAL)
         CH4G_BATCH64(true, true);
@@ -509,6 +542,7 @@ void launch_batch_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots
     else
         CH4G_BATCH64(false, true);
 #undef CH4G_BATCH64
+#undef CH4G_BATCH64N_
 }
 
 // LB_FLUID_FORCING_NOZEROMODE (forcing.c:1123-1152): sums over all nodes of
