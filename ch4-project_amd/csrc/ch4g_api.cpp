@@ -991,11 +991,12 @@ int ch4g_dump_rulers(ch4g_lattice *L, ch4g_output *rx, ch4g_output *ry, ch4g_out
     if (rc) return rc;
     const ch4g_config &c = L->cfg;
     const size_t planes = (size_t)c.NX + c.NY + c.NZ;
-    if (!L->d_rul && (rc = dalloc(L, (void **)&L->d_rul, planes * NOUT * sizeof(double)))) return rc;
+    if (!L->d_rul && (rc = dalloc(L, (void **)&L->d_rul, (planes * NOUT + ruler_scratch_doubles(L->base)) * sizeof(double))))
+        return rc;
     double *dx = L->d_rul, *dy = dx + (size_t)c.NX * NOUT, *dz = dy + (size_t)c.NY * NOUT;
     gather(L, nullptr, nullptr, L->d_dens, L->d_u, L->d_t);
-    launch_rulers(L->base, L->d_dens, L->d_u, L->d_t, L->nu, L->kappa, rx ? dx : nullptr, ry ? dy : nullptr,
-                  rz ? dz : nullptr, L->stream);
+    launch_rulers(L->base, L->d_dens, L->d_u, L->d_t, L->nu, L->kappa, L->d_rul + planes * NOUT, rx ? dx : nullptr,
+                  ry ? dy : nullptr, rz ? dz : nullptr, L->stream);
     HIPCHK(hipGetLastError());
     std::vector<double> h(planes * NOUT);
     HIPCHK(hipMemcpyAsync(h.data(), L->d_rul, h.size() * sizeof(double), hipMemcpyDeviceToHost, L->stream));

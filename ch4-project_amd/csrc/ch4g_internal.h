@@ -472,8 +472,10 @@ constexpr int NOUT = 26;
 int reduce_blocks(const KParams &P);
 void launch_averages(const KParams &P, const double *dens, const double *u, const double *t, double nu, double kappa,
                      double *partials, double *result, hipStream_t s);
-// plane sums of the same terms along x, y, z: [NX|NY|NZ][NOUT], null to skip
+// plane sums of the same terms along x, y, z: [NX|NY|NZ][NOUT], null to skip;
+// scratch: ruler_scratch_doubles of them for partial sums
+size_t ruler_scratch_doubles(const KParams &P);
 void launch_rulers(const KParams &P, const double *dens, const double *u, const double *t, double nu, double kappa,
-                   double *rx, double *ry, double *rz, hipStream_t s);
+                   double *scratch, double *rx, double *ry, double *rz, hipStream_t s);
 
 }  // namespace ch4g

@@ -94,7 +94,7 @@ struct ch4g_lattice {
     // lazily allocated FP64 scratch
     double *d_dens = nullptr, *d_u = nullptr, *d_t = nullptr;
     double *d_part = nullptr, *d_res = nullptr;
-    double *d_rul = nullptr;  // ruler plane sums [NX + NY + NZ][NOUT]
+    double *d_rul = nullptr;  // ruler plane sums [NX + NY + NZ][NOUT], then their partial sums
     float4 *d_uT32 = nullptr;  // [N] (u_x, u_y, u_z, T) in float for particles (float storage)
     double *d_fs = nullptr, *d_gs = nullptr;
     // FP32-deviation per-row base state

@@ -92,31 +92,102 @@ void launch_load(const KParams &P, const double *fs, const double *gs, void *f, 
 // ---------------------------------------------------------------------------
 // dump_averages (output.c:183-491): per-node FP64 contributions, centred
 // differences with periodic wrap, one-sided second order at y walls
-// (gradients.c:78-499, :505-626), block partials in LDS tree order, then one
-// block sums the partials in block order.  Output order = ch4g_output.
+// (gradients.c:78-499, :505-626), summed in a fixed order.  Output order =
+// ch4g_output.
+//
+// Every node's terms need the fields of seven nodes (29 doubles of which 5
+// are new), so a wave takes 64 x of a row and marches: along y for the sums
+// over x-y planes (k_plane_sums: averages, z ruler), along z for those over
+// the other planes (k_column_sums: x and y rulers), with the node and its two
+// neighbours along the march in registers and the sums in registers over the
+// whole march.  256^3, us, one node per thread and one LDS tree per term ->
+// this: averages 630 -> 280 (0.67 GB of fields), final sum 616 -> 8; rulers,
+// one block per plane before, x 3480, y 744, z 660 -> 670 together.  Small
+// lattices: 32 -> 10 for the averages.
 
-constexpr int RED_THREADS = 256;
+constexpr int RED_THREADS = 256, RED_WAVES = RED_THREADS / 64;
+constexpr int NTERM = 25;  // ch4g_output without lb, which is formed from the sums
 
+// work of one block: unit = (z plane, part of it); a part is RED_WAVES waves,
+// each 64 x of `rows` consecutive rows
+struct PlaneWork {
+    int nxt, rows, parts;
+    int64_t units;
+};
+
+static PlaneWork plane_work(const KParams &P)
+{
+    PlaneWork w;
+    w.nxt = (P.NX + 63) / 64;
+    // rows per wave: up to 16 (the two rows next to a march are read again),
+    // fewer where that would leave less than 4 waves per SIMD
+    const int64_t waves = (int64_t)w.nxt * P.NY * P.NZ;
+    const int64_t r = waves / 4096;
+    w.rows = (int)(r < 1 ? 1 : (r > 16 ? 16 : r));
+    const int64_t tasks = (int64_t)w.nxt * ((P.NY + w.rows - 1) / w.rows);
+    w.parts = (int)((tasks + RED_WAVES - 1) / RED_WAVES);
+    w.units = (int64_t)w.parts * P.NZ;
+    return w;
+}
+
+// blocks of the averages' sum, each over every gridDim-th unit
 int reduce_blocks(const KParams &P)
 {
-    int64_t nb = (P.N + RED_THREADS - 1) / RED_THREADS;
+    const int64_t nb = plane_work(P).units;
     return (int)(nb < 2048 ? nb : 2048);
 }
 
-// Per-node terms of dump_averages (output.c:183-491) at node n = (x,y,z),
-// added into a[] in the order of ch4g_output.  u is [N][3], fields of the
-// current step; periodic images, one-sided differences at y walls.
-__device__ __forceinline__ void node_terms(const KParams &P, const double *__restrict__ dens,
-                                           const double *__restrict__ u, const double *__restrict__ t, double nu,
-                                           double kappa, int64_t n, int x, int y, int z, double a[NOUT])
+// the fields of one node (0 for a set the lattice lacks)
+struct FieldNode {
+    double u[3], t;
+};
+
+struct Fields {
+    const double *__restrict__ dens, *__restrict__ u, *__restrict__ t;
+    int fluid, thermal;
+    __device__ __forceinline__ FieldNode at(int64_t n) const
+    {
+        FieldNode v;
+        v.u[0] = fluid ? u[3 * n] : 0.0;
+        v.u[1] = fluid ? u[3 * n + 1] : 0.0;
+        v.u[2] = fluid ? u[3 * n + 2] : 0.0;
+        v.t = thermal ? t[n] : 0.0;
+        return v;
+    }
+};
+
+__device__ __forceinline__ FieldNode centred(const FieldNode &p, const FieldNode &m, bool flat)
 {
-    const int NX = P.NX, NY = P.NY, NZ = P.NZ;
-    auto id = [&](int i, int j, int k) -> int64_t { return ((int64_t)k * NY + j) * NX + i; };
-    const int xp = wrapc(x + 1, NX), xm = wrapc(x - 1, NX);
-    const int yp = wrapc(y + 1, NY), ym = wrapc(y - 1, NY);
-    const int zp = wrapc(z + 1, NZ), zm = wrapc(z - 1, NZ);
+    FieldNode g;
+    for (int c = 0; c < 3; c++) g.u[c] = flat ? 0.0 : (p.u[c] - m.u[c]) / 2.0;
+    g.t = (p.t - m.t) / 2.0;
+    return g;
+}
+
+// y derivative at row y of column (x, z) from the rows next to it
+__device__ __forceinline__ FieldNode dy_at(const KParams &P, const Fields &F, const FieldNode &c, const FieldNode &m,
+                                           const FieldNode &p, int64_t n, int y)
+{
+    FieldNode g = centred(p, m, P.NY == 1);
+    if ((P.wall_f || P.wall_t) && P.NY >= 3 && (y == 0 || y == P.NY - 1)) {
+        const bool lo = y == 0;
+        const FieldNode e = F.at(lo ? n + 2 * (int64_t)P.NX : n - 2 * (int64_t)P.NX);
+        if (P.wall_f)
+            for (int k = 0; k < 3; k++)
+                g.u[k] = lo ? -1.5 * c.u[k] + 2.0 * p.u[k] - 0.5 * e.u[k] : 1.5 * c.u[k] - 2.0 * m.u[k] + 0.5 * e.u[k];
+        if (P.wall_t) g.t = lo ? -1.5 * c.t + 2.0 * p.t - 0.5 * e.t : 1.5 * c.t - 2.0 * m.t + 0.5 * e.t;
+    }
+    return g;
+}
+
+// Per-node terms of dump_averages (output.c:183-491) added into a[] in the
+// order of ch4g_output, from the node's fields and their derivatives.
+__device__ __forceinline__ void add_terms(const KParams &P, double nu, double kappa, double dens, const FieldNode &c,
+                                          const FieldNode &dx, const FieldNode &dy, const FieldNode &dz, int x, int y,
+                                          int z, double a[NTERM])
+{
+    const double ux = c.u[0], uy = c.u[1], uz = c.u[2];
     if (P.fluid) {
-        const double ux = u[3 * n], uy = u[3 * n + 1], uz = u[3 * n + 2];
         a[0] += (double)x + 0.5;
         a[1] += (double)y + 0.5;
         a[2] += (double)z + 0.5;
@@ -126,157 +197,230 @@ __device__ __forceinline__ void node_terms(const KParams &P, const double *__res
         a[6] += ux * ux;
         a[7] += uy * uy;
         a[8] += uz * uz;
-        a[9] += dens[n];
+        a[9] += dens;
         a[10] += 0.5 * (ux * ux + uy * uy + uz * uz);
-        a[12] += dens[n] * dens[n];
-        double G[3][3];  // G[c][d] = d u_c / d x_d
-        for (int c = 0; c < 3; c++) {
-            G[c][0] = (u[3 * id(xp, y, z) + c] - u[3 * id(xm, y, z) + c]) / 2.0;
-            G[c][1] = (u[3 * id(x, yp, z) + c] - u[3 * id(x, ym, z) + c]) / 2.0;
-            G[c][2] = (u[3 * id(x, y, zp) + c] - u[3 * id(x, y, zm) + c]) / 2.0;
-            if (P.wall_f && NY >= 3) {
-                if (y == 0)
-                    G[c][1] = -1.5 * u[3 * n + c] + 2.0 * u[3 * id(x, 1, z) + c] - 0.5 * u[3 * id(x, 2, z) + c];
-                if (y == NY - 1)
-                    G[c][1] = 1.5 * u[3 * n + c] - 2.0 * u[3 * id(x, NY - 2, z) + c] +
-                              0.5 * u[3 * id(x, NY - 3, z) + c];
-            }
-            if (NX == 1) G[c][0] = 0.0;
-            if (NY == 1) G[c][1] = 0.0;
-            if (NZ == 1) G[c][2] = 0.0;
-        }
+        a[12] += dens * dens;
         double e = 0.0;
-        for (int c = 0; c < 3; c++)
+        for (int i = 0; i < 3; i++) {
+            const double G[3] = {dx.u[i], dy.u[i], dz.u[i]}, H[3] = {i == 0 ? dx.u[0] : i == 1 ? dy.u[0] : dz.u[0],
+                                                                     i == 0 ? dx.u[1] : i == 1 ? dy.u[1] : dz.u[1],
+                                                                     i == 0 ? dx.u[2] : i == 1 ? dy.u[2] : dz.u[2]};
             for (int d = 0; d < 3; d++) {
-                double s = G[c][d] + G[d][c];
+                const double s = G[d] + H[d];
                 e += s * s;
             }
+        }
         a[11] += e * 0.5 * nu;
     }
     if (P.thermal) {
-        const double tn = t[n];
-        double gx = (t[id(xp, y, z)] - t[id(xm, y, z)]) / 2.0;
-        double gy = (t[id(x, yp, z)] - t[id(x, ym, z)]) / 2.0;
-        double gz = (t[id(x, y, zp)] - t[id(x, y, zm)]) / 2.0;
-        if (P.wall_t && NY >= 3) {
-            if (y == 0) gy = -1.5 * tn + 2.0 * t[id(x, 1, z)] - 0.5 * t[id(x, 2, z)];
-            if (y == NY - 1) gy = 1.5 * tn - 2.0 * t[id(x, NY - 2, z)] + 0.5 * t[id(x, NY - 3, z)];
-        }
-        double ux = 0.0, uy = 0.0, uz = 0.0;
-        if (P.fluid) {
-            ux = u[3 * n];
-            uy = u[3 * n + 1];
-            uz = u[3 * n + 2];
-        }
-        a[13] += tn;
-        a[14] += tn * tn;
+        const double t = c.t, gx = dx.t, gy = dy.t, gz = dz.t;
+        a[13] += t;
+        a[14] += t * t;
         a[15] += kappa * (gx * gx + gy * gy + gz * gz);
         a[16] += gx;
         a[17] += gy;
         a[18] += gz;
-        a[19] += ux * tn;
-        a[20] += uy * tn;
-        a[21] += uz * tn;
-        a[22] += -kappa * gx + ux * tn;
-        a[23] += -kappa * gy + uy * tn;
-        a[24] += -kappa * gz + uz * tn;
+        a[19] += ux * t;
+        a[20] += uy * t;
+        a[21] += uz * t;
+        a[22] += -kappa * gx + ux * t;
+        a[23] += -kappa * gy + uy * t;
+        a[24] += -kappa * gz + uz * t;
     }
 }
 
-__global__ void __launch_bounds__(RED_THREADS) k_averages(KParams P, const double *__restrict__ dens,
-                                                          const double *__restrict__ u,
-                                                          const double *__restrict__ t, double nu, double kappa,
-                                                          double *__restrict__ partials)
+// sum over the 64 lanes, the same in every lane
+__device__ __forceinline__ double wave_sum(double v)
 {
-    double a[NOUT];
-    for (int k = 0; k < NOUT; k++) a[k] = 0.0;
-    for (int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; n < P.N;
-         n += (int64_t)gridDim.x * blockDim.x) {
-        const int x = (int)(n % P.NX);
-        const int y = (int)((n / P.NX) % P.NY);
-        const int z = (int)(n / ((int64_t)P.NX * P.NY));
-        node_terms(P, dens, u, t, nu, kappa, n, x, y, z, a);
-    }
-    __shared__ double sh[RED_THREADS];
-    for (int k = 0; k < NOUT; k++) {
-        sh[threadIdx.x] = a[k];
-        __syncthreads();
-        for (int w = RED_THREADS / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) partials[(int64_t)blockIdx.x * NOUT + k] = sh[0];
-        __syncthreads();
-    }
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
 }
 
-__global__ void k_final(const double *__restrict__ partials, int nb, double *__restrict__ out)
+// Sums over parts of x-y planes.  PER_UNIT: out[unit] (z ruler); else
+// out[block], over every gridDim-th unit (averages).
+template <bool PER_UNIT>
+__global__ void __launch_bounds__(RED_THREADS) k_plane_sums(KParams P, Fields F, double nu, double kappa, PlaneWork w,
+                                                            double *__restrict__ out)
 {
-    const int k = threadIdx.x;
-    if (k >= NOUT) return;
-    double s = 0.0;
-    for (int b = 0; b < nb; b++) s += partials[(int64_t)b * NOUT + k];
-    out[k] = s;
-}
-
-// dump_averages rulers (output.c:212-491): block p sums the per-node terms of
-// plane p along AXIS (0: x = p, 1: y = p, 2: z = p) over its nodes, LDS tree
-// order, into out[p][NOUT].
-template <int AXIS>
-__global__ void __launch_bounds__(RED_THREADS) k_rulers(KParams P, const double *__restrict__ dens,
-                                                        const double *__restrict__ u, const double *__restrict__ t,
-                                                        double nu, double kappa, double *__restrict__ out)
-{
-    double a[NOUT];
-    for (int k = 0; k < NOUT; k++) a[k] = 0.0;
-    const int p = blockIdx.x;
     const int NX = P.NX, NY = P.NY, NZ = P.NZ;
-    const int64_t M = AXIS == 0 ? (int64_t)NY * NZ : (AXIS == 1 ? (int64_t)NX * NZ : (int64_t)NX * NY);
-    for (int64_t m = threadIdx.x; m < M; m += RED_THREADS) {
-        int x, y, z;
-        if (AXIS == 0) {
-            x = p;
-            y = (int)(m % NY);
-            z = (int)(m / NY);
-        } else if (AXIS == 1) {
-            x = (int)(m % NX);
-            y = p;
-            z = (int)(m / NX);
-        } else {
-            x = (int)(m % NX);
-            y = (int)(m / NX);
-            z = p;
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    double a[NTERM];
+    for (int k = 0; k < NTERM; k++) a[k] = 0.0;
+    const uint32_t first = xcd_block(blockIdx.x, gridDim.x);
+    for (int64_t unit = first; unit < w.units; unit += gridDim.x) {
+        const int z = (int)(unit / w.parts), task = (int)(unit - (int64_t)z * w.parts) * RED_WAVES + wave;
+        const int x = task % w.nxt * 64 + lane, y0 = task / w.nxt * w.rows, y1 = min(y0 + w.rows, NY);
+        if (x < NX && y0 < NY) {
+            const int64_t plane = (int64_t)z * NY * NX;
+            const int64_t dzp = (int64_t)(wrapc(z + 1, NZ) - z) * NY * NX, dzm = (int64_t)(wrapc(z - 1, NZ) - z) * NY * NX;
+            const int dxp = wrapc(x + 1, NX) - x, dxm = wrapc(x - 1, NX) - x;
+            FieldNode m = F.at(plane + (int64_t)wrapc(y0 - 1, NY) * NX + x), c = F.at(plane + (int64_t)y0 * NX + x);
+            for (int y = y0; y < y1; y++) {
+                const int64_t n = plane + (int64_t)y * NX + x;
+                const FieldNode p = F.at(plane + (int64_t)wrapc(y + 1, NY) * NX + x);
+                const FieldNode dx = centred(F.at(n + dxp), F.at(n + dxm), NX == 1);
+                const FieldNode dz = centred(F.at(n + dzp), F.at(n + dzm), NZ == 1);
+                add_terms(P, nu, kappa, P.fluid ? F.dens[n] : 0.0, c, dx, dy_at(P, F, c, m, p, n, y), dz, x, y, z, a);
+                m = c;
+                c = p;
+            }
         }
-        const int64_t n = ((int64_t)z * NY + y) * NX + x;
-        node_terms(P, dens, u, t, nu, kappa, n, x, y, z, a);
+        if constexpr (PER_UNIT) break;  // one unit per block
     }
-    __shared__ double sh[RED_THREADS];
-    for (int k = 0; k < NOUT; k++) {
-        sh[threadIdx.x] = a[k];
-        __syncthreads();
-        for (int w = RED_THREADS / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
+    __shared__ double sh[RED_WAVES][NTERM];
+    for (int k = 0; k < NTERM; k++) {
+        const double v = wave_sum(a[k]);
+        if (lane == 0) sh[wave][k] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < NOUT) {
+        double s = 0.0;
+        if (threadIdx.x < NTERM)
+            for (int i = 0; i < RED_WAVES; i++) s += sh[i][threadIdx.x];
+        out[(int64_t)first * NOUT + threadIdx.x] = s;
+    }
+}
+
+// columns of the x and y rulers: a block is RED_WAVES waves on consecutive
+// groups of `rows` rows, 64 x and zc planes
+struct ColumnWork {
+    int nxt, rows, nyb, zc, nzc;
+};
+
+static ColumnWork column_work(const KParams &P)
+{
+    ColumnWork w;
+    w.nxt = (P.NX + 63) / 64;
+    w.zc = P.NZ < 32 ? P.NZ : 32;
+    w.nzc = (P.NZ + w.zc - 1) / w.zc;
+    const int64_t blocks = (int64_t)w.nxt * ((P.NY + RED_WAVES - 1) / RED_WAVES) * w.nzc, r = blocks / 2048;
+    w.rows = (int)(r < 1 ? 1 : (r > 8 ? 8 : r));
+    w.nyb = (P.NY + RED_WAVES * w.rows - 1) / (RED_WAVES * w.rows);
+    return w;
+}
+
+// Sums along z, then over the rows of a block (px[yb * nzc + zi][x]) and over
+// the 64 x of a wave (py[xt * nzc + zi][y]).
+__global__ void __launch_bounds__(RED_THREADS) k_column_sums(KParams P, Fields F, double nu, double kappa,
+                                                             ColumnWork w, double *__restrict__ px,
+                                                             double *__restrict__ py)
+{
+    const int NX = P.NX, NY = P.NY, NZ = P.NZ;
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
+    const int xt = lb % w.nxt, yb = lb / w.nxt % w.nyb, zi = lb / w.nxt / w.nyb;
+    const int x = xt * 64 + lane, z0 = zi * w.zc, z1 = min(z0 + w.zc, NZ);
+    const int64_t plane = (int64_t)NX * NY;
+    double cx[NTERM];
+    for (int k = 0; k < NTERM; k++) cx[k] = 0.0;
+    for (int r = 0; r < w.rows; r++) {
+        const int y = (yb * RED_WAVES + wave) * w.rows + r;
+        if (y >= NY) break;
+        double a[NTERM];
+        for (int k = 0; k < NTERM; k++) a[k] = 0.0;
+        if (x < NX) {
+            const int64_t row = (int64_t)y * NX + x;
+            const int dxp = wrapc(x + 1, NX) - x, dxm = wrapc(x - 1, NX) - x;
+            const int64_t dyp = (int64_t)(wrapc(y + 1, NY) - y) * NX, dym = (int64_t)(wrapc(y - 1, NY) - y) * NX;
+            FieldNode m = F.at(row + wrapc(z0 - 1, NZ) * plane), c = F.at(row + z0 * plane);
+            for (int z = z0; z < z1; z++) {
+                const int64_t n = row + z * plane;
+                const FieldNode p = F.at(row + wrapc(z + 1, NZ) * plane);
+                const FieldNode dx = centred(F.at(n + dxp), F.at(n + dxm), NX == 1);
+                const FieldNode dy = dy_at(P, F, c, F.at(n + dym), F.at(n + dyp), n, y);
+                add_terms(P, nu, kappa, P.fluid ? F.dens[n] : 0.0, c, dx, dy, centred(p, m, NZ == 1), x, y, z, a);
+                m = c;
+                c = p;
+            }
         }
-        if (threadIdx.x == 0) out[(int64_t)p * NOUT + k] = sh[0];
+        double *o = py + ((int64_t)(xt * w.nzc + zi) * NY + y) * NOUT;
+        for (int k = 0; k < NTERM; k++) {
+            cx[k] += a[k];
+            const double v = wave_sum(a[k]);
+            if (lane == 0) o[k] = v;
+        }
+        if (lane == 0) o[NTERM] = 0.0;
+    }
+    // the block's waves, term by term
+    __shared__ double sh[RED_WAVES][64];
+    for (int k = 0; k < NTERM; k++) {
+        sh[wave][lane] = cx[k];
+        __syncthreads();
+        if (wave == 0 && x < NX) {
+            double s = 0.0;
+            for (int i = 0; i < RED_WAVES; i++) s += sh[i][lane];
+            px[((int64_t)(yb * w.nzc + zi) * NX + x) * NOUT + k] = s;
+        }
         __syncthreads();
     }
+    if (wave == 0 && x < NX) px[((int64_t)(yb * w.nzc + zi) * NX + x) * NOUT + NTERM] = 0.0;
+}
+
+// out[p] = sum of the `count` records in[p * pstride + i * istride] (records
+// of NOUT doubles; 32 lanes a record, 32 records at a time, then a tree)
+constexpr int SUM_ROWS = 32;
+__global__ void __launch_bounds__(32 * SUM_ROWS) k_sum_records(const double *__restrict__ in, int64_t count,
+                                                               int64_t istride, int64_t pstride,
+                                                               double *__restrict__ out)
+{
+    const int k = threadIdx.x % 32, r = threadIdx.x / 32;
+    const double *p = in + (int64_t)blockIdx.x * pstride * NOUT;
+    double s = 0.0;
+    if (k < NOUT) {
+        // eight loads in flight: one at a time, 2048 records take 30 us
+        int64_t i = r;
+        for (; i + 7 * SUM_ROWS < count; i += 8 * SUM_ROWS) {
+            double v[8];
+            for (int j = 0; j < 8; j++) v[j] = p[(i + j * SUM_ROWS) * istride * NOUT + k];
+            for (int j = 0; j < 8; j++) s += v[j];
+        }
+        for (; i < count; i += SUM_ROWS) s += p[i * istride * NOUT + k];
+    }
+    __shared__ double sh[SUM_ROWS][32];
+    sh[r][k] = s;
+    for (int h = SUM_ROWS / 2; h > 0; h >>= 1) {
+        __syncthreads();
+        if (r < h) sh[r][k] += sh[r + h][k];
+    }
+    if (r == 0 && k < NOUT) out[(int64_t)blockIdx.x * NOUT + k] = sh[0][k];
+}
+
+size_t ruler_scratch_doubles(const KParams &P)
+{
+    const ColumnWork c = column_work(P);
+    const int64_t planes = plane_work(P).units;
+    const int64_t cols = (int64_t)c.nzc * ((int64_t)c.nyb * P.NX + (int64_t)c.nxt * P.NY);
+    return (size_t)(planes > cols ? planes : cols) * NOUT;
 }
 
 void launch_rulers(const KParams &P, const double *dens, const double *u, const double *t, double nu, double kappa,
-                   double *rx, double *ry, double *rz, hipStream_t s)
+                   double *scratch, double *rx, double *ry, double *rz, hipStream_t s)
 {
-    if (rx) hipLaunchKernelGGL(k_rulers<0>, dim3(P.NX), dim3(RED_THREADS), 0, s, P, dens, u, t, nu, kappa, rx);
-    if (ry) hipLaunchKernelGGL(k_rulers<1>, dim3(P.NY), dim3(RED_THREADS), 0, s, P, dens, u, t, nu, kappa, ry);
-    if (rz) hipLaunchKernelGGL(k_rulers<2>, dim3(P.NZ), dim3(RED_THREADS), 0, s, P, dens, u, t, nu, kappa, rz);
+    const Fields F{dens, u, t, P.fluid, P.thermal};
+    const dim3 sum(32 * SUM_ROWS);
+    if (rz) {
+        const PlaneWork w = plane_work(P);
+        hipLaunchKernelGGL(k_plane_sums<true>, dim3((unsigned)w.units), dim3(RED_THREADS), 0, s, P, F, nu, kappa, w,
+                           scratch);
+        hipLaunchKernelGGL(k_sum_records, dim3(P.NZ), sum, 0, s, scratch, w.parts, 1, w.parts, rz);
+    }
+    if (rx || ry) {
+        const ColumnWork w = column_work(P);
+        double *px = scratch, *py = scratch + (int64_t)w.nyb * w.nzc * P.NX * NOUT;
+        hipLaunchKernelGGL(k_column_sums, dim3((unsigned)w.nxt * w.nyb * w.nzc), dim3(RED_THREADS), 0, s, P, F, nu,
+                           kappa, w, px, py);
+        if (rx) hipLaunchKernelGGL(k_sum_records, dim3(P.NX), sum, 0, s, px, (int64_t)w.nyb * w.nzc, P.NX, 1, rx);
+        if (ry) hipLaunchKernelGGL(k_sum_records, dim3(P.NY), sum, 0, s, py, (int64_t)w.nxt * w.nzc, P.NY, 1, ry);
+    }
 }
 
 void launch_averages(const KParams &P, const double *dens, const double *u, const double *t, double nu, double kappa,
                      double *partials, double *result, hipStream_t s)
 {
-    int nb = reduce_blocks(P);
-    hipLaunchKernelGGL(k_averages, dim3(nb), dim3(RED_THREADS), 0, s, P, dens, u, t, nu, kappa, partials);
-    hipLaunchKernelGGL(k_final, dim3(1), dim3(64), 0, s, partials, nb, result);
+    const int nb = reduce_blocks(P);
+    hipLaunchKernelGGL(k_plane_sums<false>, dim3(nb), dim3(RED_THREADS), 0, s, P, Fields{dens, u, t, P.fluid, P.thermal},
+                       nu, kappa, plane_work(P), partials);
+    hipLaunchKernelGGL(k_sum_records, dim3(1), dim3(32 * SUM_ROWS), 0, s, partials, nb, 1, 0, result);
 }
 
 }  // namespace ch4g

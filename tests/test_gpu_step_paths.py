@@ -48,3 +48,23 @@ def test_streamed_block_order(shape, precision):
         print(f"  {shape}: L2 rel err of u {err:.2e}")
         assert err <= 1e-5
     lat.close()
+
+
+# The averages' and rulers' marches: fewer rows, columns or planes than one
+# wave covers, a last wave, row group, z chunk and unit that are partial
+# (1 x 300 x 2048: 16 rows per wave of the plane sums, two of the column sums,
+# several units per block).  Tolerance: sums of up to N terms in another
+# order, N eps of the largest member (614400 * 2.2e-16 = 1.4e-10 at most).
+@pytest.mark.parametrize("shape", [(3, 5, 2), (64, 3, 1), (65, 7, 33), (130, 41, 70), (1, 300, 2048)], ids=str)
+def test_diagnostics_at_partial_waves(shape):
+    cfg = configs.rb2d(*shape, Ra=1e4, seed=9, noise=0.05)
+    o, lat = run(Oracle(cfg), 3), run(Lattice(cfg), 3)
+    eps = cfg.nodes() * 2.3e-16
+    got, want = lat.dump_averages(), o.dump_averages()
+    flux = max(abs(want[k]) for k in want if k not in ("x", "y", "z"))
+    for k in want:
+        assert abs(got[k] - want[k]) <= eps * max(abs(want[k]), flux), (k, got[k], want[k])
+    for r, w in zip(lat.dump_rulers(), o.dump_rulers()[1:]):
+        a, b = r.view(np.float64).reshape(len(r), -1), w.view(np.float64).reshape(len(w), -1)
+        assert np.abs(a - b).max() <= eps * np.abs(b).max()
+    lat.close()
