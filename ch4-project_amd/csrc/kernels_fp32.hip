@@ -1499,19 +1499,41 @@ using TZ_ = TileZ<FL, TH, TX, TY, HOLD>;
 // flight during step B 6.5, 32 x 5 all in LDS (two blocks per CU) 7.3,
 // 64 x 8 held 6.0, the same through buffer resources 5.6-5.9; 3-D channel
 // 256^3: single 0.46, 64 x 8 held 0.35.  Double arithmetic needs more
-// registers than an 11-wave block allows: 64 x 4.  z ranges: at least 1024
-// blocks (four per CU) and at most 128 planes (channel 192^3 with ranges of
-// 128 planes: 144 blocks, 0.30 ms; of 32 planes: 0.18 ms).
+// registers than an 11-wave block allows: 64 x 4.
+//
+// z ranges: a CU holds one block (LDS), and a block of zc planes takes zc + 2
+// iterations of the same length, so the launch takes ceil(blocks / 256) (zc +
+// 2) of them: the most ranges that 1 to 8 full rounds of blocks hold, whichever
+// makes this least.  us per step, at least 1024 blocks of at most 128 planes
+// (before) -> this: channel 128^3 49.8 -> 47.6 (16 planes), 192^3 188 -> 158
+// (28); Rayleigh-Benard 128^3 93.4 -> 89.5, 192^3 351 -> 302, 256^3 703 -> 658
+// (128), 320^3 1543 -> 1410, 192x120x280 323 -> 288 (26), 320x100x90 168 ->
+// 138 (13), 512^3 5640 -> 5640 (256); double arithmetic 256^3 975 -> 911.
+static int z_range(int64_t columns, int NZ)
+{
+    constexpr int64_t CUS = 256;
+    int64_t best = 0, zbest = NZ;
+    for (int64_t round = 1; round <= 8; round++) {
+        const int64_t most = (NZ + 3) / 4, fit = round * CUS / columns;
+        const int64_t r = fit < 1 ? 1 : (fit > most ? most : fit);
+        const int64_t zc = (NZ + r - 1) / r, blocks = columns * ((NZ + zc - 1) / zc);
+        const int64_t cost = (blocks + CUS - 1) / CUS * (zc + 2);
+        // (more blocks even out the rounds: taken at half a percent more)
+        if (round == 1 || cost * 200 <= best * 201) {
+            best = cost;
+            zbest = zc;
+        }
+    }
+    return (int)zbest;
+}
+
 void launch_two_steps_3d(const KParams &P, const float *fin, const float *gin, float *fout, float *gout,
                          const float *tl_in, float *tl_out, hipStream_t s)
 {
     const bool tall = P.fluid && !(P.thermal && P.arith64);
     const int TY = tall ? 8 : 4;
     const int64_t columns = (int64_t)((P.NX + 63) / 64) * ((P.NY + TY - 1) / TY);
-    int64_t zc = (int64_t)P.NZ * columns / 1024;
-    zc = zc < 8 ? 8 : (zc > 128 ? 128 : zc);
-    zc = zc > P.NZ ? P.NZ : zc;
-    const int z = (int)zc;
+    const int z = z_range(columns, P.NZ);
 #define Z2(...) launch_z2<TZ_<__VA_ARGS__>>(P, fin, gin, fout, gout, tl_in, tl_out, z, s)
     if (P.fluid && P.thermal) {
         if (P.arith64)
