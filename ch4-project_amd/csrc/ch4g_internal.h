@@ -415,11 +415,12 @@ inline int64_t batch2_tiles(int NX, int NY) { return (int64_t)((NX + 63) / 64) *
 // arithmetic, FP64) listed in its slots
 // population sets of a batched launch (one kernel instance per kind)
 enum { BATCH_FLUID = 1, BATCH_THERMAL = 2, BATCH_FLUID_THERMAL = 3 };
-// gen: some lattice of the launch uses the HIT / LES / two-way paths
+// gen: some lattice of the launch uses the HIT / LES / two-way paths; buf
+// (FP64): every lattice's planes are within the reach of buffer resources
 void launch_batch_fp32(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
                        bool dense, bool gen, int arith64, StepOrder order, hipStream_t s);
 void launch_batch_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
-                       bool dense, StepOrder order, hipStream_t s);
+                       bool dense, bool gen, bool buf, StepOrder order, hipStream_t s);
 // two steps per launch for 2-D float-storage lattices (two_step_ok); nblocks
 // = 64 x 4 tiles of the launch
 void launch_batch2_fp32(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,

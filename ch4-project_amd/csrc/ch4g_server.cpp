@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "ch4g_lattice.h"
+#include "ch4g_planes.h"
 
 using namespace ch4g;
 
@@ -32,6 +33,7 @@ struct Batch {
         int dev32, arith64, kind;
         bool dense;                       // lanes decode their own rows (dense_rows)
         bool gen;                         // LES lattices (the kernel instance with those paths)
+        bool buf;                         // planes within the reach of buffer resources (FP64)
         StepOrder order;                  // block order and stores, by the group's state bytes
         bool two;                         // two steps per launch (k_step2_batch32)
         int first, count;                 // range in the entry table
@@ -170,6 +172,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         G.count = 0;
         int64_t bytes = 0;
         bool whole_lines = true;
+        G.buf = true;
         // members of the group and their launches per chunk (two-step
         // groups: pairs, then the single step of an odd share)
         size_t i1 = i;
@@ -206,6 +209,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
             npair.push_back(G.two ? st / 2 : 0);
             ntile.push_back(G.two ? batch2_tiles(L->cfg.NX, L->cfg.NY) : batch_tiles(L->cfg.NX, L->cfg.NY, L->cfg.NZ));
             bytes += 2 * (int64_t)Q * L->N * (L->dev32 ? 4 : 8) * ((L->base.fluid ? 1 : 0) + (L->base.thermal ? 1 : 0));
+            G.buf = G.buf && planes_ok(L->base, 8);
             whole_lines = whole_lines && (G.dense || L->cfg.NX * (L->dev32 ? 4 : 8) % 128 == 0);
             G.count++;
         }
@@ -326,7 +330,7 @@ int launch_steps(Batch &B)
             else if (G.dev32)
                 launch_batch_fp32(tab, sl, ns, nb, G.kind, G.dense, G.gen, G.arith64, G.order, st);
             else
-                launch_batch_fp64(tab, sl, ns, nb, G.kind, G.dense, G.order, st);
+                launch_batch_fp64(tab, sl, ns, nb, G.kind, G.dense, G.gen, G.buf, G.order, st);
         }
     }
     for (size_t g = 1; g < ng; g++) {

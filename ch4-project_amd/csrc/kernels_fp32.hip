@@ -14,7 +14,7 @@
 //   df*   = df - (df - df_eq)/tau + (1 - 1/(2 tau)) w rho (3 (c-u).F + 9 (c.u)(c.F))
 // and the same for the temperature (T = T_b + dT, no forcing term).  Step
 // semantics (lag scalar, wall rules, force lag) are those of kernels_fp64.hip.
-#include "ch4g_internal.h"
+#include "ch4g_planes.h"
 
 namespace ch4g {
 
@@ -877,40 +877,8 @@ struct RawNode {
     float f[Q], g[Q], tl;
 };
 
-// The Q planes of a population array as three buffer resources of up to
-// seven planes each: a plane is addressed by the resource of its group, a
-// scalar offset of its place in the group and the node's 32-bit byte offset
-// (planes of less than 4 GiB / 7).  Keeps the scalar registers free of 38
-// 64-bit plane addresses and the vector registers of 64-bit lane addresses.
-struct Planes {
-    __amdgpu_buffer_rsrc_t r[3];
-    uint32_t pb;  // plane stride in bytes
-};
-
-__device__ __forceinline__ Planes make_planes(const float *base, int64_t S)
-{
-    Planes p;
-    p.pb = (uint32_t)(S * 4);
-    static_for<0, 3>([&](auto gc) {
-        constexpr int gi = decltype(gc)::value;
-        constexpr int np = gi < 2 ? 7 : Q - 14;
-        p.r[gi] = __builtin_amdgcn_make_buffer_rsrc((void *)(base + (size_t)gi * 7 * (size_t)S), (short)0,
-                                                    (int)(uint32_t)((uint64_t)np * p.pb), 0x00020000);
-    });
-    return p;
-}
-
-// cache-policy bits of buffer instructions: non-temporal
-constexpr int CPOL_NT = 2;
-
-template <int q>
-__device__ __forceinline__ float bload(const Planes &p, uint32_t soff, uint32_t voff)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(p.r[q / 7], (int)voff, (int)soff, 0));
-}
-
 template <bool FLUID, bool THERMAL>
-__device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, const Planes &pf, const Planes &pg,
+__device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, const Planes<float> &pf, const Planes<float> &pg,
                                              const float *__restrict__ tl_in, uint32_t n, RawNode &r)
 {
     const uint32_t n4 = n * 4u;
@@ -919,14 +887,14 @@ __device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, con
         static_for<0, Q>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             const bool cross = P.wall_t && crosses_wall<q>(b);
-            r.g[q] = bload<q>(pg, (uint32_t)(q % 7) * pg.pb, cross ? n4 : src_index<q>(b, P.NX, P.NY) * 4u);
+            r.g[q] = plane_load<q>(pg, cross ? n4 : src_index<q>(b, P.NX, P.NY) * 4u, 0u);
         });
     }
     if constexpr (FLUID) {
         static_for<0, Q>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             if constexpr (cyq(q) == 0) {
-                r.f[q] = bload<q>(pf, (uint32_t)(q % 7) * pf.pb, src_index<q>(b, P.NX, P.NY) * 4u);
+                r.f[q] = plane_load<q>(pf, src_index<q>(b, P.NX, P.NY) * 4u, 0u);
             } else {
                 // bounce-back reads the opposite plane (same group of seven)
                 constexpr int iq = q % 7, ii = invq(q) % 7, mn = iq < ii ? iq : ii;
@@ -934,7 +902,7 @@ __device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, con
                 const bool cross = P.wall_f && crosses_wall<q>(b);
                 const uint32_t voff = cross ? n4 + (uint32_t)(ii - mn) * pf.pb
                                             : src_index<q>(b, P.NX, P.NY) * 4u + (uint32_t)(iq - mn) * pf.pb;
-                r.f[q] = bload<q>(pf, (uint32_t)mn * pf.pb, voff);
+                r.f[q] = plane_load<q / 7 * 7 + mn>(pf, voff, 0u);
             }
         });
     }
@@ -942,27 +910,21 @@ __device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, con
 
 // NodeOut through buffer resources (non-temporal stores)
 struct BufOut {
-    Planes f, g;
+    Planes<float> f, g;
     float *__restrict__ tlag;
     uint32_t n, n4;
-    template <int q>
-    __device__ void st(const Planes &p, float v) const
-    {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), p.r[q / 7], (int)n4,
-                                              (int)((uint32_t)(q % 7) * p.pb), CPOL_NT);
-    }
     __device__ void put_f(int q, float v) const
     {
         static_for<0, Q>([&](auto qc) {
             constexpr int qq = decltype(qc)::value;
-            if (qq == q) st<qq>(f, v);
+            if (qq == q) plane_store<qq, true>(f, n4, 0u, v);
         });
     }
     __device__ void put_g(int q, float v) const
     {
         static_for<0, Q>([&](auto qc) {
             constexpr int qq = decltype(qc)::value;
-            if (qq == q) st<qq>(g, v);
+            if (qq == q) plane_store<qq, true>(g, n4, 0u, v);
         });
     }
     __device__ void put_tlag(float v) const { tlag[n] = v; }
@@ -1095,7 +1057,7 @@ __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp32(KParams P, const fl
         b = make_nbr(xa, ya, za, NX, NY, NZ);
     };
     const int nit = ze - zb + 2;
-    Planes pin_f, pin_g, pout_f, pout_g;
+    Planes<float> pin_f, pin_g, pout_f, pout_g;
     if constexpr (FLUID) {
         pin_f = make_planes(fin, P.S);
         pout_f = make_planes(fout, P.S);

@@ -13,7 +13,7 @@
 // rho, u, T of step s-1 (lb.c:420-540; the u shift uses the force built from
 // the lagged temperature, as main.c's ordering implies), then collides
 // (fluid.c:1033-1225) and adds the Guo term (forcing.c:1424-1435) of step s.
-#include "ch4g_internal.h"
+#include "ch4g_planes.h"
 
 namespace ch4g {
 
@@ -38,14 +38,17 @@ __device__ __forceinline__ double m_z(const double *p)
 
 // build_forcing for one node (forcing.c:361-667), terms added in source order;
 // with NOZEROMODE the mean of those terms is removed (forcing.c:1123-1152)
-// before the particle feedback is added (main.c:118-131).
+// before the particle feedback is added (main.c:118-131).  GEN: the HIT,
+// NOZEROMODE and two-way terms are compiled in (with the LES closures of the
+// step); lattices without them run an instance without their registers.
+template <bool GEN = true>
 __device__ __forceinline__ void force_at(const KParams &P, const HitTable &tab, const double *fb, const double *f0,
                                          uint32_t n, int x, int y, int z, double T, double F[3])
 {
     F[0] = P.Fc[0];
     F[1] = P.Fc[1];
     F[2] = P.Fc[2];
-    if (P.hit) {
+    if (GEN && P.hit) {
 #pragma unroll
         for (int ii = 0; ii < CH4G_HIT_NK; ii++) {
             double ax = tab.sx[ii * P.NX + x];
@@ -64,12 +67,12 @@ __device__ __forceinline__ void force_at(const KParams &P, const HitTable &tab, 
         F[1] += fac * P.grav[1];
         F[2] += fac * P.grav[2];
     }
-    if (f0) {
+    if (GEN && f0) {
         F[0] -= f0[0];
         F[1] -= f0[1];
         F[2] -= f0[2];
     }
-    if (P.twoway) {
+    if (GEN && P.twoway) {
         const size_t N = (size_t)P.N;
         F[0] += fb[n];
         F[1] += fb[N + n];
@@ -128,44 +131,147 @@ __device__ __forceinline__ void gather_thermal(const KParams &P, const Nbr &b, c
     });
 }
 
-// population stores: non-temporal (NT) where step_order says so
-template <bool NT>
-__device__ __forceinline__ void stp64(double *p, double v)
+// the same gathers through buffer resources
+template <int UNI>
+__device__ __forceinline__ void pull_fluid64(const KParams &P, const Nbr &b, const Planes<double> &in,
+                                             const Pull<double, UNI> &o, double f[Q])
 {
-    if constexpr (NT)
-        __builtin_nontemporal_store(v, p);
-    else
-        *p = v;
+    static_for<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        f[q] = pull_fluid<q>(in, o, P.wall_f && crosses_wall<q>(b));
+    });
 }
 
-// equilibrium (lb.c:382-415)
-__device__ __forceinline__ double feq_q(const KParams &P, int q, double rho, double ux, double uy, double uz,
-                                        double u2)
+template <int UNI>
+__device__ __forceinline__ void pull_thermal64(const KParams &P, const Nbr &b, const Planes<double> &in,
+                                               const Pull<double, UNI> &o, double Tlag, double g[Q])
 {
-    double cu = ((double)cxq(q) * ux + (double)cyq(q) * uy + (double)czq(q) * uz);
-    return rho * wq(q) * (1.0 + P.invcs2 * cu + P.invtwocs4 * cu * cu - P.invtwocs2 * u2);
+    const double fac_top = 2.0 * (P.Tw_top - Tlag);
+    const double fac_bot = 2.0 * (P.Tw_bot - Tlag);
+    static_for<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        const bool cross = P.wall_t && crosses_wall<q>(b);
+        const double v = pull_thermal<q>(in, o, cross);
+        if constexpr (cyq(q) > 0)
+            g[q] = cross ? v + wq(q) * fac_bot : v;
+        else if constexpr (cyq(q) < 0)
+            g[q] = cross ? v + wq(q) * fac_top : v;
+        else
+            g[q] = v;
+    });
+}
+
+// Where a node's populations go, through buffer resources or (flat) plane
+// pointers; non-temporal (NT) where step_order says so.
+template <bool NT, int UNI>
+struct PlaneOut {
+    Planes<double> p;
+    Pull<double, UNI> o;
+    template <int q>
+    __device__ void put(double v) const
+    {
+        plane_store<q, NT>(p, o.template voff<0>(), o.template soff<0>(), v);
+    }
+};
+template <bool NT>
+struct FlatOut {
+    double *__restrict__ p;
+    size_t S;
+    uint32_t n;
+    template <int q>
+    __device__ void put(double v) const
+    {
+        double *a = p + (size_t)q * S + n;
+        if constexpr (NT)
+            __builtin_nontemporal_store(v, a);
+        else
+            *a = v;
+    }
+};
+
+// equilibrium (lb.c:382-415) of the opposite pair (q, inv q), and c.u of q:
+//   rho w (1 + c.u / cs^2 + (c.u)^2 / (2 cs^4) - u^2 / (2 cs^2)),
+// in the reference's order.  Products by a velocity component 0 or +-1 are
+// left out: c.u is one or two signed terms, and c.u of the opposite direction
+// its negative, both exact (an IEEE sum with a zero term, and of negated
+// terms, is the same number; the sign of a zero c.u cannot reach the result).
+// The zero products do one thing: a velocity that is not finite makes every
+// population NaN.  u2z carries that (u2 + 0 ux + 0 uy + 0 uz).
+// With the products, the general force paths and 64-bit lane addresses in one
+// kernel a wave ran 2068 vector instructions (1473 FP64) per node; this
+// instance 751 (680).  us per step: Rayleigh-Benard 256x128 9.8 -> 6.1,
+// 512x256 14.8 -> 12.7, 64^3 25.6 -> 24.1; channel 4x64x4 4.56 -> 3.83, 64^3
+// 14.5 -> 12.8; larger lattices are bound by memory and stay (256^3 1.0 x).
+template <int q>
+__device__ __forceinline__ double cdot64(double x, double y, double z)
+{
+    constexpr int a = cxq(q), b = cyq(q), c = czq(q);
+    const double tx = a > 0 ? x : -x, ty = b > 0 ? y : -y, tz = c > 0 ? z : -z;
+    if constexpr (a != 0 && b != 0)
+        return tx + ty;
+    else if constexpr (a != 0 && c != 0)
+        return tx + tz;
+    else if constexpr (b != 0 && c != 0)
+        return ty + tz;
+    else
+        return a != 0 ? tx : (b != 0 ? ty : tz);
+}
+
+__device__ __forceinline__ double u2_of(double ux, double uy, double uz)
+{
+    const double u2 = (ux * ux + uy * uy + uz * uz);
+    return u2 + (0.0 * ux + 0.0 * uy + 0.0 * uz);
+}
+
+// representative q of the k-th opposite pair
+__host__ __device__ constexpr int pair64(int k)
+{
+    constexpr int v[9] = {1, 3, 5, 7, 8, 11, 12, 15, 16};
+    return v[k];
+}
+
+struct EqPair {
+    double cu, eq, eqb;  // c_q.u, equilibrium of q and of inv q
+};
+template <int q>
+__device__ __forceinline__ EqPair feq_pair(const KParams &P, double rho, double ux, double uy, double uz, double u2z)
+{
+    EqPair e;
+    e.cu = cdot64<q>(ux, uy, uz);
+    const double a = P.invcs2 * e.cu, b = P.invtwocs4 * e.cu * e.cu, c = P.invtwocs2 * u2z, rw = rho * wq(q);
+    e.eq = rw * (1.0 + a + b - c);
+    e.eqb = rw * (1.0 - a + b - c);
+    return e;
+}
+__device__ __forceinline__ double feq_rest(const KParams &P, double rho, double u2z)
+{
+    return rho * wq(0) * (1.0 - P.invtwocs2 * u2z);
 }
 
 // tau_u_les, local-strain branch (les.c:20-30,:144-180,:253) with the
 // stress_tensor assignments of gradients.c:42-69.
 __device__ __forceinline__ double les_tau(const KParams &P, const double f[Q], double rho, double ux, double uy,
-                                          double uz, double u2, double tau_prev)
+                                          double uz, double u2z, double tau_prev)
 {
-    double xx = 0.0, yy = 0.0, zz = 0.0, xy = 0.0, xz = 0.0, yz = 0.0;
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-        double d = f[q] - feq_q(P, q, rho, ux, uy, uz, u2);
-        const double cx = cxq(q), cy = cyq(q), cz = czq(q);
-        xx += cx * cx * d;
-        yy += cy * cy * d;
-        zz += cz * cz * d;
-        xy += cx * cy * d;
-        xz += cx * cz * d;
-        yz += cy * cz * d;
-    }
-    (void)zz;
+    double d[Q];
+    static_for<0, 9>([&](auto kk) {
+        constexpr int q = pair64(decltype(kk)::value), qb = invq(q);
+        const EqPair e = feq_pair<q>(P, rho, ux, uy, uz, u2z);
+        d[q] = f[q] - e.eq;
+        d[qb] = f[qb] - e.eqb;
+    });
+    // sums over q in order; terms with a zero factor left out as above
+    double xx = 0.0, yy = 0.0, xy = 0.0, xz = 0.0, yz = 0.0;
+    static_for<1, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value, cx = cxq(q), cy = cyq(q), cz = czq(q);
+        if constexpr (cx != 0) xx += d[q];
+        if constexpr (cy != 0) yy += d[q];
+        if constexpr (cx * cy != 0) xy += cx * cy > 0 ? d[q] : -d[q];
+        if constexpr (cx * cz != 0) xz += cx * cz > 0 ? d[q] : -d[q];
+        if constexpr (cy * cz != 0) yz += cy * cz > 0 ? d[q] : -d[q];
+    });
     const double yx = xy, zx = 0.0, zy = yz;
-    zz = xz;
+    const double zz = xz;
     double fac = -1.0 / (2 * P.cs2 * rho * tau_prev * 1.0);
     double s_norm = fabs(fac) * sqrt(2.0 * (xx * xx + xy * xy + xz * xz + yx * yx + yy * yy + yz * yz + zx * zx +
                                             zy * zy + zz * zz));
@@ -218,13 +324,14 @@ __device__ __forceinline__ double les_tau_t(const KParams &P, double tau_les)
 
 // hydro_fields of the previous step for one node (lb.c:420-540): density and
 // velocity with the half force built from the lagged temperature.
+template <bool GEN = true>
 __device__ __forceinline__ void fluid_velocity64(const KParams &P, const double f[Q], uint32_t n, int x, int y, int z,
                                                  double Tlag, double &rho, double &ux, double &uy, double &uz)
 {
     rho = m_sum(f);
     if (P.forced) {
         double Fp[3];
-        force_at(P, P.hit_prev, P.fb_prev, P.f0p, n, x, y, z, Tlag, Fp);
+        force_at<GEN>(P, P.hit_prev, P.fb_prev, P.f0p, n, x, y, z, Tlag, Fp);
         ux = m_x(f) / rho + 0.5 * 1.0 * Fp[0];
         uy = m_y(f) / rho + 0.5 * 1.0 * Fp[1];
         uz = m_z(f) / rho + 0.5 * 1.0 * Fp[2];
@@ -235,82 +342,126 @@ __device__ __forceinline__ void fluid_velocity64(const KParams &P, const double 
     }
 }
 
-// One node of the fused step (shared by the single-lattice and the batched
-// kernels, so a lattice advances bit-identically in either).
-template <bool FIRST, bool FLUID, bool THERMAL, bool NT>
-__device__ __forceinline__ void step_node64(const KParams &P, const double *__restrict__ fin,
-                                            const double *__restrict__ gin, double *__restrict__ fout,
-                                            double *__restrict__ gout, double *__restrict__ tlag,
-                                            double *__restrict__ taules, int x, int y, int z, uint32_t n)
+// Collision and force of one node's gathered populations f (and g, of sum T);
+// shared by every step kernel, so a lattice advances bit-identically in all.
+template <bool FLUID, bool THERMAL, bool GEN, class OutF, class OutG>
+__device__ __forceinline__ void collide64(const KParams &P, const Nbr &b, const double f[Q], const double g[Q],
+                                          double Tlag, double T, double *__restrict__ taules, uint32_t n,
+                                          const OutF &outf, const OutG &outg)
 {
-    const size_t N = (size_t)P.S;  // plane stride
-    const Nbr b = make_nbr(x, y, z, P.NX, P.NY, P.NZ);
-
-    double Tlag = 0.0, T = 0.0;
-    double g[Q], f[Q];
-    if constexpr (THERMAL) {
-        Tlag = tlag[n];
-        gather_thermal<FIRST>(P, b, gin, n, Tlag, g);
-    }
-    if constexpr (FLUID) gather_fluid<FIRST>(P, b, fin, n, f);
-    if constexpr (THERMAL) T = m_sum(g);
-
+    const int x = b.x, y = b.y, z = b.z;
     double ux = 0.0, uy = 0.0, uz = 0.0;
     double tau_les = 0.0;
     if constexpr (FLUID) {
         double rho;
-        fluid_velocity64(P, f, n, x, y, z, Tlag, rho, ux, uy, uz);
-        const double u2 = (ux * ux + uy * uy + uz * uz);
+        fluid_velocity64<GEN>(P, f, n, x, y, z, Tlag, rho, ux, uy, uz);
+        const double u2z = u2_of(ux, uy, uz);
         double invtau = P.invtau_u;
-        if (P.les) {
+        if (GEN && P.les) {
             if (P.les_fd) {
                 tau_les = les_tau_fd(P, (const double *)P.vel, b, n);
             } else {
                 double tau_prev = (P.itime == 1) ? P.tau_u : taules[n];
-                tau_les = les_tau(P, f, rho, ux, uy, uz, u2, tau_prev);
+                tau_les = les_tau(P, f, rho, ux, uy, uz, u2z, tau_prev);
             }
             taules[n] = tau_les;
             invtau = 1.0 / tau_les;
         }
         double Fn[3] = {0.0, 0.0, 0.0};
-        if (P.forced) force_at(P, P.hit_now, P.fb_now, P.f0n, n, x, y, z, T, Fn);
+        if (P.forced) force_at<GEN>(P, P.hit_now, P.fb_now, P.f0n, n, x, y, z, T, Fn);
+        // r += guo w rho F . ((c - u) / cs^2 + c (c.u) / cs^4), components in
+        // order; s = +1 for q, -1 for its opposite (c (c.u) is the same for both)
+        const double gf[3] = {P.guo_fac * wq(0) * rho, P.guo_fac * wq(1) * rho, P.guo_fac * wq(7) * rho};
+        auto guo = [&](auto qc, double s, double cc, double &r) {
+            constexpr int q = decltype(qc)::value, wc = q == 0 ? 0 : (q <= 6 ? 1 : 2);
+            constexpr int c[3] = {cxq(q), cyq(q), czq(q)};
+            const double u[3] = {ux, uy, uz};
 #pragma unroll
-        for (int q = 0; q < Q; q++) {
-            double r = f[q];
-            double fcoll = -invtau * (f[q] - feq_q(P, q, rho, ux, uy, uz, u2));
-            r += fcoll;
-            if (P.forced) {
-                const double cx = cxq(q), cy = cyq(q), cz = czq(q);
-                double cu = (cx * ux + cy * uy + cz * uz);
-                double dx = (cx - ux) * P.invcs2 + cx * cu * P.invcs4;
-                double dy = (cy - uy) * P.invcs2 + cy * cu * P.invcs4;
-                double dz = (cz - uz) * P.invcs2 + cz * cu * P.invcs4;
-                r += P.guo_fac * wq(q) * rho * Fn[0] * dx;
-                r += P.guo_fac * wq(q) * rho * Fn[1] * dy;
-                r += P.guo_fac * wq(q) * rho * Fn[2] * dz;
+            for (int a = 0; a < 3; a++) {
+                const double ca = c[a] * s;  // 0 or +-1, known at compile time
+                double d = (ca - u[a]) * P.invcs2;
+                if (c[a] != 0) d += c[a] > 0 ? cc : -cc;
+                r += gf[wc] * Fn[a] * d;
             }
-            stp64<NT>(fout + (size_t)q * N + n, r);
+        };
+        {
+            double r = f[0];
+            r += -invtau * (f[0] - feq_rest(P, rho, u2z));
+            if (P.forced) guo(std::integral_constant<int, 0>{}, 1.0, 0.0, r);
+            outf.template put<0>(r);
         }
+        static_for<0, 9>([&](auto kk) {
+            constexpr int q = pair64(decltype(kk)::value), qb = invq(q);
+            const EqPair e = feq_pair<q>(P, rho, ux, uy, uz, u2z);
+            double r = f[q], rb = f[qb];
+            r += -invtau * (f[q] - e.eq);
+            rb += -invtau * (f[qb] - e.eqb);
+            if (P.forced) {
+                const double cc = e.cu * P.invcs4;
+                guo(std::integral_constant<int, q>{}, 1.0, cc, r);
+                guo(std::integral_constant<int, q>{}, -1.0, cc, rb);
+            }
+            outf.template put<q>(r);
+            outf.template put<qb>(rb);
+        });
     }
 
     if constexpr (THERMAL) {
-        const double u2 = (ux * ux + uy * uy + uz * uz);
+        const double u2z = u2_of(ux, uy, uz);
         double invtau_t = P.invtau_t;
         if constexpr (FLUID)
-            if (P.les_t) invtau_t = 1.0 / les_tau_t(P, tau_les);
-#pragma unroll
-        for (int q = 0; q < Q; q++) {
-            double r = g[q];
-            r += -invtau_t * (g[q] - feq_q(P, q, T, ux, uy, uz, u2));
-            stp64<NT>(gout + (size_t)q * N + n, r);
+            if (GEN && P.les_t) invtau_t = 1.0 / les_tau_t(P, tau_les);
+        {
+            double r = g[0];
+            r += -invtau_t * (g[0] - feq_rest(P, T, u2z));
+            outg.template put<0>(r);
         }
-        tlag[n] = T;
+        static_for<0, 9>([&](auto kk) {
+            constexpr int q = pair64(decltype(kk)::value), qb = invq(q);
+            const EqPair e = feq_pair<q>(P, T, ux, uy, uz, u2z);
+            double r = g[q], rb = g[qb];
+            r += -invtau_t * (g[q] - e.eq);
+            rb += -invtau_t * (g[qb] - e.eqb);
+            outg.template put<q>(r);
+            outg.template put<qb>(rb);
+        });
     }
+}
+
+// One node of the fused step.  UNI: what the wave shares (Pull).  BUF: planes
+// through buffer resources (planes_ok), else through pointers.
+template <bool FIRST, bool FLUID, bool THERMAL, bool NT, bool GEN, bool BUF, int UNI>
+__device__ __forceinline__ void step_node64(const KParams &P, const double *__restrict__ fin,
+                                            const double *__restrict__ gin, double *__restrict__ fout,
+                                            double *__restrict__ gout, double *__restrict__ tlag,
+                                            double *__restrict__ taules, int x, int y, int z, uint32_t n)
+{
+    const Nbr b = make_nbr(x, y, z, P.NX, P.NY, P.NZ);
+    double Tlag = 0.0, T = 0.0;
+    double g[Q], f[Q];
+    if constexpr (THERMAL) Tlag = tlag[n];
+    if constexpr (BUF) {
+        static_assert(!FIRST, "the first step reads pre-collision populations");
+        const Pull<double, UNI> o(b, P.NX, P.NY);
+        if constexpr (THERMAL) pull_thermal64(P, b, make_planes(gin, P.S), o, Tlag, g);
+        if constexpr (FLUID) pull_fluid64(P, b, make_planes(fin, P.S), o, f);
+        if constexpr (THERMAL) T = m_sum(g);
+        const PlaneOut<NT, UNI> outf{make_planes(FLUID ? fout : gout, P.S), o};
+        const PlaneOut<NT, UNI> outg{make_planes(THERMAL ? gout : fout, P.S), o};
+        collide64<FLUID, THERMAL, GEN>(P, b, f, g, Tlag, T, taules, n, outf, outg);
+    } else {
+        if constexpr (THERMAL) gather_thermal<FIRST>(P, b, gin, n, Tlag, g);
+        if constexpr (FLUID) gather_fluid<FIRST>(P, b, fin, n, f);
+        if constexpr (THERMAL) T = m_sum(g);
+        collide64<FLUID, THERMAL, GEN>(P, b, f, g, Tlag, T, taules, n, FlatOut<NT>{fout, (size_t)P.S, n},
+                                       FlatOut<NT>{gout, (size_t)P.S, n});
+    }
+    if constexpr (THERMAL) tlag[n] = T;
 }
 
 // Row grid or, DENSE, a linear grid with one node per lane (see dense_rows),
 // in the block order of step_order.
-template <bool FIRST, bool FLUID, bool THERMAL, bool DENSE, bool NT>
+template <bool FIRST, bool FLUID, bool THERMAL, bool DENSE, bool NT, bool GEN, bool BUF>
 __global__ void __launch_bounds__(256) k_step_fp64(KParams P, const double *__restrict__ fin,
                                                    const double *__restrict__ gin, double *__restrict__ fout,
                                                    double *__restrict__ gout, double *__restrict__ tlag,
@@ -334,7 +485,7 @@ __global__ void __launch_bounds__(256) k_step_fp64(KParams P, const double *__re
         z = (int)(row / (uint32_t)P.NY);
         n = row * (uint32_t)P.NX + x;
     }
-    step_node64<FIRST, FLUID, THERMAL, NT>(P, fin, gin, fout, gout, tlag, taules, x, y, z, n);
+    step_node64<FIRST, FLUID, THERMAL, NT, GEN, BUF, DENSE ? PULL_LINEAR : PULL_ROW>(P, fin, gin, fout, gout, tlag, taules, x, y, z, n);
 }
 
 // Velocity of the step at every node (the u[] that add_collision reads,
@@ -361,7 +512,7 @@ __global__ void __launch_bounds__(256) k_velocity64(KParams P, const double *__r
 }
 
 // Many lattices in one launch (see k_step_batch32).
-template <bool FLUID, bool THERMAL, bool DENSE, bool NT>
+template <bool FLUID, bool THERMAL, bool DENSE, bool NT, bool GEN, bool BUF>
 __global__ void __launch_bounds__(256) k_step_batch64(const BatchEntry *__restrict__ tab,
                                                       const BatchSlot *__restrict__ slots, int nslots, int run)
 {
@@ -403,7 +554,7 @@ __global__ void __launch_bounds__(256) k_step_batch64(const BatchEntry *__restri
         z = row / (uint32_t)P.NY;
         n = row * (uint32_t)P.NX + x;
     }
-    step_node64<false, FLUID, THERMAL, NT>(P, fin, gin, fout, gout, tl, tau, (int)x, (int)y, (int)z, n);
+    step_node64<false, FLUID, THERMAL, NT, GEN, BUF, DENSE ? PULL_LINEAR : PULL_ROW>(P, fin, gin, fout, gout, tl, tau, (int)x, (int)y, (int)z, n);
 }
 
 // Streaming of the last step + hydro_fields, without a new collision:
@@ -479,31 +630,37 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
     const StepOrder o = step_order(state_bytes(P, 8), dense || P.NX % 16 == 0, RANGE_BYTES_64);
     // ranges and plain stores go together (see step_order)
     const bool nt = o.nts && o.run == RUN_GROUP;
-#define CH4G_LAUNCH64N_(F_, FL_, TH_, D_)                                                                             \
-    do {                                                                                                              \
-        if (nt)                                                                                                       \
-            hipLaunchKernelGGL((k_step_fp64<F_, FL_, TH_, D_, true>), grid, block, 0, s, P, fin, gin, fout, gout,    \
-                               tlag, taules, o.run);                                                                  \
-        else                                                                                                          \
-            hipLaunchKernelGGL((k_step_fp64<F_, FL_, TH_, D_, false>), grid, block, 0, s, P, fin, gin, fout, gout,   \
-                               tlag, taules, o.run);                                                                  \
-    } while (0)
-#define CH4G_LAUNCH64(F_, FL_, TH_)                                                                                   \
-    do {                                                                                                              \
-        if (!(F_) && dense)                                                                                           \
-            CH4G_LAUNCH64N_(false, FL_, TH_, true);                                                                   \
-        else                                                                                                          \
-            CH4G_LAUNCH64N_(F_, FL_, TH_, false);                                                                     \
-    } while (0)
-    if (P.fluid && P.thermal) {
-        if (P.first) CH4G_LAUNCH64(true, true, true); else CH4G_LAUNCH64(false, true, true);
-    } else if (P.fluid) {
-        if (P.first) CH4G_LAUNCH64(true, true, false); else CH4G_LAUNCH64(false, true, false);
-    } else {
-        if (P.first) CH4G_LAUNCH64(true, false, true); else CH4G_LAUNCH64(false, false, true);
-    }
-#undef CH4G_LAUNCH64
-#undef CH4G_LAUNCH64N_
+    // planes beyond the reach of buffer resources take the general instance
+    const bool buf = planes_ok(P, 8), gen = P.hit || P.les || P.twoway || P.nozero || !buf;
+    auto sets = [&](auto fl, auto th) {
+        constexpr bool FL = decltype(fl)::value, TH = decltype(th)::value;
+        if (P.first) {
+            hipLaunchKernelGGL((k_step_fp64<true, FL, TH, false, false, true, false>), grid, block, 0, s, P, fin, gin,
+                               fout, gout, tlag, taules, o.run);
+            return;
+        }
+        with_bool(dense, [&](auto d) {
+            with_bool(nt, [&](auto n) {
+                constexpr bool D = decltype(d)::value, NT = decltype(n)::value;
+                auto go = [&](auto g, auto bf) {
+                    hipLaunchKernelGGL((k_step_fp64<false, FL, TH, D, NT, decltype(g)::value, decltype(bf)::value>),
+                                       grid, block, 0, s, P, fin, gin, fout, gout, tlag, taules, o.run);
+                };
+                if (!gen)
+                    go(std::false_type{}, std::true_type{});
+                else if (buf)
+                    go(std::true_type{}, std::true_type{});
+                else
+                    go(std::true_type{}, std::false_type{});
+            });
+        });
+    };
+    if (P.fluid && P.thermal)
+        sets(std::true_type{}, std::true_type{});
+    else if (P.fluid)
+        sets(std::true_type{}, std::false_type{});
+    else
+        sets(std::false_type{}, std::true_type{});
 }
 
 void launch_velocity_fp64(const KParams &P, const double *fin, const double *tlag, hipStream_t s)
@@ -517,32 +674,35 @@ void launch_velocity_fp64(const KParams &P, const double *fin, const double *tla
 }
 
 void launch_batch_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
-                       bool dense, StepOrder o, hipStream_t s)
+                       bool dense, bool gen, bool buf, StepOrder o, hipStream_t s)
 {
     dim3 grid((unsigned)nblocks), block(256);
+    gen = gen || !buf;
     const bool nt = o.nts && o.run == RUN_GROUP;
-#define CH4G_BATCH64N_(FL_, TH_, D_)                                                                                  \
-    do {                                                                                                              \
-        if (nt)                                                                                                       \
-            hipLaunchKernelGGL((k_step_batch64<FL_, TH_, D_, true>), grid, block, 0, s, tab, slots, nslots, o.run);  \
-        else                                                                                                          \
-            hipLaunchKernelGGL((k_step_batch64<FL_, TH_, D_, false>), grid, block, 0, s, tab, slots, nslots, o.run); \
-    } while (0)
-#define CH4G_BATCH64(FL_, TH_)                                                                                        \
-    do {                                                                                                              \
-        if (dense)                                                                                                    \
-            CH4G_BATCH64N_(FL_, TH_, true);                                                                           \
-        else                                                                                                          \
-            CH4G_BATCH64N_(FL_, TH_, false);                                                                          \
-    } while (0)
+    auto sets = [&](auto fl, auto th) {
+        constexpr bool FL = decltype(fl)::value, TH = decltype(th)::value;
+        with_bool(dense, [&](auto d) {
+            with_bool(nt, [&](auto n) {
+                constexpr bool D = decltype(d)::value, NT = decltype(n)::value;
+                auto go = [&](auto g, auto bf) {
+                    hipLaunchKernelGGL((k_step_batch64<FL, TH, D, NT, decltype(g)::value, decltype(bf)::value>), grid,
+                                       block, 0, s, tab, slots, nslots, o.run);
+                };
+                if (!gen)
+                    go(std::false_type{}, std::true_type{});
+                else if (buf)
+                    go(std::true_type{}, std::true_type{});
+                else
+                    go(std::true_type{}, std::false_type{});
+            });
+        });
+    };
     if (kind == BATCH_FLUID_THERMAL)
-        CH4G_BATCH64(true, true);
+        sets(std::true_type{}, std::true_type{});
     else if (kind == BATCH_FLUID)
-        CH4G_BATCH64(true, false);
+        sets(std::true_type{}, std::false_type{});
     else
-        CH4G_BATCH64(false, true);
-#undef CH4G_BATCH64
-#undef CH4G_BATCH64N_
+        sets(std::false_type{}, std::true_type{});
 }
 
 // LB_FLUID_FORCING_NOZEROMODE (forcing.c:1123-1152): sums over all nodes of
