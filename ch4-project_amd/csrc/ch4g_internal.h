@@ -370,21 +370,25 @@ int launch_reorder(const PartParams &P, const ReorderBufs &B, hipStream_t s);
 constexpr int BATCH_WAVE = 64;
 constexpr int BATCH_WAVES_PER_BLOCK = 4;
 
-// Lattices whose rows fill less than 90 % of the 64-lane waves that cover
-// them (NX = 78: 61 %) are stepped with one node per lane in linear order,
-// each lane decoding its own row, instead of row-aligned waves.
-inline bool dense_rows(int NX)
+// Lattices stepped with one node per lane in linear order, each lane decoding
+// its own row, instead of row-aligned waves: those whose rows fill less than
+// 90 % of the 64-lane waves that cover them (NX = 78: 61 %), and streamed ones
+// whose rows are not whole cache lines, whose row stores would be partial
+// lines in memory (us per step, rows -> linear: float 125^3 146 -> 113, 186^3
+// 444 -> 375, channel 185^3 222 -> 176; FP64 120^3 244 -> 216, 250^3 2040 ->
+// 1850, 969x487 59.1 -> 55.5; in cache rows are as fast, FP64 channel 60^3 11.3
+// against 11.7).
+inline bool dense_rows(const KParams &P, int64_t rsz)
 {
-    const int64_t lanes = (int64_t)(NX + BATCH_WAVE - 1) / BATCH_WAVE * BATCH_WAVE;
-    return (int64_t)NX * 10 < lanes * 9;
+    const int64_t lanes = (int64_t)(P.NX + BATCH_WAVE - 1) / BATCH_WAVE * BATCH_WAVE;
+    return (int64_t)P.NX * 10 < lanes * 9 || (P.NX * rsz % 128 != 0 && state_bytes(P, rsz) > CACHED_BYTES);
 }
 
 // wave tiles of a lattice in the batched step
-inline int64_t batch_tiles(int NX, int NY, int NZ)
+inline int64_t batch_tiles(const KParams &P, bool dense)
 {
-    const int64_t N = (int64_t)NX * NY * NZ;
-    if (dense_rows(NX)) return (N + BATCH_WAVE - 1) / BATCH_WAVE;
-    return (int64_t)NY * NZ * ((NX + BATCH_WAVE - 1) / BATCH_WAVE);
+    if (dense) return (P.N + BATCH_WAVE - 1) / BATCH_WAVE;
+    return (int64_t)P.NY * P.NZ * ((P.NX + BATCH_WAVE - 1) / BATCH_WAVE);
 }
 
 // One lattice of a batched step: its constants and its two state buffers

@@ -151,11 +151,12 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
     std::vector<int> order;
     for (size_t i = 0; i < lats.size(); i++)
         if (!solo[i]) order.push_back((int)i);
+    auto dense_of = [](const ch4g_lattice *L) { return dense_rows(L->base, L->dev32 ? 4 : 8); };
     auto key = [&](int i) {
         const ch4g_lattice *L = lats[(size_t)i];
         const int two = B.two[(size_t)i];
         return (L->base.les << 6) | (two << 5) | (L->dev32 << 4) | (L->base.arith64 << 3) |
-               ((int)(!two && dense_rows(L->cfg.NX)) << 2) | kind_of(L);
+               ((int)(!two && dense_of(L)) << 2) | kind_of(L);
     };
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return key(a) < key(b); });
     for (size_t i = 0; i < order.size();) {
@@ -166,7 +167,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         G.arith64 = L0->base.arith64;
         G.kind = kind_of(L0);
         G.two = B.two[(size_t)order[i]] != 0;
-        G.dense = !G.two && dense_rows(L0->cfg.NX);
+        G.dense = !G.two && dense_of(L0);
         G.gen = L0->base.les != 0;
         G.first = (int)B.host.size();
         G.count = 0;
@@ -207,7 +208,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
             for (int s_ = 0; s_ < nl; s_++) a[(size_t)(((int64_t)s_ * KG) / nl)] = s_;
             at.push_back(a);
             npair.push_back(G.two ? st / 2 : 0);
-            ntile.push_back(G.two ? batch2_tiles(L->cfg.NX, L->cfg.NY) : batch_tiles(L->cfg.NX, L->cfg.NY, L->cfg.NZ));
+            ntile.push_back(G.two ? batch2_tiles(L->cfg.NX, L->cfg.NY) : batch_tiles(L->base, G.dense));
             bytes += 2 * (int64_t)Q * L->N * (L->dev32 ? 4 : 8) * ((L->base.fluid ? 1 : 0) + (L->base.thermal ? 1 : 0));
             G.buf = G.buf && planes_ok(L->base, 8);
             whole_lines = whole_lines && (G.dense || L->cfg.NX * (L->dev32 ? 4 : 8) % 128 == 0);

@@ -908,7 +908,8 @@ __device__ __forceinline__ void load_raw_buf(const KParams &P, const Nbr &b, con
     }
 }
 
-// NodeOut through buffer resources (non-temporal stores)
+// NodeOut through buffer resources
+template <bool NT>
 struct BufOut {
     Planes<float> f, g;
     float *__restrict__ tlag;
@@ -917,14 +918,14 @@ struct BufOut {
     {
         static_for<0, Q>([&](auto qc) {
             constexpr int qq = decltype(qc)::value;
-            if (qq == q) plane_store<qq, true>(f, n4, 0u, v);
+            if (qq == q) plane_store<qq, NT>(f, n4, 0u, v);
         });
     }
     __device__ void put_g(int q, float v) const
     {
         static_for<0, Q>([&](auto qc) {
             constexpr int qq = decltype(qc)::value;
-            if (qq == q) plane_store<qq, true>(g, n4, 0u, v);
+            if (qq == q) plane_store<qq, NT>(g, n4, 0u, v);
         });
     }
     __device__ void put_tlag(float v) const { tlag[n] = v; }
@@ -1016,7 +1017,7 @@ __device__ __forceinline__ void ring_put(float *t, int m, int it, const float rf
 // not written.  Per two steps the state is read (1 + 2/zc) x M/T times and
 // written once; the temperature lag is read from tl_in and written to tl_out
 // (halo nodes of one block are tile nodes of another).
-template <bool FLUID, bool THERMAL, typename A, class TZ>
+template <bool FLUID, bool THERMAL, typename A, bool NTS, class TZ>
 __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp32(KParams P, const float *__restrict__ fin,
                                                              const float *__restrict__ gin, float *__restrict__ fout,
                                                              float *__restrict__ gout,
@@ -1150,7 +1151,7 @@ __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp32(KParams P, const fl
                 collide_thermal<A, false>(P, R, yb, g, dT, ux, uy, uz, tau_les, out);
             }
             };
-            collide2(BufOut{pout_f, pout_g, tl_out, n, n * 4u});
+            collide2(BufOut<NTS>{pout_f, pout_g, tl_out, n, n * 4u});
         }
         __syncthreads();
         // ---- C (HOLD): the c_z >= 0 results of plane j into rings Z, P, W
@@ -1358,7 +1359,7 @@ void launch_step_fp32(const KParams &P, const float *fin, const float *gin, floa
                       float *taules, hipStream_t s)
 {
     int bx = block_x32(P);
-    const bool dense = !P.first && dense_rows(P.NX);
+    const bool dense = !P.first && dense_rows(P, 4);
     dim3 grid((P.NX + bx - 1) / bx, P.NY, P.NZ), block(bx);
     if (dense) {
         grid = dim3((unsigned)((P.N + 255) / 256));
@@ -1416,53 +1417,18 @@ void launch_step_fp32(const KParams &P, const float *fin, const float *gin, floa
 // with narrower last tiles 78x40 4.69 -> 3.85, 1000x500 38.6 -> 28.9,
 // 1500x700 76.3 -> 48.2 (against the dense single-step grid).
 //
-// 3-D lattices (k_step2z_fp32) need enough tile columns to fill the GPU and
-// rows that fill their 64-wide tiles; measured against single steps with
-// graph replay (us per step): channel 64^3 8.4 vs 20.3, 96^3 28.6 vs 46.0,
-// 128^3 62.2 vs 49.5, 160^3 (rows of 2.5 tiles) 116 vs 122, 192^3 196 vs 185;
-// Rayleigh-Benard 96^3 57.1 vs 66.9, 128^3 126.9 vs 92.6, 192^3 406 vs 344.
+// 3-D lattices: see z_marching_pays.
+static bool z_marching_pays(const KParams &P);
+
 bool two_step_ok(const KParams &P)
 {
     // 2-D: 32-bit byte offsets into the Q population planes; 3-D: 32-bit
     // byte offsets within a group of seven planes
     const bool off32 = (int64_t)Q * P.S * 4 < ((int64_t)1 << 32);
-    const int64_t tiles_x = (P.NX + 63) / 64;
-    const bool big3d = P.N >= ((int64_t)1 << 21) && 10 * (int64_t)P.NX >= 9 * 64 * tiles_x;
-    const bool fits = P.NZ == 1 ? off32 : (big3d && 7 * P.S * 4 < ((int64_t)1 << 32));
+    const bool fits = P.NZ == 1 ? off32 : (planes_ok(P, 4) && z_marching_pays(P));
     return fits && !P.first && !P.hit && !P.les && !P.twoway && !P.nozero;
 }
 
-namespace {
-
-// Two steps per launch for 3-D lattices (k_step2z_fp32), z ranges of zc
-// planes.
-template <class TZ>
-void launch_z2(const KParams &P, const float *fin, const float *gin, float *fout, float *gout, const float *tl_in,
-               float *tl_out, int zc, hipStream_t s)
-{
-    const unsigned bx = (unsigned)((P.NX + TZ::TX - 1) / TZ::TX), by = (unsigned)((P.NY + TZ::TY - 1) / TZ::TY);
-    const dim3 grid(bx, by, (unsigned)((P.NZ + zc - 1) / zc));
-#define CH4G_Z2_(FL_, TH_, A_)                                                                                        \
-    hipLaunchKernelGGL((k_step2z_fp32<FL_, TH_, A_, TZ>), grid, dim3(TZ::THREADS), 0, s, P, fin, gin, fout, gout,   \
-                       tl_in, tl_out, zc)
-    constexpr bool FL = TZ::F == 1, TH = TZ::H == 1;
-    if (P.arith64)
-        CH4G_Z2_(FL, TH, double);
-    else
-        CH4G_Z2_(FL, TH, float);
-#undef CH4G_Z2_
-}
-
-template <bool FL, bool TH, int TX, int TY, bool HOLD>
-using TZ_ = TileZ<FL, TH, TX, TY, HOLD>;
-
-// Tiles (measured at 512^3 fluid + T, FP32-deviation, ms per step, single
-// steps 7.9): 64 x 4 held in registers 6.9, with the next plane's loads in
-// flight during step B 6.5, 32 x 5 all in LDS (two blocks per CU) 7.3,
-// 64 x 8 held 6.0, the same through buffer resources 5.6-5.9; 3-D channel
-// 256^3: single 0.46, 64 x 8 held 0.35.  Double arithmetic needs more
-// registers than an 11-wave block allows: 64 x 4.
-//
 // z ranges: a CU holds one block (LDS), and a block of zc planes takes zc + 2
 // iterations of the same length, so the launch takes ceil(blocks / 256) (zc +
 // 2) of them: the most ranges that 1 to 8 full rounds of blocks hold, whichever
@@ -1489,13 +1455,77 @@ static int z_range(int64_t columns, int NZ)
     return (int)zbest;
 }
 
+// rows of a z-marching tile (see launch_two_steps_3d)
+static int z_rows(const KParams &P) { return P.fluid && !(P.thermal && P.arith64) ? 8 : 4; }
+
+static int64_t z_columns(const KParams &P)
+{
+    const int TY = z_rows(P);
+    return (int64_t)((P.NX + 63) / 64) * ((P.NY + TY - 1) / TY);
+}
+
+// Whether two z-marching steps are faster than two single steps.  From 2^21
+// nodes whose rows fill 90 % of their tiles; below, for float arithmetic, by a
+// launch's iterations (z_range) at 9.5 us (fluid and temperature; fluid alone 5.1),
+// 7.8 (3.8) while the caches hold the state, against the nodes at 59 ps a step
+// (29), 54 (25) in cache.  us per step, single -> marching: Rayleigh-Benard
+// 96^3 50 -> 43, 120^3 101 -> 83, 125^3 113 -> 90, 160^3 242 -> 183, 208^3 525 ->
+// 438, 256x80x80 97 -> 74; the rule leaves 64^3 (13.5 against 19.4), 78^3 (23.8
+// against 37) and 100^3 (58.6 against 61.4) single.  Channel 113^3 34.1 -> 31.7,
+// 125^3 49 -> 45, 185^3 176 -> 150; 96^3 (21.9 against 22.7) single; channels
+// whose rows fill less than 85 % of their tiles stay single (160^3 117 against
+// 105).
+static bool z_marching_pays(const KParams &P)
+{
+    const int64_t tiles_x = (P.NX + 63) / 64, fill = (int64_t)P.NX * 100 / (64 * tiles_x);
+    if (P.N >= ((int64_t)1 << 21) && fill >= 90) return true;
+    if (P.arith64 || !P.fluid || (!P.thermal && fill < 85)) return false;
+    const bool cached = state_bytes(P, 4) <= CACHED_BYTES;
+    const double t_iter = P.thermal ? (cached ? 7.8 : 9.5) : (cached ? 3.8 : 5.1);           // us
+    const double t_node = P.thermal ? (cached ? 54e-6 : 59e-6) : (cached ? 25e-6 : 29e-6);  // us
+    const int64_t columns = z_columns(P), zc = z_range(columns, P.NZ);
+    const int64_t its = (columns * ((P.NZ + zc - 1) / zc) + 255) / 256 * (zc + 2);
+    return (double)its * t_iter < 2.0 * (double)P.N * t_node;
+}
+
+namespace {
+
+// Two steps per launch for 3-D lattices (k_step2z_fp32), z ranges of zc
+// planes.
+template <class TZ>
+void launch_z2(const KParams &P, const float *fin, const float *gin, float *fout, float *gout, const float *tl_in,
+               float *tl_out, int zc, hipStream_t s)
+{
+    const unsigned bx = (unsigned)((P.NX + TZ::TX - 1) / TZ::TX), by = (unsigned)((P.NY + TZ::TY - 1) / TZ::TY);
+    const dim3 grid(bx, by, (unsigned)((P.NZ + zc - 1) / zc));
+    constexpr bool FL = TZ::F == 1, TH = TZ::H == 1;
+    // non-temporal stores when streamed and rows are whole half lines: others
+    // would write partial lines to memory (us per step, non-temporal against
+    // plain: 185x191x187 380, 281; 125^3 114, 90; 144^3 156, 166; 160^3 183, 188)
+    with_bool(step_order(state_bytes(P, 4), P.NX % 16 == 0, 0).nts, [&](auto nt) {
+        constexpr bool N = decltype(nt)::value;
+        if (P.arith64)
+            hipLaunchKernelGGL((k_step2z_fp32<FL, TH, double, N, TZ>), grid, dim3(TZ::THREADS), 0, s, P, fin, gin,
+                               fout, gout, tl_in, tl_out, zc);
+        else
+            hipLaunchKernelGGL((k_step2z_fp32<FL, TH, float, N, TZ>), grid, dim3(TZ::THREADS), 0, s, P, fin, gin, fout,
+                               gout, tl_in, tl_out, zc);
+    });
+}
+
+template <bool FL, bool TH, int TX, int TY, bool HOLD>
+using TZ_ = TileZ<FL, TH, TX, TY, HOLD>;
+
+// Tiles (measured at 512^3 fluid + T, FP32-deviation, ms per step, single
+// steps 7.9): 64 x 4 held in registers 6.9, with the next plane's loads in
+// flight during step B 6.5, 32 x 5 all in LDS (two blocks per CU) 7.3,
+// 64 x 8 held 6.0, the same through buffer resources 5.6-5.9; 3-D channel
+// 256^3: single 0.46, 64 x 8 held 0.35.  Double arithmetic needs more
+// registers than an 11-wave block allows: 64 x 4.
 void launch_two_steps_3d(const KParams &P, const float *fin, const float *gin, float *fout, float *gout,
                          const float *tl_in, float *tl_out, hipStream_t s)
 {
-    const bool tall = P.fluid && !(P.thermal && P.arith64);
-    const int TY = tall ? 8 : 4;
-    const int64_t columns = (int64_t)((P.NX + 63) / 64) * ((P.NY + TY - 1) / TY);
-    const int z = z_range(columns, P.NZ);
+    const int z = z_range(z_columns(P), P.NZ);
 #define Z2(...) launch_z2<TZ_<__VA_ARGS__>>(P, fin, gin, fout, gout, tl_in, tl_out, z, s)
     if (P.fluid && P.thermal) {
         if (P.arith64)

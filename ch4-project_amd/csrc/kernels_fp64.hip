@@ -621,7 +621,7 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
                       double *tlag, double *taules, hipStream_t s)
 {
     int bx = block_x(P);
-    const bool dense = !P.first && dense_rows(P.NX);
+    const bool dense = !P.first && dense_rows(P, 8);
     dim3 grid = grid_of(P, bx), block(bx);
     if (dense) {
         grid = dim3((unsigned)((P.N + 255) / 256));

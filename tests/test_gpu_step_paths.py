@@ -28,8 +28,8 @@ def run(x, steps):
 
 # Block orders (step_order): FP64 beyond 1.5 GiB and float beyond 320 MiB of
 # state go in groups of 64 blocks with non-temporal stores where these are
-# whole lines; 113-wide float rows take the linear grid, 128-wide ones the row
-# grid, 500-wide rows are not whole lines.  Block counts that are no multiple
+# whole lines; 113-wide float rows and 500-wide ones (no whole lines) take the
+# linear grid, 128-wide ones the row grid.  Block counts that are no multiple
 # of 64 leave a partial last group.
 @pytest.mark.parametrize("shape,precision", [
     ((113, 97, 103), abi.FP32_DEV), ((128, 95, 93), abi.FP32_DEV), ((500, 49, 47), abi.FP32_DEV),
@@ -48,6 +48,26 @@ def test_streamed_block_order(shape, precision):
         print(f"  {shape}: L2 rel err of u {err:.2e}")
         assert err <= 1e-5
     lat.close()
+
+
+# 3-D two-step launches below 2^21 nodes: in cache (96^3), streamed with rows
+# that are no whole lines (plain stores) or half lines, a channel, partial
+# tiles in x and y and a shorter last z range.  Equal, bit for bit, to the same
+# lattice advanced one step per launch.
+@pytest.mark.parametrize("shape,channel", [((96, 96, 96), False), ((125, 113, 101), False), ((208, 63, 90), False),
+                                           ((113, 113, 113), True)], ids=str)
+def test_small_3d_two_step_launches(shape, channel):
+    from ch4g import workloads
+    cfg = workloads.channel3d(*shape) if channel else configs.rb2d(*shape, Ra=1e6, precision=abi.FP32_DEV, seed=5)
+    two, one = Lattice(cfg), Lattice(cfg)
+    one.set_fusion(False)
+    assert (two.steps_per_launch(), one.steps_per_launch()) == (2, 1)
+    for lat in (two, one):
+        run(lat, 8)
+    for a, b in zip(two.get_populations(), one.get_populations()):
+        assert np.array_equal(a, b)
+    two.close()
+    one.close()
 
 
 # The averages' and rulers' marches: fewer rows, columns or planes than one
