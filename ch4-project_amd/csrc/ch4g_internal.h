@@ -465,7 +465,8 @@ void launch_force_mean64(const KParams &P, bool step, const double *gin, const d
 void launch_velocity_fp32(const KParams &P, const float *fin, const float *tlag, hipStream_t s);
 
 // Initial state from a per-row fluid profile prow[NY][19] and a temperature
-// field t0[N]; restart load from FP64 SoA staging.  dev = FP32-deviation.
+// field t0[N]; restart load from FP64 records [N][Q] (fs, gs on the device).
+// dev = FP32-deviation.
 void launch_init(const KParams &P, const double *prow, const double *t0, void *f, void *g, void *tlag, int dev,
                  hipStream_t s);
 void launch_load(const KParams &P, const double *fs, const double *gs, void *f, void *g, void *tlag, int dev,

@@ -42,7 +42,9 @@ __global__ void k_init(KParams P, const double *__restrict__ prow, const double 
     }
 }
 
-// Load populations from FP64 SoA staging (restart), tlag <- sum g.
+// Load populations from the host's FP64 records [N][19] (restart), tlag <-
+// sum g.  A wave reads 64 consecutive records: their lines stay in the L1
+// over the 19 strided reads.
 template <typename R>
 __global__ void k_load(KParams P, const double *__restrict__ fs, const double *__restrict__ gs, R *__restrict__ f,
                        R *__restrict__ g, R *__restrict__ tlag, int dev)
@@ -53,12 +55,12 @@ __global__ void k_load(KParams P, const double *__restrict__ fs, const double *_
     const double rb = dev ? P.row64[2 * y] : 0.0, tb = dev ? P.row64[2 * y + 1] : 0.0;
     if (P.fluid && fs)
         for (int q = 0; q < Q; q++) {
-            double v = fs[q * P.N + n];
+            double v = fs[n * Q + q];
             f[q * P.S + n] = dev ? (R)(v - wq(q) * rb) : (R)v;
         }
     if (P.thermal && gs) {
         double gq[Q];
-        for (int q = 0; q < Q; q++) gq[q] = gs[q * P.N + n];
+        for (int q = 0; q < Q; q++) gq[q] = gs[n * Q + q];
         for (int q = 0; q < Q; q++) g[q * P.S + n] = dev ? (R)(gq[q] - wq(q) * tb) : (R)gq[q];
         double T = msum19(gq);
         tlag[n] = dev ? (R)(T - tb) : (R)T;

@@ -1290,7 +1290,6 @@ __global__ void __launch_bounds__(256) k_gather_fp32(KParams P, const float *__r
     if (x >= P.NX) return;
     const int y = blockIdx.y, z = blockIdx.z;
     const uint32_t n = ((uint32_t)z * P.NY + y) * P.NX + x;
-    const size_t N = (size_t)P.N;
     const Row R = row_of(P, y);
     const Nbr b = make_nbr(x, y, z, P.NX, P.NY, P.NZ);
     const double rb = P.row64[2 * y], tb = P.row64[2 * y + 1];
@@ -1307,7 +1306,7 @@ __global__ void __launch_bounds__(256) k_gather_fp32(KParams P, const float *__r
         double s = 0.0;
         for (int q = 0; q < Q; q++) {
             s += (double)g[q];
-            if (gpost) gpost[q * N + n] = wq(q) * tb + (double)g[q];
+            if (gpost) gpost[(size_t)n * Q + q] = wq(q) * tb + (double)g[q];
         }
         if (t) t[n] = tb + s;
         ft = (float)(tb + s);
@@ -1325,7 +1324,7 @@ __global__ void __launch_bounds__(256) k_gather_fp32(KParams P, const float *__r
             jx += cxq(q) * d;
             jy += cyq(q) * d;
             jz += czq(q) * d;
-            if (fpost) fpost[q * N + n] = wq(q) * rb + d;
+            if (fpost) fpost[(size_t)n * Q + q] = wq(q) * rb + d;
         }
         double rho = rb + drho;
         double ux = jx / rho, uy = jy / rho, uz = jz / rho;

@@ -558,7 +558,7 @@ __global__ void __launch_bounds__(256) k_step_batch64(const BatchEntry *__restri
 }
 
 // Streaming of the last step + hydro_fields, without a new collision:
-// produces the reference's p, g (AoS order not applied here: SoA planes),
+// produces the reference's p, g (records [N][19], as the host takes them),
 // dens, u and t of the current step.  Any output may be null.
 __global__ void __launch_bounds__(256) k_gather_fp64(KParams P, const double *__restrict__ fin,
                                                      const double *__restrict__ gin,
@@ -570,7 +570,6 @@ __global__ void __launch_bounds__(256) k_gather_fp64(KParams P, const double *__
     if (x >= P.NX) return;
     const int y = blockIdx.y, z = blockIdx.z;
     const uint32_t n = ((uint32_t)z * P.NY + y) * P.NX + x;
-    const size_t N = (size_t)P.N;
     const Nbr b = make_nbr(x, y, z, P.NX, P.NY, P.NZ);
     double Tlag = 0.0;
     if (P.thermal) {
@@ -581,7 +580,7 @@ __global__ void __launch_bounds__(256) k_gather_fp64(KParams P, const double *__
         else
             gather_thermal<false>(P, b, gin, n, Tlag, g);
         if (gpost)
-            for (int q = 0; q < Q; q++) gpost[q * N + n] = g[q];
+            for (int q = 0; q < Q; q++) gpost[(size_t)n * Q + q] = g[q];
         if (t) t[n] = m_sum(g);
     }
     if (P.fluid) {
@@ -591,7 +590,7 @@ __global__ void __launch_bounds__(256) k_gather_fp64(KParams P, const double *__
         else
             gather_fluid<false>(P, b, fin, n, f);
         if (fpost)
-            for (int q = 0; q < Q; q++) fpost[q * N + n] = f[q];
+            for (int q = 0; q < Q; q++) fpost[(size_t)n * Q + q] = f[q];
         const double rho = m_sum(f);
         double ux, uy, uz;
         if (P.forced) {
