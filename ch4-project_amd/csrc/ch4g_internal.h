@@ -342,6 +342,18 @@ struct FeedbackBufs {
 };
 int launch_feedback(const PartParams &P, const FeedbackBufs &B, hipStream_t s);
 size_t feedback_sort_bytes(int64_t nitems, int key_bits);
+// Records of the live particles in reference order: their rows into src
+// (flag, rank, row: [np] by reference index), then ch4g_particle records of
+// RECORD_CHUNK particles at a time.
+constexpr int64_t RECORD_CHUNK = 1 << 16;
+struct RecordBufs {
+    int *flag, *rank, *row, *src;
+    void *tmp;
+    size_t tmp_bytes;
+};
+size_t live_scan_bytes(int64_t np);
+int launch_live_rows(const PartParams &P, const RecordBufs &B, hipStream_t s);
+int launch_records(const PartParams &P, const int *src, int64_t m, double *out, hipStream_t s);
 // Rows, alive flags and reference-order indices of the particles reordered
 // by cell (z, y, x of the position's node), for locality of the corner reads.
 // The rows a reordering moves: every row a kernel of the configuration

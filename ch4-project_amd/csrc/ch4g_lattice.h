@@ -52,6 +52,12 @@ struct Particles {
     size_t ro_tmp_bytes = 0;
     int cell_bits = 32;
     int64_t last_reorder = 0;
+    // reading the records back: [4][cap] flags, ranks and rows by reference
+    // index and live rows, scan scratch, one chunk of records
+    int *d_live = nullptr;
+    void *d_scan_tmp = nullptr;
+    size_t scan_tmp_bytes = 0;
+    double *d_records = nullptr;
     PermRows perm{};             // rows the reordering moves (set by each upload)
     std::vector<ch4g_particle_type> types;  // per-type values of the last initialisation
     void *d_sort_tmp = nullptr;

@@ -274,7 +274,7 @@ void free_state(Particles *P)
 {
     void *ptrs[] = {P->d_state, P->d_alive, P->d_ndraw, P->d_bsum, P->d_kin, P->d_vin, P->d_vout, P->d_sort_tmp,
                     P->d_keys[0], P->d_keys[1], P->d_rec, P->d_dep, P->d_ord, P->d_head, P->d_orig, P->d_orig2, P->d_alive2,
-                    P->d_state2, P->d_ck, P->d_ck2, P->d_cv, P->d_cv2, P->d_ro_tmp};
+                    P->d_state2, P->d_ck, P->d_ck2, P->d_cv, P->d_cv2, P->d_ro_tmp, P->d_live, P->d_scan_tmp, P->d_records};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     P->d_state = nullptr;
@@ -289,6 +289,9 @@ void free_state(Particles *P)
     P->d_ck = P->d_ck2 = P->d_cv = P->d_cv2 = nullptr;
     P->d_ro_tmp = nullptr;
     P->ro_tmp_bytes = 0;
+    P->d_live = nullptr;
+    P->d_scan_tmp = nullptr;
+    P->d_records = nullptr;
     P->d_keys[0] = P->d_keys[1] = nullptr;
     P->nkeys[0] = P->nkeys[1] = 0;
     P->cap = 0;
@@ -1011,81 +1014,40 @@ int ch4g_get_particles(ch4g_lattice *L, ch4g_particle *out, int64_t cap, int64_t
     *n = 0;
     Particles *Q = L->part;
     if (!Q || Q->np == 0) return 0;
-    const int64_t ld = Q->cap, np = Q->np;
-    std::vector<double> rows((size_t)PF_COUNT * ld);
-    std::vector<int> alive((size_t)np), orig((size_t)np);
-    HIPCHK(hipMemcpyAsync(rows.data(), Q->d_state, rows.size() * sizeof(double), hipMemcpyDeviceToHost, L->stream));
-    HIPCHK(hipMemcpyAsync(alive.data(), Q->d_alive, alive.size() * sizeof(int), hipMemcpyDeviceToHost, L->stream));
-    HIPCHK(hipMemcpyAsync(orig.data(), Q->d_orig, orig.size() * sizeof(int), hipMemcpyDeviceToHost, L->stream));
-    HIPCHK(hipStreamSynchronize(L->stream));
-    // records in the reference's particle order (rows may be in cell order)
-    std::vector<int64_t> row_of((size_t)np);
-    for (int64_t p = 0; p < np; p++) row_of[(size_t)orig[(size_t)p]] = p;
-    int64_t k = 0;
-    for (int64_t o = 0; o < np; o++) {
-        const int64_t p = row_of[(size_t)o];
-        if (!alive[(size_t)p]) continue;
-        if (k < cap) {
-            auto S = [&](int f) { return rows[(size_t)f * ld + p]; };
-            ch4g_particle &r = out[k];
-            r.name = S(PNAME);
-            r.x = S(PX);
-            r.y = S(PY);
-            r.z = S(PZ);
-            r.vx = S(PVX);
-            r.vy = S(PVY);
-            r.vz = S(PVZ);
-            r.vx_old = S(PVXO);
-            r.vy_old = S(PVYO);
-            r.vz_old = S(PVZO);
-            r.ax = S(PAX);
-            r.ay = S(PAY);
-            r.az = S(PAZ);
-            r.ax_old = S(PAXO);
-            r.ay_old = S(PAYO);
-            r.az_old = S(PAZO);
-            r.ux = S(PUX);
-            r.uy = S(PUY);
-            r.uz = S(PUZ);
-            r.ux_old = S(PUXO);
-            r.uy_old = S(PUYO);
-            r.uz_old = S(PUZO);
-            double *g = &r.dx_ux;
-            for (int m = 0; m < 9; m++) g[m] = S(PG + m);
-            r.Dt_ux = S(PDTU);
-            r.Dt_uy = S(PDTU + 1);
-            r.Dt_uz = S(PDTU + 2);
-            r.t = S(PT);
-            r.t_old = S(PTOLD);
-            r.dt_t = S(PDTT);
-            r.dx_t = S(PGT);
-            r.dy_t = S(PGT + 1);
-            r.dz_t = S(PGT + 2);
-            r.tau_drag = S(PTAU);
-            r.beta_coeff = S(PBETA);
-            r.px = S(PPO);
-            r.py = S(PPO + 1);
-            r.pz = S(PPO + 2);
-            r.dt_px = S(PDTP);
-            r.dt_py = S(PDTP + 1);
-            r.dt_pz = S(PDTP + 2);
-            r.aspect_ratio = S(PASP);
-            r.gyrotaxis_velocity = S(PGYV);
-            r.swim_velocity = S(PSWIM);
-            double *nv = &r.nx;
-            for (int m = 0; m < 6; m++) nv[m] = S(PNO + m);
-            r.t_p = S(PTP);
-            r.cp_p = S(PCP);
-            r.gravity_coeff = S(PGC);
-            r.sediment = S(PSED);
-            double *ct = &r.cxx;
-            for (int m = 0; m < 12; m++) ct[m] = S(PCT + m);
-            double *jr = &r.critical_shear_rate;
-            for (int m = 0; m < 7; m++) jr[m] = S(PCSR + m);
-        }
-        k++;
+    // records formed on the device in the reference's particle order (rows may
+    // be in cell order) and copied straight to the caller: reading all rows
+    // back and forming them on the host took 220 ms for 500,000 particles
+    const int64_t np = Q->np, c = Q->cap;
+    int rc;
+    if (!Q->d_live) {
+        const size_t chunk = (size_t)(c < RECORD_CHUNK ? c : RECORD_CHUNK);
+        Q->scan_tmp_bytes = live_scan_bytes(c);
+        if ((rc = dalloc(L, (void **)&Q->d_records, chunk * sizeof(ch4g_particle)))) return rc;
+        if ((rc = dalloc(L, &Q->d_scan_tmp, Q->scan_tmp_bytes > 0 ? Q->scan_tmp_bytes : 1))) return rc;
+        if ((rc = dalloc(L, (void **)&Q->d_live, (size_t)4 * c * sizeof(int)))) return rc;
     }
-    *n = k;
+    const PartParams P = part_params(L);
+    RecordBufs B;
+    B.flag = Q->d_live;
+    B.rank = Q->d_live + c;
+    B.row = Q->d_live + 2 * c;
+    B.src = Q->d_live + 3 * c;
+    B.tmp = Q->d_scan_tmp;
+    B.tmp_bytes = Q->scan_tmp_bytes;
+    if (launch_live_rows(P, B, L->stream)) return fail(-2, "particle readback failed: %s", hipGetErrorString(hipGetLastError()));
+    int last[2] = {0, 0};
+    HIPCHK(hipMemcpyAsync(&last[0], B.flag + np - 1, sizeof(int), hipMemcpyDeviceToHost, L->stream));
+    HIPCHK(hipMemcpyAsync(&last[1], B.rank + np - 1, sizeof(int), hipMemcpyDeviceToHost, L->stream));
+    HIPCHK(hipStreamSynchronize(L->stream));
+    const int64_t live = (int64_t)last[0] + last[1], want = live < cap ? live : cap;
+    for (int64_t k = 0; k < want; k += RECORD_CHUNK) {
+        const int64_t m = want - k < RECORD_CHUNK ? want - k : RECORD_CHUNK;
+        if (launch_records(P, B.src + k, m, Q->d_records, L->stream))
+            return fail(-2, "particle readback failed: %s", hipGetErrorString(hipGetLastError()));
+        HIPCHK(hipMemcpyAsync(out + k, Q->d_records, (size_t)m * sizeof(ch4g_particle), hipMemcpyDeviceToHost, L->stream));
+    }
+    HIPCHK(hipStreamSynchronize(L->stream));
+    *n = live;
     return 0;
 }
 

@@ -1553,6 +1553,53 @@ __global__ void __launch_bounds__(PB) k_permute(PartParams P, const uint32_t *sr
     }
 }
 
+// Row of each member of ch4g_particle, in the struct's order.
+constexpr int NREC = (int)(sizeof(ch4g_particle) / sizeof(double));
+struct RecordRows {
+    uint8_t row[NREC];
+    int n;
+    constexpr RecordRows() : row(), n(0)
+    {
+        // runs of consecutive rows: {first row, count}
+        constexpr int run[][2] = {{PNAME, 1}, {PX, 3}, {PVX, 3}, {PVXO, 3}, {PAX, 3}, {PAXO, 3}, {PUX, 3}, {PUXO, 3},
+                                  {PG, 9}, {PDTU, 3}, {PT, 3}, {PTAU, 2}, {PGT, 3}, {PPO, 6}, {PASP, 3}, {PNO, 6},
+                                  {PTP, 2}, {PGC, 1}, {PSED, 1}, {PCT, 12}, {PCSR, 7}};
+        for (auto &r : run)
+            for (int k = 0; k < r[1]; k++) row[n++] = (uint8_t)(r[0] + k);
+    }
+};
+__constant__ constexpr RecordRows record_rows;
+static_assert(record_rows.n == NREC, "the runs cover the record");
+
+// alive flag and row of each particle by reference index
+__global__ void __launch_bounds__(PB) k_by_reference(PartParams P, int *flag, int *row)
+{
+    const int64_t p = (int64_t)blockIdx.x * PB + threadIdx.x;
+    if (p >= P.np) return;
+    const int o = P.orig[p];
+    flag[o] = P.alive[p] ? 1 : 0;
+    row[o] = (int)p;
+}
+
+// rows of the live particles, in reference order (rank: exclusive sum of flag)
+__global__ void __launch_bounds__(PB) k_live_rows(int64_t np, const int *flag, const int *rank, const int *row, int *src)
+{
+    const int64_t o = (int64_t)blockIdx.x * PB + threadIdx.x;
+    if (o < np && flag[o]) src[rank[o]] = row[o];
+}
+
+// Records of m particles: a thread per member, so that records are written as
+// one stream; the rows are read a value at a time.  Bound by the copy to the
+// host that follows (624 B a record over the host link).
+__global__ void __launch_bounds__(PB) k_records(PartParams P, const int *__restrict__ src, uint32_t m,
+                                                double *__restrict__ out)
+{
+    const uint32_t i = blockIdx.x * PB + threadIdx.x;
+    if (i >= m * NREC) return;
+    const uint32_t k = i / NREC, f = i - k * NREC;
+    out[i] = P.s[(int64_t)record_rows.row[f] * P.ld + src[k]];
+}
+
 int blocks_of(int64_t n, int b) { return (int)((n + b - 1) / b); }
 
 }  // namespace
@@ -1622,6 +1669,32 @@ int launch_reorder(const PartParams &P, const ReorderBufs &B, hipStream_t s)
     if (B.rows.n < 1 || B.rows.n > PF_COUNT) return -1;
     hipLaunchKernelGGL(k_permute, dim3(nb, B.rows.n), dim3(PB), 0, s, P, (const uint32_t *)B.vout, B.s_out,
                        B.alive_out, B.orig_out, B.rows);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+size_t live_scan_bytes(int64_t np)
+{
+    size_t bytes = 0;
+    (void)hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (const int *)nullptr, (int *)nullptr, (int)np);
+    return bytes;
+}
+
+int launch_live_rows(const PartParams &P, const RecordBufs &B, hipStream_t s)
+{
+    if (P.np == 0) return 0;
+    const int nb = blocks_of(P.np, PB);
+    hipLaunchKernelGGL(k_by_reference, dim3(nb), dim3(PB), 0, s, P, B.flag, B.row);
+    size_t bytes = B.tmp_bytes;
+    if (hipcub::DeviceScan::ExclusiveSum(B.tmp, bytes, B.flag, B.rank, (int)P.np, s) != hipSuccess) return -2;
+    hipLaunchKernelGGL(k_live_rows, dim3(nb), dim3(PB), 0, s, P.np, (const int *)B.flag, (const int *)B.rank,
+                       (const int *)B.row, B.src);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+int launch_records(const PartParams &P, const int *src, int64_t m, double *out, hipStream_t s)
+{
+    if (m == 0) return 0;
+    hipLaunchKernelGGL(k_records, dim3(blocks_of(m * NREC, PB)), dim3(PB), 0, s, P, src, (uint32_t)m, out);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

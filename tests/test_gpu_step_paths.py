@@ -112,3 +112,39 @@ def test_fp64_numbers_that_are_not_finite(cfg):
         assert np.array_equal(a, b, equal_nan=True)
     assert np.isnan(o.get_populations()[0]).any()
     lat.close()
+
+
+# Records read back in chunks of 65536 live particles: one particle, chunk
+# edges, particles dropped (x = -1e-18 wraps onto the upper face) at the
+# edges, all of them, and a caller's array shorter than the live count.
+@pytest.mark.parametrize("n,dead", [(1, []), (1, [0]), (65536, []), (65537, [0, 65536]), (131073, [65535, 65536, 70000])],
+                         ids=str)
+def test_particle_records_in_chunks(n, dead):
+    import ctypes as C
+    lat = Lattice(configs.poiseuille(8, 8, 8, tau=0.8, g=0.0))
+    lat.initial_conditions()
+    lat.particles_init(abi.make_particle_config(abi.LAGRANGE_WRAP, 1))
+    rng = np.random.default_rng(n)
+    a = np.zeros(n, dtype=abi.particle_dtype())
+    for k in a.dtype.names:
+        a[k] = rng.uniform(1.0, 7.0, n)
+    a["name"], a["tau_drag"] = np.arange(n), 0.0
+    for k in ("vx_old", "vy_old", "vz_old"):  # tracers of a fluid at rest stay where they are
+        a[k] = 0.0
+    a["x"][dead] = -1e-18
+    lat.set_particles(a)
+    back = lat.particles()
+    assert all(np.array_equal(back[k], a[k]) for k in a.dtype.names)
+    lat.step(1)
+    alive = np.setdiff1d(np.arange(n), dead)
+    back = lat.particles()
+    assert np.array_equal(back["name"], alive) and np.array_equal(back["y"], a["y"][alive])
+    assert np.array_equal(back["jump_time"], a["jump_time"][alive])
+    short = np.zeros(max(len(alive) // 2, 1) + 1, dtype=a.dtype)
+    got = C.c_int64()
+    cap = len(short) - 1
+    assert lat._L.ch4g_get_particles(lat.handle, short.ctypes.data, cap, C.byref(got)) == 0
+    assert got.value == len(alive)
+    m = min(cap, len(alive))
+    assert np.array_equal(short[:m], back[:m]) and not short[-1:].view(np.float64).any()
+    lat.close()
