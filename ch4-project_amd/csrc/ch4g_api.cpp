@@ -98,48 +98,74 @@ void hit_walk(ch4g_lattice *L)
         }
 }
 
-// sin(2 pi (k x / L + phi)) tables of the current phases (forcing.c:582-584).
+// sin(2 pi (k x / L + phi)) tables of the current phases (forcing.c:582-584);
+// a mode with k = 0 along an axis has one value there.
 void hit_tables(const ch4g_lattice *L, double *h)
 {
-    const int NX = L->cfg.NX, NY = L->cfg.NY, NZ = L->cfg.NZ;
-    const double LX = NX, LY = NY, LZ = NZ;
-    double *sx = h, *sy = h + CH4G_HIT_NK * NX, *sz = sy + CH4G_HIT_NK * NY;
-    for (int ii = 0; ii < CH4G_HIT_NK; ii++) {
-        for (int i = 0; i < NX; i++) {
-            double x = (double)i + 0.5;
-            sx[ii * NX + i] = sin(2 * 3.14159265359 * (L->vk[ii][0] * x / LX + L->phi[ii][0]));
-        }
-        for (int j = 0; j < NY; j++) {
-            double y = (double)j + 0.5;
-            sy[ii * NY + j] = sin(2 * 3.14159265359 * (L->vk[ii][1] * y / LY + L->phi[ii][1]));
-        }
-        for (int k = 0; k < NZ; k++) {
-            double z = (double)k + 0.5;
-            sz[ii * NZ + k] = sin(2 * 3.14159265359 * (L->vk[ii][2] * z / LZ + L->phi[ii][2]));
+    const int n[3] = {L->cfg.NX, L->cfg.NY, L->cfg.NZ};
+    for (int a = 0; a < 3; a++) {
+        const double LA = n[a];
+        for (int ii = 0; ii < CH4G_HIT_NK; ii++, h += n[a]) {
+            const double k = L->vk[ii][a], phi = L->phi[ii][a];
+            if (k == 0.0) {
+                const double v = sin(2 * 3.14159265359 * (0.0 + phi));
+                for (int i = 0; i < n[a]; i++) h[i] = v;
+            } else {
+                for (int i = 0; i < n[a]; i++) {
+                    const double x = (double)i + 0.5;
+                    h[i] = sin(2 * 3.14159265359 * (k * x / LA + phi));
+                }
+            }
         }
     }
 }
 
-// Upload the tables of the current phases into device slot `slot`.
-int hit_upload(ch4g_lattice *L, int slot)
+// Tables of `count` steps (each after one more step of the phase walk, or of
+// the phases as they are) to the device in one copy.  One table and one copy
+// per step kept small lattices waiting for the host (19^3 12 us per step, of
+// which the kernel 5).
+int hit_upload(ch4g_lattice *L, int count, bool walk)
 {
-    int r = L->ring;
+    const int r = L->ring;
     L->ring = (L->ring + 1) % HIT_RING;
     HIPCHK(hipEventSynchronize(L->ev_ring[r]));
-    hit_tables(L, L->h_ring[r]);
-    HIPCHK(hipMemcpyAsync(L->d_hit[slot], L->h_ring[r], L->hit_len * sizeof(double), hipMemcpyHostToDevice,
-                          L->stream));
+    for (int k = 0; k < count; k++) {
+        if (walk) hit_walk(L);
+        hit_tables(L, L->h_ring[r] + (size_t)k * L->hit_len);
+    }
+    // the other half holds the table of the current force
+    L->hit_half ^= 1;
+    HIPCHK(hipMemcpyAsync(L->d_hit[L->hit_half], L->h_ring[r], (size_t)count * L->hit_len * sizeof(double),
+                          hipMemcpyHostToDevice, L->stream));
     HIPCHK(hipEventRecord(L->ev_ring[r], L->stream));
+    L->hit_at = L->d_hit[L->hit_half];
+    L->hit_have = count;
     return 0;
 }
 
-// build_forcing at initialisation (main.c:38): one phase step, tables of
-// Phi_1 into slot 1 (the force of step 0).
+// The next table made ahead becomes that of the current force.
+void hit_take(ch4g_lattice *L)
+{
+    L->hit_cur = L->hit_at;
+    L->hit_at += L->hit_len;
+    L->hit_have--;
+}
+
+// build_forcing at initialisation (main.c:38): one phase step, the table of
+// Phi_1 (the force of step 0).
 int first_build_forcing(ch4g_lattice *L)
 {
     if (!has(L->cfg, CH4G_FLUID_FORCING_HIT)) return 0;
-    hit_walk(L);
-    return hit_upload(L, (int)((L->itime + 1) & 1));
+    const int rc = hit_upload(L, 1, true);
+    if (rc) return rc;
+    hit_take(L);
+    return 0;
+}
+
+HitTable hit_table(const ch4g_lattice *L, const double *t)
+{
+    const int NX = L->cfg.NX, NY = L->cfg.NY;
+    return {t, t + CH4G_HIT_NK * NX, t + CH4G_HIT_NK * (NX + NY)};
 }
 
 }  // namespace
@@ -162,16 +188,8 @@ KParams params_for(const ch4g_lattice *L, int first, int itime)
             P.fb_now = (const double *)L->part->d_fb[itime & 1];
         }
     }
-    if (P.hit) {
-        const int NX = L->cfg.NX, NY = L->cfg.NY;
-        int sp = itime & 1, sn = (itime + 1) & 1;
-        P.hit_prev.sx = L->d_hit[sp];
-        P.hit_prev.sy = L->d_hit[sp] + CH4G_HIT_NK * NX;
-        P.hit_prev.sz = L->d_hit[sp] + CH4G_HIT_NK * (NX + NY);
-        P.hit_now.sx = L->d_hit[sn];
-        P.hit_now.sy = L->d_hit[sn] + CH4G_HIT_NK * NX;
-        P.hit_now.sz = L->d_hit[sn] + CH4G_HIT_NK * (NX + NY);
-    }
+    // the current force's table; a step replaces hit_now by the next one
+    if (P.hit) P.hit_prev = P.hit_now = hit_table(L, L->hit_cur);
     return P;
 }
 
@@ -234,29 +252,29 @@ void destroy_graphs(ch4g_lattice *L)
 
 namespace {
 
-// One step: host forcing tables (HIT), then the fused kernel.
-int launch_one_step(ch4g_lattice *L)
+// One step: host forcing tables (HIT), then the fused kernel.  `ahead`: steps
+// of the call from this one on whose tables may be made now.
+int launch_one_step(ch4g_lattice *L, int ahead)
 {
     int itime = (int)L->itime + 1;
-    if (L->base.hit) {
-        // build_forcing of this step: Phi_{itime+1}
-        if (L->part && L->part->rng_on_device) {
-            int rc = rng_to_host(L);
-            if (rc) return rc;
-        }
-        hit_walk(L);
-        if (L->part && L->part->rng_on_device) {
-            int rc = rng_to_device(L);
-            if (rc) return rc;
-        }
-        int rc = hit_upload(L, (itime + 1) & 1);
+    if (L->base.hit && L->hit_have == 0) {
+        // build_forcing of this step: Phi_{itime+1}; with the drand48 stream on
+        // the device its draws come in between, one step at a time
+        const bool dev_rng = L->part && L->part->rng_on_device;
+        int rc = dev_rng ? rng_to_host(L) : 0;
         if (rc) return rc;
+        if ((rc = hit_upload(L, dev_rng ? 1 : (ahead < HIT_AHEAD ? ahead : HIT_AHEAD), true))) return rc;
+        if (dev_rng && (rc = rng_to_device(L))) return rc;
     }
     if (L->part) {
         int rc = particles_before_step(L, itime);
         if (rc) return rc;
     }
     KParams P = params_for(L, L->first, itime);
+    if (P.hit) {
+        hit_take(L);
+        P.hit_now = hit_table(L, L->hit_cur);
+    }
     // the particles of the previous step move on the fields this kernel gathers
     const bool fused = L->part && L->part->pending;
     if (fused) {
@@ -367,7 +385,7 @@ int replay_graph(ch4g_lattice *L)
         if (two_step_eligible(L)) {
             for (int k = 0; k < GRAPH_STEPS / 2 && !rc; k++) rc = launch_two_steps(L);
         } else {
-            for (int k = 0; k < GRAPH_STEPS && !rc; k++) rc = launch_one_step(L);
+            for (int k = 0; k < GRAPH_STEPS && !rc; k++) rc = launch_one_step(L, 1);
         }
         hipError_t e = hipStreamEndCapture(L->stream, &g);
         // capture records work without running it: restore the counters
@@ -609,9 +627,11 @@ int ch4g_create(const ch4g_config *cfg, ch4g_lattice **out)
     if (L->base.hit) {
         L->hit_len = (size_t)CH4G_HIT_NK * (cfg->NX + cfg->NY + cfg->NZ);
         for (int b = 0; b < 2; b++)
-            if ((rc = dalloc(L, (void **)&L->d_hit[b], L->hit_len * sizeof(double)))) goto err;
+            if ((rc = dalloc(L, (void **)&L->d_hit[b], HIT_AHEAD * L->hit_len * sizeof(double)))) goto err;
+        L->hit_cur = L->d_hit[0];
         for (int r = 0; r < HIT_RING; r++) {
-            hipError_t e = hipHostMalloc((void **)&L->h_ring[r], L->hit_len * sizeof(double), hipHostMallocDefault);
+            hipError_t e = hipHostMalloc((void **)&L->h_ring[r], HIT_AHEAD * L->hit_len * sizeof(double),
+                                         hipHostMallocDefault);
             if (e != hipSuccess) {
                 rc = fail(-3, "hipHostMalloc failed: %s", hipGetErrorString(e));
                 goto err;
@@ -764,6 +784,9 @@ int ch4g_step(ch4g_lattice *L, int nsteps)
     if (!L) return fail(-1, "null lattice");
     if (nsteps < 0) return fail(-1, "negative step count");
     int s = 0;
+    // HIT tables ahead: 1, 2, 4, ... steps, so that the first kernel does not
+    // wait for all of them
+    int ahead = 1;
     while (s < nsteps) {
         // Steady-state steps (not the first, no per-step host forcing tables,
         // no particles) depend only on the buffer parities: replay a captured
@@ -780,8 +803,10 @@ int ch4g_step(ch4g_lattice *L, int nsteps)
             s += 2;
             continue;
         }
-        int rc = launch_one_step(L);
+        const bool refill = L->hit_have == 0;
+        int rc = launch_one_step(L, ahead < nsteps - s ? ahead : nsteps - s);
         if (rc) return rc;
+        if (refill && ahead < HIT_AHEAD) ahead *= 2;
         s++;
     }
     return particles_flush(L);
@@ -1032,7 +1057,10 @@ int ch4g_set_hit_phases(ch4g_lattice *L, const double *phi)
     if (!L || !phi) return fail(-1, "null argument");
     if (!L->base.hit) return fail(-1, "lattice has no HIT forcing");
     memcpy(L->phi, phi, sizeof L->phi);
-    return hit_upload(L, (int)((L->itime + 1) & 1));
+    const int rc = hit_upload(L, 1, false);
+    if (rc) return rc;
+    hit_take(L);
+    return 0;
 }
 
 int ch4g_synchronize(ch4g_lattice *L)

@@ -10,7 +10,10 @@
 
 namespace ch4g {
 
-constexpr int HIT_RING = 8;
+// HIT tables of up to HIT_AHEAD steps go to the device in one copy, from one
+// of HIT_RING pinned buffers
+constexpr int HIT_RING = 2;
+constexpr int HIT_AHEAD = 8;
 // steps between reorderings of the particle rows by cell
 constexpr int REORDER_STEPS = 32;
 // steps per captured graph (even: the graph starts and ends on the same buffer)
@@ -85,11 +88,15 @@ struct ch4g_lattice {
     // constants of the step
     ch4g::KParams base;
     double nu = 0, kappa = 0, deltaT = 0;
-    // HIT forcing: phases of the current force (Phi_{itime+1}), device tables
-    // for the two most recent steps, pinned staging ring
+    // HIT forcing: phases of the last table made, device tables (two halves of
+    // HIT_AHEAD, written in turn), pinned staging ring
     double phi[CH4G_HIT_NK][3];
     double vk[CH4G_HIT_NK][3];
     double *d_hit[2] = {nullptr, nullptr};
+    int hit_half = 0;                // half the last copy went to
+    const double *hit_cur = nullptr; // table of the current force
+    const double *hit_at = nullptr;  // next table made ahead,
+    int hit_have = 0;                // and how many there are
     // LB_FLUID_FORCING_NOZEROMODE: means [6] + block partial sums [512][6]
     double *d_f0 = nullptr;
     double *h_ring[ch4g::HIT_RING] = {};
