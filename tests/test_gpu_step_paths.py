@@ -148,3 +148,45 @@ def test_particle_records_in_chunks(n, dead):
     m = min(cap, len(alive))
     assert np.array_equal(short[:m], back[:m]) and not short[-1:].view(np.float64).any()
     lat.close()
+
+
+# HIT tables made ahead (batches of 1, 2, 4, 8, 8, ... steps in a call, cut at
+# its end): calls of every length to past three batches, one step at a time,
+# and new phases between calls give the same states, bit for bit, and the
+# oracle's phases; also with the drand48 stream on the device (randomly
+# oriented particles draw from it between two steps' walks).
+@pytest.mark.parametrize("shape,draws", [(12, False), (19, False), (12, True)], ids=str)
+def test_hit_tables_ahead(shape, draws):
+    cfg = configs.hit(shape, tau=0.55, amp=1e-4, les=False)
+    calls = [1, 2, 3, 7, 8, 9, 15, 16, 17, 31]
+    if draws:
+        flags = (abi.LAGRANGE_ADD_TRACER | abi.LAGRANGE_WRAP | abi.LAGRANGE_GRADIENT | abi.LAGRANGE_ADDEDMASS |
+                 abi.LAGRANGE_ORIENTATION | abi.LAGRANGE_ORIENTATION_JEFFREY)
+        pc = abi.make_particle_config(flags, 50, aspect_ratio=(2, 0.5, 4.0), flags2=abi.LAGRANGE_ORIENTATION_RANDOM)
+
+    def advance(x, single):
+        x.initial_conditions()
+        if draws:
+            x.particles_init(pc)
+        for n in calls:
+            if single:
+                for _ in range(n):
+                    x.step(1)
+            else:
+                x.step(n)
+        return x
+
+    a, b, o = advance(Lattice(cfg), False), advance(Lattice(cfg), True), advance(Oracle(cfg), False)
+    np.testing.assert_array_equal(a.hit_phases(), o.hit_phases())
+    np.testing.assert_array_equal(b.hit_phases(), o.hit_phases())
+    pa, pb = a.get_populations()[0], b.get_populations()[0]
+    assert np.array_equal(pa, pb)
+    new = o.hit_phases()[::-1] * 0.5 + 0.125
+    for x in (a, b):
+        x.set_hit_phases(new)
+    a.step(5)
+    for _ in range(5):
+        b.step(1)
+    assert np.array_equal(a.get_populations()[0], b.get_populations()[0])
+    a.close()
+    b.close()
