@@ -331,11 +331,22 @@ int launch_one_step(ch4g_lattice *L, int ahead)
 
 namespace ch4g {
 
-// Two steady-state steps in one launch (2-D FP32-storage lattices, see
-// two_step_ok): the lag moves to the other array.
+// Two steady-state steps in one launch (see two_step_ok, two_step_ok64): the
+// lag moves to the other array.
 bool two_step_eligible(const ch4g_lattice *L)
 {
-    return L->use_fusion && L->dev32 && !L->first && !L->part && two_step_ok(L->base);
+    return L->use_fusion && !L->first && !L->part && (L->dev32 ? two_step_ok(L->base) : two_step_ok64(L->base));
+}
+
+// the launch, from buffers `in` and lag array `tl` to the others
+void two_steps_on(const ch4g_lattice *L, const KParams &P, int in, const void *tl, void *ta, hipStream_t s)
+{
+    if (L->dev32)
+        launch_two_steps_fp32(P, (const float *)L->f[in], (const float *)L->g[in], (float *)L->f[in ^ 1],
+                              (float *)L->g[in ^ 1], (const float *)tl, (float *)ta, s);
+    else
+        launch_two_steps_fp64(P, (const double *)L->f[in], (const double *)L->g[in], (double *)L->f[in ^ 1],
+                              (double *)L->g[in ^ 1], (const double *)tl, (double *)ta, s);
 }
 
 int ensure_tlag_alt(ch4g_lattice *L)
@@ -344,18 +355,26 @@ int ensure_tlag_alt(ch4g_lattice *L)
     return 0;
 }
 
+// ... with the second lag array in place; single steps where no memory is left
+bool two_step_ready(ch4g_lattice *L)
+{
+    if (!two_step_eligible(L)) return false;
+    if (!ensure_tlag_alt(L)) return true;
+    (void)hipGetLastError();
+    g_err[0] = 0;
+    L->use_fusion = false;
+    return false;
+}
+
 }  // namespace ch4g
 
 namespace {
 
 int launch_two_steps(ch4g_lattice *L)
 {
-    int rc = ensure_tlag_alt(L); // allocated before any capture (replay_graph)
-    if (rc) return rc;
-    KParams P = params_for(L, 0, (int)L->itime + 1);
+    const KParams P = params_for(L, 0, (int)L->itime + 1);
     const int in = L->cur, out = 1 - L->cur;
-    launch_two_steps_fp32(P, (const float *)L->f[in], (const float *)L->g[in], (float *)L->f[out],
-                          (float *)L->g[out], (const float *)L->tlag, (float *)L->tlag_alt, L->stream);
+    two_steps_on(L, P, in, L->tlag, L->tlag_alt, L->stream);
     HIPCHK(hipGetLastError());
     L->cur = out;
     if (L->base.thermal) {
@@ -371,10 +390,7 @@ int launch_two_steps(ch4g_lattice *L)
 // buffer parities.
 int replay_graph(ch4g_lattice *L)
 {
-    if (two_step_eligible(L)) {
-        int rc = ensure_tlag_alt(L);
-        if (rc) return rc;
-    }
+    const bool two = two_step_ready(L); // allocates before any capture
     const int start = L->cur | (L->tpar << 1);
     if (!L->graph[start]) {
         hipGraph_t g = nullptr;
@@ -383,7 +399,7 @@ int replay_graph(ch4g_lattice *L)
         const int cur0 = L->cur, tpar0 = L->tpar;
         void *tl0 = L->tlag, *ta0 = L->tlag_alt;
         int rc = 0;
-        if (two_step_eligible(L)) {
+        if (two) {
             for (int k = 0; k < GRAPH_STEPS / 2 && !rc; k++) rc = launch_two_steps(L);
         } else {
             for (int k = 0; k < GRAPH_STEPS && !rc; k++) rc = launch_one_step(L, 1);
@@ -799,7 +815,7 @@ int ch4g_step(ch4g_lattice *L, int nsteps)
             s += GRAPH_STEPS;
             continue;
         }
-        if (nsteps - s >= 2 && two_step_eligible(L)) {
+        if (nsteps - s >= 2 && two_step_ready(L)) {
             int rc = launch_two_steps(L);
             if (rc) return rc;
             s += 2;
@@ -826,7 +842,7 @@ int ch4g_steps_per_launch(const ch4g_lattice *L, int *steps)
     if (!L || !steps) return fail(-1, "null argument");
     ch4g::KParams P = L->base;
     P.first = 0;  // steady state
-    *steps = (L->use_fusion && L->dev32 && !L->part && two_step_ok(P)) ? 2 : 1;
+    *steps = (L->use_fusion && !L->part && (L->dev32 ? two_step_ok(P) : two_step_ok64(P))) ? 2 : 1;
     return 0;
 }
 

@@ -460,9 +460,12 @@ void launch_fields_f32(const KParams &P, const float *fin, const float *gin, con
 // multiple of 64, steady steps without HIT tables, LES or particles): reads
 // the state (f, g in; temperature lag tl_in), writes the state two steps on
 // (f, g out; lag tl_out, a different array).
-bool two_step_ok(const KParams &P);
+bool two_step_ok(const KParams &P);    // float storage
+bool two_step_ok64(const KParams &P);  // FP64
 void launch_two_steps_fp32(const KParams &P, const float *fin, const float *gin, float *fout, float *gout,
                            const float *tl_in, float *tl_out, hipStream_t s);
+void launch_two_steps_fp64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,
+                           const double *tl_in, double *tl_out, hipStream_t s);
 
 // Velocity of the step at every node into P.vel (the finite-difference LES
 // closure reads it at the six neighbours); same gather and moments as the

@@ -139,10 +139,9 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         ch4g_lattice *L = lats[i];
         // two steps per launch: 2-D lattices in the batched two-step kernel,
         // large 3-D lattices on their own branch
-        B.two[i] = two_step_eligible(L);
+        B.two[i] = two_step_ready(L);
         solo[i] = B.two[i] && L->cfg.NZ > 1;
         if (solo[i]) B.solo.push_back((int)i);
-        if (B.two[i] && (rc = ensure_tlag_alt(L))) return rc;
         // two-step lattices: the population buffer flips with every launch,
         // the lag array with every two-step launch
         const int pairs = steps[i] / 2, launches = pairs + steps[i] % 2;
@@ -306,14 +305,16 @@ int launch_steps(Batch &B)
         int cur = L->cur;
         void *tl = L->tlag, *ta = L->tlag_alt;
         for (int s_ = 0; s_ + 1 < st; s_ += 2) {
-            launch_two_steps_fp32(P, (const float *)L->f[cur], (const float *)L->g[cur], (float *)L->f[cur ^ 1],
-                                  (float *)L->g[cur ^ 1], (const float *)tl, (float *)ta, t);
+            two_steps_on(L, P, cur, tl, ta, t);
             cur ^= 1;
             if (L->base.thermal) std::swap(tl, ta);
         }
-        if (st & 1)
+        if ((st & 1) && L->dev32)
             launch_step_fp32(P, (const float *)L->f[cur], (const float *)L->g[cur], (float *)L->f[cur ^ 1],
                              (float *)L->g[cur ^ 1], (float *)tl, (float *)L->taules, t);
+        else if (st & 1)
+            launch_step_fp64(P, (const double *)L->f[cur], (const double *)L->g[cur], (double *)L->f[cur ^ 1],
+                             (double *)L->g[cur ^ 1], (double *)tl, (double *)L->taules, t);
         HIPCHK(hipEventRecord(B.sdone[k], t));
     }
     for (size_t g = 0; g < ng; g++) {

@@ -14,6 +14,7 @@
 // the lagged temperature, as main.c's ordering implies), then collides
 // (fluid.c:1033-1225) and adds the Guo term (forcing.c:1424-1435) of step s.
 #include "ch4g_planes.h"
+#include "ch4g_ztile.h"
 
 namespace ch4g {
 
@@ -342,90 +343,106 @@ __device__ __forceinline__ void fluid_velocity64(const KParams &P, const double 
     }
 }
 
-// Collision and force of one node's gathered populations f (and g, of sum T);
-// shared by every step kernel, so a lattice advances bit-identically in all.
+// What the fluid's collision leaves for the temperature's.
+struct Moved64 {
+    double ux = 0.0, uy = 0.0, uz = 0.0, tau_les = 0.0;
+};
+
+// Collision and force of one node's gathered populations, shared by every
+// step kernel, so a lattice advances bit-identically in all: the fluid's f...
+template <bool GEN, class OutF>
+__device__ __forceinline__ void collide_fluid64(const KParams &P, const Nbr &b, const double f[Q], double Tlag, double T,
+                                                double *__restrict__ taules, uint32_t n, const OutF &outf, Moved64 &mv)
+{
+    const int x = b.x, y = b.y, z = b.z;
+    double &ux = mv.ux, &uy = mv.uy, &uz = mv.uz, &tau_les = mv.tau_les;
+    double rho;
+    fluid_velocity64<GEN>(P, f, n, x, y, z, Tlag, rho, ux, uy, uz);
+    const double u2z = u2_of(ux, uy, uz);
+    double invtau = P.invtau_u;
+    if (GEN && P.les) {
+        if (P.les_fd) {
+            tau_les = les_tau_fd(P, (const double *)P.vel, b, n);
+        } else {
+            double tau_prev = (P.itime == 1) ? P.tau_u : taules[n];
+            tau_les = les_tau(P, f, rho, ux, uy, uz, u2z, tau_prev);
+        }
+        taules[n] = tau_les;
+        invtau = 1.0 / tau_les;
+    }
+    double Fn[3] = {0.0, 0.0, 0.0};
+    if (P.forced) force_at<GEN>(P, P.hit_now, P.fb_now, P.f0n, n, x, y, z, T, Fn);
+    // r += guo w rho F . ((c - u) / cs^2 + c (c.u) / cs^4), components in
+    // order; s = +1 for q, -1 for its opposite (c (c.u) is the same for both)
+    const double gf[3] = {P.guo_fac * wq(0) * rho, P.guo_fac * wq(1) * rho, P.guo_fac * wq(7) * rho};
+    auto guo = [&](auto qc, double s, double cc, double &r) {
+        constexpr int q = decltype(qc)::value, wc = q == 0 ? 0 : (q <= 6 ? 1 : 2);
+        constexpr int c[3] = {cxq(q), cyq(q), czq(q)};
+        const double u[3] = {ux, uy, uz};
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            const double ca = c[a] * s;  // 0 or +-1, known at compile time
+            double d = (ca - u[a]) * P.invcs2;
+            if (c[a] != 0) d += c[a] > 0 ? cc : -cc;
+            r += gf[wc] * Fn[a] * d;
+        }
+    };
+    {
+        double r = f[0];
+        r += -invtau * (f[0] - feq_rest(P, rho, u2z));
+        if (P.forced) guo(std::integral_constant<int, 0>{}, 1.0, 0.0, r);
+        outf.template put<0>(r);
+    }
+    static_for<0, 9>([&](auto kk) {
+        constexpr int q = pair64(decltype(kk)::value), qb = invq(q);
+        const EqPair e = feq_pair<q>(P, rho, ux, uy, uz, u2z);
+        double r = f[q], rb = f[qb];
+        r += -invtau * (f[q] - e.eq);
+        rb += -invtau * (f[qb] - e.eqb);
+        if (P.forced) {
+            const double cc = e.cu * P.invcs4;
+            guo(std::integral_constant<int, q>{}, 1.0, cc, r);
+            guo(std::integral_constant<int, q>{}, -1.0, cc, rb);
+        }
+        outf.template put<q>(r);
+        outf.template put<qb>(rb);
+    });
+}
+
+// ... and the temperature's g, of sum T.
+template <bool FLUID, bool GEN, class OutG>
+__device__ __forceinline__ void collide_thermal64(const KParams &P, const double g[Q], double T, const Moved64 &mv,
+                                                  const OutG &outg)
+{
+    const double ux = mv.ux, uy = mv.uy, uz = mv.uz, tau_les = mv.tau_les;
+    const double u2z = u2_of(ux, uy, uz);
+    double invtau_t = P.invtau_t;
+    if constexpr (FLUID)
+        if (GEN && P.les_t) invtau_t = 1.0 / les_tau_t(P, tau_les);
+    {
+        double r = g[0];
+        r += -invtau_t * (g[0] - feq_rest(P, T, u2z));
+        outg.template put<0>(r);
+    }
+    static_for<0, 9>([&](auto kk) {
+        constexpr int q = pair64(decltype(kk)::value), qb = invq(q);
+        const EqPair e = feq_pair<q>(P, T, ux, uy, uz, u2z);
+        double r = g[q], rb = g[qb];
+        r += -invtau_t * (g[q] - e.eq);
+        rb += -invtau_t * (g[qb] - e.eqb);
+        outg.template put<q>(r);
+        outg.template put<qb>(rb);
+    });
+}
+
 template <bool FLUID, bool THERMAL, bool GEN, class OutF, class OutG>
 __device__ __forceinline__ void collide64(const KParams &P, const Nbr &b, const double f[Q], const double g[Q],
                                           double Tlag, double T, double *__restrict__ taules, uint32_t n,
                                           const OutF &outf, const OutG &outg)
 {
-    const int x = b.x, y = b.y, z = b.z;
-    double ux = 0.0, uy = 0.0, uz = 0.0;
-    double tau_les = 0.0;
-    if constexpr (FLUID) {
-        double rho;
-        fluid_velocity64<GEN>(P, f, n, x, y, z, Tlag, rho, ux, uy, uz);
-        const double u2z = u2_of(ux, uy, uz);
-        double invtau = P.invtau_u;
-        if (GEN && P.les) {
-            if (P.les_fd) {
-                tau_les = les_tau_fd(P, (const double *)P.vel, b, n);
-            } else {
-                double tau_prev = (P.itime == 1) ? P.tau_u : taules[n];
-                tau_les = les_tau(P, f, rho, ux, uy, uz, u2z, tau_prev);
-            }
-            taules[n] = tau_les;
-            invtau = 1.0 / tau_les;
-        }
-        double Fn[3] = {0.0, 0.0, 0.0};
-        if (P.forced) force_at<GEN>(P, P.hit_now, P.fb_now, P.f0n, n, x, y, z, T, Fn);
-        // r += guo w rho F . ((c - u) / cs^2 + c (c.u) / cs^4), components in
-        // order; s = +1 for q, -1 for its opposite (c (c.u) is the same for both)
-        const double gf[3] = {P.guo_fac * wq(0) * rho, P.guo_fac * wq(1) * rho, P.guo_fac * wq(7) * rho};
-        auto guo = [&](auto qc, double s, double cc, double &r) {
-            constexpr int q = decltype(qc)::value, wc = q == 0 ? 0 : (q <= 6 ? 1 : 2);
-            constexpr int c[3] = {cxq(q), cyq(q), czq(q)};
-            const double u[3] = {ux, uy, uz};
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                const double ca = c[a] * s;  // 0 or +-1, known at compile time
-                double d = (ca - u[a]) * P.invcs2;
-                if (c[a] != 0) d += c[a] > 0 ? cc : -cc;
-                r += gf[wc] * Fn[a] * d;
-            }
-        };
-        {
-            double r = f[0];
-            r += -invtau * (f[0] - feq_rest(P, rho, u2z));
-            if (P.forced) guo(std::integral_constant<int, 0>{}, 1.0, 0.0, r);
-            outf.template put<0>(r);
-        }
-        static_for<0, 9>([&](auto kk) {
-            constexpr int q = pair64(decltype(kk)::value), qb = invq(q);
-            const EqPair e = feq_pair<q>(P, rho, ux, uy, uz, u2z);
-            double r = f[q], rb = f[qb];
-            r += -invtau * (f[q] - e.eq);
-            rb += -invtau * (f[qb] - e.eqb);
-            if (P.forced) {
-                const double cc = e.cu * P.invcs4;
-                guo(std::integral_constant<int, q>{}, 1.0, cc, r);
-                guo(std::integral_constant<int, q>{}, -1.0, cc, rb);
-            }
-            outf.template put<q>(r);
-            outf.template put<qb>(rb);
-        });
-    }
-
-    if constexpr (THERMAL) {
-        const double u2z = u2_of(ux, uy, uz);
-        double invtau_t = P.invtau_t;
-        if constexpr (FLUID)
-            if (GEN && P.les_t) invtau_t = 1.0 / les_tau_t(P, tau_les);
-        {
-            double r = g[0];
-            r += -invtau_t * (g[0] - feq_rest(P, T, u2z));
-            outg.template put<0>(r);
-        }
-        static_for<0, 9>([&](auto kk) {
-            constexpr int q = pair64(decltype(kk)::value), qb = invq(q);
-            const EqPair e = feq_pair<q>(P, T, ux, uy, uz, u2z);
-            double r = g[q], rb = g[qb];
-            r += -invtau_t * (g[q] - e.eq);
-            rb += -invtau_t * (g[qb] - e.eqb);
-            outg.template put<q>(r);
-            outg.template put<qb>(rb);
-        });
-    }
+    Moved64 mv;
+    if constexpr (FLUID) collide_fluid64<GEN>(P, b, f, Tlag, T, taules, n, outf, mv);
+    if constexpr (THERMAL) collide_thermal64<FLUID, GEN>(P, g, T, mv, outg);
 }
 
 // One node of the fused step.  UNI: what the wave shares (Pull).  BUF: planes
@@ -486,6 +503,146 @@ __global__ void __launch_bounds__(256) k_step_fp64(KParams P, const double *__re
         n = row * (uint32_t)P.NX + x;
     }
     step_node64<FIRST, FLUID, THERMAL, NT, GEN, BUF, DENSE ? PULL_LINEAR : PULL_ROW>(P, fin, gin, fout, gout, tlag, taules, x, y, z, n);
+}
+
+// Results of a node kept in registers (step A of k_step2z_fp64)
+struct RegOut64 {
+    double *__restrict__ r;
+    template <int q>
+    __device__ void put(double v) const
+    {
+        r[q] = v;
+    }
+};
+
+// Two steps per launch for 3-D lattices: k_step2z_fp32's march along z
+// (ch4g_ztile.h) with this file's arithmetic, so the same bits as two single
+// steps.
+//
+// A single step moves the state at 5 TB/s and is bound by that; here it is
+// read (with the tile's halo, 1.33 times) and written once per two steps.  us
+// per step, single -> this: Rayleigh-Benard 96^3 112 -> 81, 128^3 249 -> 186,
+// 185^3 752 -> 589, 256^3 1996 -> 1492, 96x80x112 111 -> 83; channel 113^3
+// 91 -> 72, 128^3 120 -> 86, 192^3 413 -> 280.  An iteration (11.6 us at 256^3)
+// is now loads, collision, barrier, collision and stores in turn, one block
+// per CU: bound by their latencies.  us per step at 256^3 of what did not
+// help: the temperature's populations gathered once in step B (9 registers
+// spilled) 1564; 64 x 4 tiles 1498 (96^3 98), 32 x 9 1543, 16 x 16 1711, two
+// blocks of 16 x 8 per CU 1826; the next plane's loads in flight during B
+// (53 registers spilled) 2663, its lines touched ahead 1542.
+template <bool FLUID, bool THERMAL, bool NT, class TZ>
+__global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp64(KParams P, const double *__restrict__ fin,
+                                                             const double *__restrict__ gin, double *__restrict__ fout,
+                                                             double *__restrict__ gout,
+                                                             const double *__restrict__ tl_in,
+                                                             double *__restrict__ tl_out, int zc)
+{
+    constexpr int M = TZ::M, W = TZ::W, TX = TZ::TX, TY = TZ::TY;
+    static_assert(TZ::HOLD, "one slot of ring Z");
+    __shared__ double t[TZ::REALS];
+    const int NX = P.NX, NY = P.NY, NZ = P.NZ;
+    const uint32_t nbx = gridDim.x, nby = gridDim.y;
+    const uint32_t bid = xcd_block(block_linear(), nbx * nby * gridDim.z);
+    const int x0 = (int)(bid % nbx) * TX, y0 = (int)((bid / nbx) % nby) * TY;
+    const int zb = (int)(bid / (nbx * nby)) * zc, ze = min(zb + zc, NZ);
+    const int w = NX - x0 < TX ? NX - x0 : TX;
+    // step A node of this thread (tile + halo)
+    const int m = threadIdx.x, lx = m % W, ly = m / W;
+    const bool act_a = m < M && lx <= w + 1;
+    int xa = x0 - 1 + lx;
+    xa = xa < 0 ? xa + NX : (xa >= NX ? xa - NX : xa);
+    int ya = (y0 - 1 + ly) % NY;
+    ya = ya < 0 ? ya + NY : ya;
+    const bool tile_a = act_a && lx >= 1 && lx <= w && ly >= 1 && ly <= TY;
+    const int tn_a = (ly - 1) * TX + (lx - 1);
+    // step B node of this thread (tile)
+    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+    const int xb = x0 + tx, yb = y0 + ty;
+    const bool act_b = ty < TY && tx < w && yb < NY;
+    const int at = (ty + 1) * W + tx + 1, tn = ty * TX + tx;
+
+    const Planes<double> pin_f = make_planes(FLUID ? fin : gin, P.S), pin_g = make_planes(THERMAL ? gin : fin, P.S);
+    const Planes<double> pout_f = make_planes(FLUID ? fout : gout, P.S),
+                         pout_g = make_planes(THERMAL ? gout : fout, P.S);
+    // step A's node at iteration it (plane zb - 1 + it, periodic in z)
+    auto node_a = [&](int it) {
+        const int j = zb - 1 + it;
+        return make_nbr(xa, ya, j < 0 ? j + NZ : (j >= NZ ? j - NZ : j), NX, NY, NZ);
+    };
+    auto index = [&](const Nbr &b) { return ((uint32_t)b.z * NY + b.y) * NX + b.x; };
+    // the fixed-temperature rule of pull_thermal64
+    auto walls = [&](const Nbr &b, double Tlag, double (&g)[Q]) {
+        const double fac_top = 2.0 * (P.Tw_top - Tlag);
+        const double fac_bot = 2.0 * (P.Tw_bot - Tlag);
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            const bool cross = P.wall_t && crosses_wall<q>(b);
+            if constexpr (cyq(q) > 0) g[q] = cross ? g[q] + wq(q) * fac_bot : g[q];
+            if constexpr (cyq(q) < 0) g[q] = cross ? g[q] + wq(q) * fac_top : g[q];
+        });
+    };
+    const int nit = ze - zb + 2;
+    for (int it = 0; it < nit; it++) {
+        double rf[Q], rg[Q], rt = 0.0;
+        // ---- A: step 1 at plane zb - 1 + it
+        if (act_a) {
+            const Nbr b = node_a(it);
+            const uint32_t n = index(b);
+            const Pull<double, PULL_LINEAR> o(b, NX, NY);
+            double f[Q], g[Q], Tlag = 0.0;
+            if constexpr (THERMAL) {
+                Tlag = tl_in[n];
+                pull_thermal64(P, b, pin_g, o, Tlag, g);
+            }
+            if constexpr (FLUID) pull_fluid64(P, b, pin_f, o, f);
+            if constexpr (THERMAL) rt = m_sum(g);
+            collide64<FLUID, THERMAL, false>(P, b, f, g, Tlag, rt, nullptr, n, RegOut64{rf}, RegOut64{rg});
+            ring_put<TZ, FLUID, THERMAL>(t, m, it, rf, rg, rt, tile_a, tn_a, true, false);
+        }
+        __syncthreads();
+        // ---- B: step 2 one plane below (planes of the block's range only)
+        const int p = zb - 2 + it;
+        if (act_b && p >= zb) {
+            const Nbr b = make_nbr(xb, yb, p, NX, NY, NZ);
+            const RingSlots<TZ> rs(it);
+            const Pull<double, PULL_LINEAR> o(b, NX, NY);
+            double Tlag = 0.0, T = 0.0;
+            Moved64 mv;
+            // read twice, for T and for the collision, so that they hold no
+            // registers during the fluid's
+            auto g_of = [&](double (&g)[Q]) {
+                static_for<0, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    g[q] = ring_src<TZ, q, 1>(t, at, tn, rs, P.wall_t && crosses_wall<q>(b));
+                });
+                walls(b, Tlag, g);
+            };
+            if constexpr (THERMAL) {
+                double g[Q];
+                Tlag = t[TZ::lag(rs.z) * M + at];
+                g_of(g);
+                T = m_sum(g);
+                tl_out[index(b)] = T;
+            }
+            if constexpr (FLUID) {
+                double f[Q];
+                static_for<0, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    f[q] = ring_src<TZ, q, 0>(t, at, tn, rs, P.wall_f && crosses_wall<q>(b));
+                });
+                collide_fluid64<false>(P, b, f, Tlag, T, nullptr, 0u, PlaneOut<NT, PULL_LINEAR>{pout_f, o}, mv);
+            }
+            if constexpr (THERMAL) {
+                asm volatile("" ::: "memory");
+                double g[Q];
+                g_of(g);
+                collide_thermal64<FLUID, false>(P, g, T, mv, PlaneOut<NT, PULL_LINEAR>{pout_g, o});
+            }
+        }
+        __syncthreads();
+        // ---- C: the c_z >= 0 results of A into rings Z, P, W
+        if (act_a) ring_put<TZ, FLUID, THERMAL>(t, m, it, rf, rg, rt, tile_a, tn_a, false, true);
+    }
 }
 
 // Velocity of the step at every node (the u[] that add_collision reads,
@@ -660,6 +817,57 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
         sets(std::true_type{}, std::false_type{});
     else
         sets(std::false_type{}, std::true_type{});
+}
+
+// Two steps per launch (k_step2z_fp64): 3-D lattices with the fluid whose
+// planes buffer resources reach, without the general force paths.
+// Tiles: 32 x 8 with the temperature (141 KB of LDS), 64 x 8 without (135 KB).
+using Tile64 = TileZ<true, true, 32, 8, true>;
+using Tile64F = TileZ<true, false, 64, 8, true>;
+
+static int64_t z_columns64(const KParams &P)
+{
+    const int tx = P.thermal ? Tile64::TX : Tile64F::TX, ty = P.thermal ? Tile64::TY : Tile64F::TY;
+    return (int64_t)((P.NX + tx - 1) / tx) * ((P.NY + ty - 1) / ty);
+}
+
+// ... where a launch's iterations (z_range) take less time than two single
+// steps: 11.6 us each with the temperature (9.5 without), 9.1 (6.5) while the
+// caches hold the state, against the nodes at 119 ps a step (57), 92 (49) in
+// cache.  The rule leaves Rayleigh-Benard 64^3 (24 us per step against 27) and
+// channels of 64^3 (13 against 19) and 78^3 (23 against 28) single, and takes
+// channel 96^3 (46 against 39).
+bool two_step_ok64(const KParams &P)
+{
+    if (P.NZ == 1 || !P.fluid || P.first || P.hit || P.les || P.twoway || P.nozero || !planes_ok(P, 8)) return false;
+    const bool cached = state_bytes(P, 8) <= CACHED_BYTES;
+    const double t_iter = P.thermal ? (cached ? 9.1 : 11.6) : (cached ? 6.5 : 9.5);           // us
+    const double t_node = P.thermal ? (cached ? 92e-6 : 119e-6) : (cached ? 49e-6 : 57e-6);  // us
+    const int64_t columns = z_columns64(P);
+    return (double)z_iterations(columns, P.NZ, z_range(columns, P.NZ)) * t_iter < 2.0 * (double)P.N * t_node;
+}
+
+template <class TZ>
+static void launch_z2_64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,
+                         const double *tl_in, double *tl_out, hipStream_t s)
+{
+    const int zc = z_range(z_columns64(P), P.NZ);
+    const dim3 grid((unsigned)((P.NX + TZ::TX - 1) / TZ::TX), (unsigned)((P.NY + TZ::TY - 1) / TZ::TY),
+                    (unsigned)((P.NZ + zc - 1) / zc));
+    constexpr bool FL = TZ::F == 1, TH = TZ::H == 1;
+    with_bool(step_order(state_bytes(P, 8), P.NX % 8 == 0, 0).nts, [&](auto nt) {
+        hipLaunchKernelGGL((k_step2z_fp64<FL, TH, decltype(nt)::value, TZ>), grid, dim3(TZ::THREADS), 0, s, P, fin,
+                           gin, fout, gout, tl_in, tl_out, zc);
+    });
+}
+
+void launch_two_steps_fp64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,
+                           const double *tl_in, double *tl_out, hipStream_t s)
+{
+    if (P.thermal)
+        launch_z2_64<Tile64>(P, fin, gin, fout, gout, tl_in, tl_out, s);
+    else
+        launch_z2_64<Tile64F>(P, fin, gin, fout, gout, tl_in, tl_out, s);
 }
 
 void launch_velocity_fp64(const KParams &P, const double *fin, const double *tlag, hipStream_t s)

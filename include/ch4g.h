@@ -195,13 +195,12 @@ int ch4g_set_graphs(ch4g_lattice *lat, int enable);
  * reference counterpart (launch mechanics of this library).                 */
 int ch4g_set_fusion(ch4g_lattice *lat, int enable);
 
-/* Steps one steady-state launch advances: 2 for float-storage lattices
- * without HIT forcing, LES, NOZEROMODE or two-way particles that are 2-D
- * (k_step2_fp32: two steps through an LDS tile) or 3-D and large enough
- * (k_step2z_fp32: x-y tiles marching along z through an LDS ring of planes;
- * from about 96^3 with temperature, 113^3 without where rows fill their
- * 64-wide tiles), else 1.  Odd remainders
- * run as single steps; results are identical either way.  No reference
+/* Steps one steady-state launch advances: 2 for lattices without HIT forcing,
+ * LES, NOZEROMODE or particles that are 2-D with float storage (k_step2_fp32:
+ * two steps through an LDS tile) or 3-D and large enough (k_step2z_fp32,
+ * k_step2z_fp64: x-y tiles marching along z through an LDS ring of planes;
+ * from about 96^3 where rows fill their tiles), else 1.  Odd remainders run
+ * as single steps; results are identical either way.  No reference
  * counterpart (launch mechanics of this library).                          */
 int ch4g_steps_per_launch(const ch4g_lattice *lat, int *steps);
 

@@ -70,6 +70,39 @@ def test_small_3d_two_step_launches(shape, channel):
     one.close()
 
 
+# FP64 3-D two-step launches: whole tiles with non-temporal stores; partial
+# tiles in x and y and a shorter last z range; a channel in cache (61: one
+# narrow tile) and one streamed with rows that are no whole lines.  Random
+# populations, so that every direction differs; equal, bit for bit, to the same
+# lattice advanced one step per launch.
+@pytest.mark.parametrize("shape,channel", [((96, 80, 112), False), ((93, 79, 110), False), ((125, 113, 101), False),
+                                           ((61, 61, 240), True), ((113, 113, 113), True)], ids=str)
+def test_fp64_3d_two_step_launches(shape, channel):
+    from ch4g import workloads
+    if channel:
+        cfg = workloads.channel3d(*shape, precision=abi.FP64)
+    else:
+        cfg = configs.rb2d(*shape, Ra=1e6, precision=abi.FP64, seed=5)
+    two, one = Lattice(cfg), Lattice(cfg)
+    one.set_fusion(False)
+    assert (two.steps_per_launch(), one.steps_per_launch()) == (2, 1)
+    two.initial_conditions()
+    p, g = two.get_populations()
+    rng = np.random.default_rng(3)
+    p = p * (1.0 + 1e-2 * rng.uniform(-1, 1, p.shape))
+    if not channel:
+        g = g * (1.0 + 1e-2 * rng.uniform(-1, 1, g.shape))
+    for lat in (two, one):
+        lat.set_populations(p, None if channel else g)
+        lat.step(1)
+        lat.step(7)
+        lat.step(34)
+    for a, b in zip(two.get_populations(), one.get_populations()):
+        assert np.array_equal(a, b)
+    two.close()
+    one.close()
+
+
 # The averages' and rulers' marches: fewer rows, columns or planes than one
 # wave covers, a last wave, row group, z chunk and unit that are partial
 # (1 x 300 x 2048: 16 rows per wave of the plane sums, two of the column sums,
