@@ -137,9 +137,9 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         if (steps[i] < 1) return fail(-1, "steps per chunk must be >= 1");
         B.chunk = std::max(B.chunk, steps[i]);
         ch4g_lattice *L = lats[i];
-        // two steps per launch: 2-D lattices in the batched two-step kernel,
-        // large 3-D lattices on their own branch
-        B.two[i] = two_step_ready(L);
+        // two steps per launch: 2-D float lattices in the batched two-step
+        // kernel, large 3-D lattices on their own branch
+        B.two[i] = (L->dev32 || L->cfg.NZ > 1) && two_step_ready(L);
         solo[i] = B.two[i] && L->cfg.NZ > 1;
         if (solo[i]) B.solo.push_back((int)i);
         // two-step lattices: the population buffer flips with every launch,

@@ -645,6 +645,112 @@ __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp64(KParams P, const do
     }
 }
 
+// Two steps per launch for 2-D lattices (k_step2_fp32 with this file's
+// arithmetic): the first step of a TX x TY tile and its one-node halo goes
+// into LDS, one node per thread, the second from there into the global state.
+//
+// Small lattices pay one launch's ramp and drain, large ones one read (1.6
+// times, with the halo) and write of the state, for two steps.  32 x 4 tiles:
+// two blocks of 64 KB of LDS on a CU, so one's loads overlap the other's
+// collisions.  us per step, single -> this: Rayleigh-Benard 64x32 3.92 -> 3.56,
+// 256x128 6.1 -> 4.2, 512x256 12.5 -> 10.6, 969x487 58.7 -> 39.2, 1024x512 67
+// -> 45, 2048x1024 248 -> 152; channel 512x256 7.7 -> 6.4, 1024x512 24.5 ->
+// 17.2.  Other tiles at 512x256 and 2048x1024: 16 x 8 10.6 and 161, 32 x 5
+// 10.9 and 151, 32 x 8 (one block a CU) 11.7 and 185, 64 x 4 11.7 and 184.
+template <bool FLUID, bool THERMAL, int TX_, int TY_>
+struct Tile2D {
+    static constexpr int TX = TX_, TY = TY_, W = TX + 2, M = W * (TY + 2);
+    static constexpr int THREADS = (M + 63) / 64 * 64;
+    static constexpr int F = FLUID ? 1 : 0, H = THERMAL ? 1 : 0;
+    static constexpr int GOFS = F * Q, LAG = GOFS + Q, PLANES = F * Q + H * (Q + 1);
+};
+
+// A node's results into LDS planes
+template <int OFS, int M>
+struct TileOut64 {
+    double *t;
+    int m;
+    template <int q>
+    __device__ void put(double v) const
+    {
+        t[(OFS + q) * M + m] = v;
+    }
+};
+
+template <bool FLUID, bool THERMAL, bool NT, class T2>
+__global__ void __launch_bounds__(T2::THREADS) k_step2_fp64(KParams P, const double *__restrict__ fin,
+                                                            const double *__restrict__ gin, double *__restrict__ fout,
+                                                            double *__restrict__ gout,
+                                                            const double *__restrict__ tl_in,
+                                                            double *__restrict__ tl_out, int run)
+{
+    constexpr int M = T2::M, W = T2::W, TX = T2::TX, TY = T2::TY, G = T2::GOFS;
+    __shared__ double t[T2::PLANES * M];
+    const int NX = P.NX, NY = P.NY;
+    const uint32_t lb = xcd_run(run, block_linear(), gridDim.x * gridDim.y), row = lb / gridDim.x;
+    const int x0 = (int)(lb - row * gridDim.x) * TX, y0 = (int)row * TY;
+    const int w = NX - x0 < TX ? NX - x0 : TX;
+    // first step (columns beyond the halo of a narrower last tile are never
+    // read: skipped)
+    if (const int m = threadIdx.x; m < M && m % W <= w + 1) {
+        int x = x0 - 1 + m % W;  // in [-1, NX]
+        x = x < 0 ? x + NX : (x >= NX ? x - NX : x);
+        int y = (y0 - 1 + m / W) % NY;
+        y = y < 0 ? y + NY : y;
+        const uint32_t n = (uint32_t)y * NX + x;
+        const Nbr b = make_nbr(x, y, 0, NX, NY, 1);
+        const Pull<double, PULL_LINEAR> o(b, NX, NY);
+        double f[Q], g[Q], Tlag = 0.0, T = 0.0;
+        if constexpr (THERMAL) {
+            Tlag = tl_in[n];
+            pull_thermal64(P, b, make_planes(gin, P.S), o, Tlag, g);
+        }
+        if constexpr (FLUID) pull_fluid64(P, b, make_planes(fin, P.S), o, f);
+        if constexpr (THERMAL) {
+            T = m_sum(g);
+            t[T2::LAG * M + m] = T;
+        }
+        collide64<FLUID, THERMAL, false>(P, b, f, g, Tlag, T, nullptr, n, TileOut64<0, M>{t, m}, TileOut64<G, M>{t, m});
+    }
+    __syncthreads();
+    // second step
+    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+    const int x = x0 + tx, y = y0 + ty;
+    if (ty >= TY || y >= NY || tx >= w) return;
+    const int at = (ty + 1) * W + tx + 1;
+    const uint32_t n = (uint32_t)y * NX + x;
+    const Nbr b = make_nbr(x, y, 0, NX, NY, 1);
+    const Pull<double, PULL_LINEAR> o(b, NX, NY);
+    double f[Q], g[Q], Tlag = 0.0, T = 0.0;
+    if constexpr (THERMAL) {
+        Tlag = t[T2::LAG * M + at];
+        const double fac_top = 2.0 * (P.Tw_top - Tlag);
+        const double fac_bot = 2.0 * (P.Tw_bot - Tlag);
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            const bool cross = P.wall_t && crosses_wall<q>(b);
+            const double v = t[(G + q) * M + (cross ? at : at - cxq(q) - cyq(q) * W)];
+            if constexpr (cyq(q) > 0)
+                g[q] = cross ? v + wq(q) * fac_bot : v;
+            else if constexpr (cyq(q) < 0)
+                g[q] = cross ? v + wq(q) * fac_top : v;
+            else
+                g[q] = v;
+        });
+        T = m_sum(g);
+        tl_out[n] = T;
+    }
+    if constexpr (FLUID)
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            const bool cross = P.wall_f && crosses_wall<q>(b);
+            f[q] = cross ? t[invq(q) * M + at] : t[q * M + at - cxq(q) - cyq(q) * W];
+        });
+    collide64<FLUID, THERMAL, false>(P, b, f, g, Tlag, T, nullptr, n,
+                                     PlaneOut<NT, PULL_LINEAR>{make_planes(FLUID ? fout : gout, P.S), o},
+                                     PlaneOut<NT, PULL_LINEAR>{make_planes(THERMAL ? gout : fout, P.S), o});
+}
+
 // Velocity of the step at every node (the u[] that add_collision reads,
 // fluid.c:1056-1080), for the finite-difference LES closure.
 template <bool FIRST>
@@ -819,8 +925,9 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
         sets(std::false_type{}, std::true_type{});
 }
 
-// Two steps per launch (k_step2z_fp64): 3-D lattices with the fluid whose
-// planes buffer resources reach, without the general force paths.
+// Two steps per launch (k_step2_fp64, k_step2z_fp64): lattices with the fluid
+// whose planes buffer resources reach, without the general force paths.  2-D:
+// always (faster at every size measured, see k_step2_fp64).
 // Tiles: 32 x 8 with the temperature (141 KB of LDS), 64 x 8 without (135 KB).
 using Tile64 = TileZ<true, true, 32, 8, true>;
 using Tile64F = TileZ<true, false, 64, 8, true>;
@@ -831,7 +938,7 @@ static int64_t z_columns64(const KParams &P)
     return (int64_t)((P.NX + tx - 1) / tx) * ((P.NY + ty - 1) / ty);
 }
 
-// ... where a launch's iterations (z_range) take less time than two single
+// 3-D: where a launch's iterations (z_range) take less time than two single
 // steps: 11.6 us each with the temperature (9.5 without), 9.1 (6.5) while the
 // caches hold the state, against the nodes at 119 ps a step (57), 92 (49) in
 // cache.  The rule leaves Rayleigh-Benard 64^3 (24 us per step against 27) and
@@ -839,7 +946,8 @@ static int64_t z_columns64(const KParams &P)
 // channel 96^3 (46 against 39).
 bool two_step_ok64(const KParams &P)
 {
-    if (P.NZ == 1 || !P.fluid || P.first || P.hit || P.les || P.twoway || P.nozero || !planes_ok(P, 8)) return false;
+    if (!P.fluid || P.first || P.hit || P.les || P.twoway || P.nozero || !planes_ok(P, 8)) return false;
+    if (P.NZ == 1) return true;
     const bool cached = state_bytes(P, 8) <= CACHED_BYTES;
     const double t_iter = P.thermal ? (cached ? 9.1 : 11.6) : (cached ? 6.5 : 9.5);           // us
     const double t_node = P.thermal ? (cached ? 92e-6 : 119e-6) : (cached ? 49e-6 : 57e-6);  // us
@@ -861,9 +969,29 @@ static void launch_z2_64(const KParams &P, const double *fin, const double *gin,
     });
 }
 
+template <class T2>
+static void launch_2d_64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,
+                         const double *tl_in, double *tl_out, hipStream_t s)
+{
+    const dim3 grid((unsigned)((P.NX + T2::TX - 1) / T2::TX), (unsigned)((P.NY + T2::TY - 1) / T2::TY));
+    const StepOrder o = step_order(state_bytes(P, 8), P.NX % 16 == 0, RANGE_BYTES_2D);
+    constexpr bool FL = T2::F == 1, TH = T2::H == 1;
+    with_bool(o.nts, [&](auto nt) {
+        hipLaunchKernelGGL((k_step2_fp64<FL, TH, decltype(nt)::value, T2>), grid, dim3(T2::THREADS), 0, s, P, fin, gin,
+                           fout, gout, tl_in, tl_out, o.run);
+    });
+}
+
 void launch_two_steps_fp64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,
                            const double *tl_in, double *tl_out, hipStream_t s)
 {
+    if (P.NZ == 1) {
+        if (P.thermal)
+            launch_2d_64<Tile2D<true, true, 32, 4>>(P, fin, gin, fout, gout, tl_in, tl_out, s);
+        else
+            launch_2d_64<Tile2D<true, false, 32, 4>>(P, fin, gin, fout, gout, tl_in, tl_out, s);
+        return;
+    }
     if (P.thermal)
         launch_z2_64<Tile64>(P, fin, gin, fout, gout, tl_in, tl_out, s);
     else

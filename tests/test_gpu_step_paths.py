@@ -70,14 +70,18 @@ def test_small_3d_two_step_launches(shape, channel):
     one.close()
 
 
-# FP64 3-D two-step launches: whole tiles with non-temporal stores; partial
+# FP64 two-step launches.  2-D: one tile that is narrower and one that is
+# shorter than 32 x 4, exact tiles, partial tiles in x and y, a streamed lattice
+# with non-temporal stores, a channel.  3-D: whole tiles with non-temporal stores; partial
 # tiles in x and y and a shorter last z range; a channel in cache (61: one
 # narrow tile) and one streamed with rows that are no whole lines.  Random
 # populations, so that every direction differs; equal, bit for bit, to the same
 # lattice advanced one step per launch.
-@pytest.mark.parametrize("shape,channel", [((96, 80, 112), False), ((93, 79, 110), False), ((125, 113, 101), False),
+@pytest.mark.parametrize("shape,channel", [((20, 3, 1), False), ((64, 32, 1), False), ((45, 27, 1), False),
+                                           ((1040, 630, 1), False), ((130, 61, 1), True),
+                                           ((96, 80, 112), False), ((93, 79, 110), False), ((125, 113, 101), False),
                                            ((61, 61, 240), True), ((113, 113, 113), True)], ids=str)
-def test_fp64_3d_two_step_launches(shape, channel):
+def test_fp64_two_step_launches(shape, channel):
     from ch4g import workloads
     if channel:
         cfg = workloads.channel3d(*shape, precision=abi.FP64)
