@@ -415,8 +415,8 @@ struct BatchEntry {
 // One lattice taking part in a batched launch: entry index (low 29 bits;
 // bit 31: parity of the lattice's population buffer at this launch; for
 // two-step launches bit 30: a single step, bit 29: parity of its lag array)
-// and its first tile in the launch (wave tiles, or 64 x 4 block tiles for
-// two-step launches).  A launch's slots are sorted by tile0; the last one is
+// and its first tile in the launch (wave tiles, or block tiles for two-step
+// launches).  A launch's slots are sorted by tile0; the last one is
 // a sentinel whose tile0 is the launch's tile count.
 struct BatchSlot {
     uint32_t entry;
@@ -441,6 +441,10 @@ void launch_batch_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots
 // = 64 x 4 tiles of the launch
 void launch_batch2_fp32(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
                         int arith64, StepOrder order, hipStream_t s);
+// the same for FP64 (two_step_ok64), in its tiles
+int64_t batch2_tiles64(int NX, int NY);
+void launch_batch2_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
+                        StepOrder order, hipStream_t s);
 
 // Kernel launchers (stream-ordered).
 void launch_step_fp64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,
@@ -456,9 +460,8 @@ void launch_gather_fp32(const KParams &P, const float *fin, const float *gin, co
 void launch_fields_f32(const KParams &P, const float *fin, const float *gin, const float *tlag, float4 *uT,
                        hipStream_t s);
 
-// Two steps in one launch for 2-D FP32-storage lattices (NZ = 1, NX a
-// multiple of 64, steady steps without HIT tables, LES or particles): reads
-// the state (f, g in; temperature lag tl_in), writes the state two steps on
+// Two steps in one launch (steady steps without HIT tables, LES, NOZEROMODE
+// or particles): reads the state (f, g in; temperature lag tl_in), writes the state two steps on
 // (f, g out; lag tl_out, a different array).
 bool two_step_ok(const KParams &P);    // float storage
 bool two_step_ok64(const KParams &P);  // FP64

@@ -25,7 +25,7 @@ namespace {
 // storage kind; lattice i takes steps[i] of them, spread evenly over the
 // chunk, so every launch carries a similar share of the work.  Each launch
 // has its own short slot list (lattice, parity of its step, first block).
-// 2-D float-storage lattices (two_step_eligible) form groups of their own
+// 2-D lattices (two_step_eligible) form groups of their own
 // whose launches advance two steps each: steps[i] takes steps[i] / 2 such
 // launches and, for an odd share, one single step at the end.
 struct Batch {
@@ -35,12 +35,12 @@ struct Batch {
         bool gen;                         // LES lattices (the kernel instance with those paths)
         bool buf;                         // planes within the reach of buffer resources (FP64)
         StepOrder order;                  // block order and stores, by the group's state bytes
-        bool two;                         // two steps per launch (k_step2_batch32)
+        bool two;                         // two steps per launch (k_step2_batch32, k_step2_batch64)
         int first, count;                 // range in the entry table
         int nlaunch;                      // launches of the group per chunk
         std::vector<int64_t> off;         // per launch: first slot in the slot table
         std::vector<int> nslot;           // per launch: slots (without the sentinel)
-        std::vector<int64_t> nblk;        // per launch: wave tiles (64 x 4 tiles for two-step groups)
+        std::vector<int64_t> nblk;        // per launch: wave tiles (block tiles for two-step groups)
     };
     std::vector<BatchEntry> host;
     std::vector<BatchSlot> slots;
@@ -61,7 +61,7 @@ struct Batch {
     std::vector<char> two;    // lattice i goes two steps per launch
     std::vector<char> flips;  // a chunk changes lattice i's buffer or lag parity
     // 3-D lattices large enough for two steps per launch alone run their own
-    // launches (k_step2z_fp32) as a branch of the chunk on a stream of their
+    // launches (k_step2z_fp32, k_step2z_fp64) as a branch of the chunk on a stream of their
     // own instead of joining a batched group
     std::vector<int> solo;    // lattice indices
     std::vector<hipStream_t> sstream;
@@ -137,9 +137,9 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         if (steps[i] < 1) return fail(-1, "steps per chunk must be >= 1");
         B.chunk = std::max(B.chunk, steps[i]);
         ch4g_lattice *L = lats[i];
-        // two steps per launch: 2-D float lattices in the batched two-step
-        // kernel, large 3-D lattices on their own branch
-        B.two[i] = (L->dev32 || L->cfg.NZ > 1) && two_step_ready(L);
+        // two steps per launch: 2-D lattices in the batched two-step kernels,
+        // large 3-D lattices on their own branch
+        B.two[i] = two_step_ready(L);
         solo[i] = B.two[i] && L->cfg.NZ > 1;
         if (solo[i]) B.solo.push_back((int)i);
         // two-step lattices: the population buffer flips with every launch,
@@ -207,7 +207,9 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
             for (int s_ = 0; s_ < nl; s_++) a[(size_t)(((int64_t)s_ * KG) / nl)] = s_;
             at.push_back(a);
             npair.push_back(G.two ? st / 2 : 0);
-            ntile.push_back(G.two ? batch2_tiles(L->cfg.NX, L->cfg.NY) : batch_tiles(L->base, G.dense));
+            ntile.push_back(!G.two     ? batch_tiles(L->base, G.dense)
+                            : L->dev32 ? batch2_tiles(L->cfg.NX, L->cfg.NY)
+                                       : batch2_tiles64(L->cfg.NX, L->cfg.NY));
             bytes += 2 * (int64_t)Q * L->N * (L->dev32 ? 4 : 8) * ((L->base.fluid ? 1 : 0) + (L->base.thermal ? 1 : 0));
             G.buf = G.buf && planes_ok(L->base, 8);
             whole_lines = whole_lines && (G.dense || L->cfg.NX * (L->dev32 ? 4 : 8) % 128 == 0);
@@ -327,7 +329,9 @@ int launch_steps(Batch &B)
             const BatchEntry *tab = B.dev + G.first;
             const BatchSlot *sl = B.dev_slots + G.off[(size_t)k];
             const int ns = G.nslot[(size_t)k];
-            if (G.two)
+            if (G.two && !G.dev32)
+                launch_batch2_fp64(tab, sl, ns, nt, G.kind, G.order, st);
+            else if (G.two)
                 launch_batch2_fp32(tab, sl, ns, nt, G.kind, G.arith64, G.order, st);
             else if (G.dev32)
                 launch_batch_fp32(tab, sl, ns, nb, G.kind, G.dense, G.gen, G.arith64, G.order, st);

@@ -657,6 +657,7 @@ __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp64(KParams P, const do
 // -> 45, 2048x1024 248 -> 152; channel 512x256 7.7 -> 6.4, 1024x512 24.5 ->
 // 17.2.  Other tiles at 512x256 and 2048x1024: 16 x 8 10.6 and 161, 32 x 5
 // 10.9 and 151, 32 x 8 (one block a CU) 11.7 and 185, 64 x 4 11.7 and 184.
+constexpr int T2D_TX = 32, T2D_TY = 4;
 template <bool FLUID, bool THERMAL, int TX_, int TY_>
 struct Tile2D {
     static constexpr int TX = TX_, TY = TY_, W = TX + 2, M = W * (TY + 2);
@@ -677,18 +678,16 @@ struct TileOut64 {
     }
 };
 
+// The two steps of the tile whose first node is (x0, y0), through the block's
+// LDS array t.
 template <bool FLUID, bool THERMAL, bool NT, class T2>
-__global__ void __launch_bounds__(T2::THREADS) k_step2_fp64(KParams P, const double *__restrict__ fin,
-                                                            const double *__restrict__ gin, double *__restrict__ fout,
-                                                            double *__restrict__ gout,
-                                                            const double *__restrict__ tl_in,
-                                                            double *__restrict__ tl_out, int run)
+__device__ __forceinline__ void step2_tile64(const KParams &P, const double *__restrict__ fin,
+                                             const double *__restrict__ gin, double *__restrict__ fout,
+                                             double *__restrict__ gout, const double *__restrict__ tl_in,
+                                             double *__restrict__ tl_out, int x0, int y0, double *t)
 {
     constexpr int M = T2::M, W = T2::W, TX = T2::TX, TY = T2::TY, G = T2::GOFS;
-    __shared__ double t[T2::PLANES * M];
     const int NX = P.NX, NY = P.NY;
-    const uint32_t lb = xcd_run(run, block_linear(), gridDim.x * gridDim.y), row = lb / gridDim.x;
-    const int x0 = (int)(lb - row * gridDim.x) * TX, y0 = (int)row * TY;
     const int w = NX - x0 < TX ? NX - x0 : TX;
     // first step (columns beyond the halo of a narrower last tile are never
     // read: skipped)
@@ -749,6 +748,58 @@ __global__ void __launch_bounds__(T2::THREADS) k_step2_fp64(KParams P, const dou
     collide64<FLUID, THERMAL, false>(P, b, f, g, Tlag, T, nullptr, n,
                                      PlaneOut<NT, PULL_LINEAR>{make_planes(FLUID ? fout : gout, P.S), o},
                                      PlaneOut<NT, PULL_LINEAR>{make_planes(THERMAL ? gout : fout, P.S), o});
+}
+
+template <bool FLUID, bool THERMAL, bool NT, class T2>
+__global__ void __launch_bounds__(T2::THREADS) k_step2_fp64(KParams P, const double *__restrict__ fin,
+                                                            const double *__restrict__ gin, double *__restrict__ fout,
+                                                            double *__restrict__ gout,
+                                                            const double *__restrict__ tl_in,
+                                                            double *__restrict__ tl_out, int run)
+{
+    __shared__ double t[T2::PLANES * T2::M];
+    const uint32_t lb = xcd_run(run, block_linear(), gridDim.x * gridDim.y), row = lb / gridDim.x;
+    step2_tile64<FLUID, THERMAL, NT, T2>(P, fin, gin, fout, gout, tl_in, tl_out,
+                                         (int)(lb - row * gridDim.x) * T2::TX, (int)row * T2::TY, t);
+}
+
+// Many 2-D lattices in one launch, two steps each or, where the slot says so,
+// one (see k_step2_batch32).
+template <bool FLUID, bool THERMAL, bool NT, class T2>
+__global__ void __launch_bounds__(T2::THREADS) k_step2_batch64(const BatchEntry *__restrict__ tab,
+                                                               const BatchSlot *__restrict__ slots, int nslots,
+                                                               int run)
+{
+    __shared__ double t[T2::PLANES * T2::M];
+    const uint32_t bt = xcd_run(run, blockIdx.x, gridDim.x);
+    if (bt >= slots[nslots].tile0) return;
+    int lo = 0, hi = nslots - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (slots[mid].tile0 <= bt)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    const BatchSlot sl = slots[lo];
+    const BatchEntry &E = tab[sl.entry & BATCH_ENTRY_MASK];
+    const KParams &P = E.P;
+    const int in = E.cur ^ (int)(sl.entry >> 31);
+    const bool tp = (sl.entry & BATCH_LAG_PARITY) != 0;
+    const double *fin = (const double *)E.f[in], *gin = (const double *)E.g[in];
+    double *fout = (double *)E.f[in ^ 1], *gout = (double *)E.g[in ^ 1];
+    double *tl_a = (double *)(tp ? E.tlag2 : E.tlag), *tl_b = (double *)(tp ? E.tlag : E.tlag2);
+    const uint32_t tile = bt - sl.tile0, txs = ((uint32_t)P.NX + T2::TX - 1) / T2::TX;
+    const int x0 = (int)(tile % txs) * T2::TX, y0 = (int)(tile / txs) * T2::TY;
+    if (sl.entry & BATCH_SINGLE) {
+        const int x = x0 + (int)threadIdx.x % T2::TX, y = y0 + (int)threadIdx.x / T2::TX;
+        if ((int)threadIdx.x >= T2::TX * T2::TY || x >= P.NX || y >= P.NY) return;
+        step_node64<false, FLUID, THERMAL, NT, false, true, PULL_LINEAR>(P, fin, gin, fout, gout, tl_a,
+                                                                         (double *)E.taules, x, y, 0,
+                                                                         (uint32_t)y * (uint32_t)P.NX + (uint32_t)x);
+        return;
+    }
+    step2_tile64<FLUID, THERMAL, NT, T2>(P, fin, gin, fout, gout, tl_a, tl_b, x0, y0, t);
 }
 
 // Velocity of the step at every node (the u[] that add_collision reads,
@@ -987,9 +1038,9 @@ void launch_two_steps_fp64(const KParams &P, const double *fin, const double *gi
 {
     if (P.NZ == 1) {
         if (P.thermal)
-            launch_2d_64<Tile2D<true, true, 32, 4>>(P, fin, gin, fout, gout, tl_in, tl_out, s);
+            launch_2d_64<Tile2D<true, true, T2D_TX, T2D_TY>>(P, fin, gin, fout, gout, tl_in, tl_out, s);
         else
-            launch_2d_64<Tile2D<true, false, 32, 4>>(P, fin, gin, fout, gout, tl_in, tl_out, s);
+            launch_2d_64<Tile2D<true, false, T2D_TX, T2D_TY>>(P, fin, gin, fout, gout, tl_in, tl_out, s);
         return;
     }
     if (P.thermal)
@@ -1038,6 +1089,28 @@ void launch_batch_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots
         sets(std::true_type{}, std::false_type{});
     else
         sets(std::false_type{}, std::true_type{});
+}
+
+int64_t batch2_tiles64(int NX, int NY)
+{
+    return (int64_t)((NX + T2D_TX - 1) / T2D_TX) * ((NY + T2D_TY - 1) / T2D_TY);
+}
+
+void launch_batch2_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots, int64_t nblocks, int kind,
+                        StepOrder o, hipStream_t s)
+{
+    auto go = [&](auto th) {
+        constexpr bool TH = decltype(th)::value;
+        using T2 = Tile2D<true, TH, T2D_TX, T2D_TY>;
+        with_bool(o.nts, [&](auto nt) {
+            hipLaunchKernelGGL((k_step2_batch64<true, TH, decltype(nt)::value, T2>), dim3((unsigned)nblocks),
+                               dim3(T2::THREADS), 0, s, tab, slots, nslots, o.run);
+        });
+    };
+    if (kind == BATCH_FLUID_THERMAL)
+        go(std::true_type{});
+    else
+        go(std::false_type{});
 }
 
 // LB_FLUID_FORCING_NOZEROMODE (forcing.c:1123-1152): sums over all nodes of

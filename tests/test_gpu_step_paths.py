@@ -107,6 +107,29 @@ def test_fp64_two_step_launches(shape, channel):
     one.close()
 
 
+# FP64 2-D lattices in one batch, two steps per launch and a single one for odd
+# counts: narrower than a tile, exact tiles, partial tiles, a channel, and a
+# float lattice beside them.  Equal, bit for bit, to each alone in single steps.
+def test_fp64_batched_two_steps():
+    from ch4g import step_batch, workloads
+    cfgs = [configs.rb2d(20, 3, 1, Ra=1e4, seed=3), configs.rb2d(64, 32, 1, Ra=1e5, seed=4),
+            configs.rb2d(45, 27, 1, Ra=1e5, seed=5), workloads.channel3d(130, 61, 1, precision=abi.FP64),
+            configs.rb2d(96, 48, 1, Ra=1e5, precision=abi.FP32_DEV, seed=6)]
+    many, one = [Lattice(c) for c in cfgs], [Lattice(c) for c in cfgs]
+    for lat in many + one:
+        run(lat, 1)
+    for lat in one:
+        lat.set_fusion(False)
+    for n in (1, 7, 10, 2):
+        step_batch(many, n)
+        for a, b in zip(many, one):
+            b.step(n)
+            for x, y in zip(a.get_populations(), b.get_populations()):
+                assert np.array_equal(x, y), (n, a.cfg.NX)
+    for lat in many + one:
+        lat.close()
+
+
 # The averages' and rulers' marches: fewer rows, columns or planes than one
 # wave covers, a last wave, row group, z chunk and unit that are partial
 # (1 x 300 x 2048: 16 rows per wave of the plane sums, two of the column sums,
