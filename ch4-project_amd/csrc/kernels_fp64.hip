@@ -802,6 +802,91 @@ __global__ void __launch_bounds__(T2::THREADS) k_step2_batch64(const BatchEntry 
     step2_tile64<FLUID, THERMAL, NT, T2>(P, fin, gin, fout, gout, tl_a, tl_b, x0, y0, t);
 }
 
+// Two steps per launch for 3-D lattices of few columns: a block owns R rows of
+// all NX NZ columns (periodic within the block) and computes one row beside
+// them in the first step, as k_step2_fp64 does with tiles.  Bound by the launch
+// and by FP64 issue, so blocks are one wave per SIMD.  us per step, single ->
+// this: channel 4x16x4 3.60 -> 2.90, 4x64x4 4.03 -> 2.95, 8x16x8 4.02 -> 2.99,
+// 4x5000x4 8.3 -> 5.2; Rayleigh-Benard 8x16x4 5.2 -> 3.8, 8x64x8 5.4 -> 4.0.
+// (One block with the whole lattice in LDS for any number of steps took 4.4 at
+// 4x64x4: one CU's FP64 issue.)
+constexpr int SLAB = 256;  // nodes of a block in the first step
+
+// Rows of a block, 0 where this is not taken: at least six of them, or fewer in
+// at most 32 blocks (3x300x21, two rows in 150 blocks: 5.4 against 4.4).
+inline int slab_rows(const KParams &P)
+{
+    const int64_t R = SLAB / ((int64_t)P.NX * P.NZ) - 2;
+    return R >= 6 || (R >= 2 && P.NY <= 32 * R) ? (int)R : 0;
+}
+
+template <bool FLUID, bool THERMAL>
+__global__ void __launch_bounds__(SLAB) k_step2y_fp64(KParams P, const double *__restrict__ fin,
+                                                      const double *__restrict__ gin, double *__restrict__ fout,
+                                                      double *__restrict__ gout, const double *__restrict__ tl_in,
+                                                      double *__restrict__ tl_out, int R)
+{
+    constexpr int G = FLUID ? Q : 0, LAG = G + Q;
+    __shared__ double t[(G + (THERMAL ? Q + 1 : 0)) * SLAB];
+    const int NX = P.NX, NY = P.NY, NZ = P.NZ, A = NX * NZ, m = threadIdx.x, r = m / A, c = m - r * A;
+    const int x = c % NX, z = c / NX, y0 = (int)blockIdx.x * R;
+    const bool act = r < R + 2;
+    int y = (y0 - 1 + r) % NY;
+    y = y < 0 ? y + NY : y;
+    const uint32_t n = ((uint32_t)z * NY + y) * NX + x;
+    const Nbr b = make_nbr(x, y, z, NX, NY, NZ);
+    const Pull<double, PULL_LINEAR> o(b, NX, NY);
+    double f[Q], g[Q], Tlag = 0.0, T = 0.0;
+    if (act) {
+        if constexpr (THERMAL) {
+            Tlag = tl_in[n];
+            pull_thermal64(P, b, make_planes(gin, P.S), o, Tlag, g);
+        }
+        if constexpr (FLUID) pull_fluid64(P, b, make_planes(fin, P.S), o, f);
+        if constexpr (THERMAL) {
+            T = m_sum(g);
+            t[LAG * SLAB + m] = T;
+        }
+        collide64<FLUID, THERMAL, false>(P, b, f, g, Tlag, T, nullptr, n, TileOut64<0, SLAB>{t, m},
+                                         TileOut64<G, SLAB>{t, m});
+    }
+    __syncthreads();
+    if (r < 1 || r > R || y0 - 1 + r >= NY) return;
+    // place in the block of the node at x - c_q
+    auto src = [&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        const int xs = cxq(q) > 0 ? b.xm : (cxq(q) < 0 ? b.xp : x), zs = czq(q) > 0 ? b.zm : (czq(q) < 0 ? b.zp : z);
+        return (r - cyq(q)) * A + zs * NX + xs;
+    };
+    if constexpr (THERMAL) {
+        Tlag = t[LAG * SLAB + m];
+        const double fac_top = 2.0 * (P.Tw_top - Tlag);
+        const double fac_bot = 2.0 * (P.Tw_bot - Tlag);
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            const bool cross = P.wall_t && crosses_wall<q>(b);
+            const double v = t[(G + q) * SLAB + (cross ? m : src(qc))];
+            if constexpr (cyq(q) > 0)
+                g[q] = cross ? v + wq(q) * fac_bot : v;
+            else if constexpr (cyq(q) < 0)
+                g[q] = cross ? v + wq(q) * fac_top : v;
+            else
+                g[q] = v;
+        });
+        T = m_sum(g);
+        tl_out[n] = T;
+    }
+    if constexpr (FLUID)
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            const bool cross = P.wall_f && crosses_wall<q>(b);
+            f[q] = cross ? t[invq(q) * SLAB + m] : t[q * SLAB + src(qc)];
+        });
+    collide64<FLUID, THERMAL, false>(P, b, f, g, Tlag, T, nullptr, n,
+                                     PlaneOut<false, PULL_LINEAR>{make_planes(FLUID ? fout : gout, P.S), o},
+                                     PlaneOut<false, PULL_LINEAR>{make_planes(THERMAL ? gout : fout, P.S), o});
+}
+
 // Velocity of the step at every node (the u[] that add_collision reads,
 // fluid.c:1056-1080), for the finite-difference LES closure.
 template <bool FIRST>
@@ -976,9 +1061,9 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
         sets(std::false_type{}, std::true_type{});
 }
 
-// Two steps per launch (k_step2_fp64, k_step2z_fp64): lattices with the fluid
-// whose planes buffer resources reach, without the general force paths.  2-D:
-// always (faster at every size measured, see k_step2_fp64).
+// Two steps per launch (k_step2_fp64, k_step2y_fp64, k_step2z_fp64): lattices
+// with the fluid whose planes buffer resources reach, without the general force
+// paths.  2-D: always (faster at every size measured, see k_step2_fp64).
 // Tiles: 32 x 8 with the temperature (141 KB of LDS), 64 x 8 without (135 KB).
 using Tile64 = TileZ<true, true, 32, 8, true>;
 using Tile64F = TileZ<true, false, 64, 8, true>;
@@ -998,7 +1083,7 @@ static int64_t z_columns64(const KParams &P)
 bool two_step_ok64(const KParams &P)
 {
     if (!P.fluid || P.first || P.hit || P.les || P.twoway || P.nozero || !planes_ok(P, 8)) return false;
-    if (P.NZ == 1) return true;
+    if (P.NZ == 1 || slab_rows(P) > 0) return true;
     const bool cached = state_bytes(P, 8) <= CACHED_BYTES;
     const double t_iter = P.thermal ? (cached ? 9.1 : 11.6) : (cached ? 6.5 : 9.5);           // us
     const double t_node = P.thermal ? (cached ? 92e-6 : 119e-6) : (cached ? 49e-6 : 57e-6);  // us
@@ -1041,6 +1126,16 @@ void launch_two_steps_fp64(const KParams &P, const double *fin, const double *gi
             launch_2d_64<Tile2D<true, true, T2D_TX, T2D_TY>>(P, fin, gin, fout, gout, tl_in, tl_out, s);
         else
             launch_2d_64<Tile2D<true, false, T2D_TX, T2D_TY>>(P, fin, gin, fout, gout, tl_in, tl_out, s);
+        return;
+    }
+    if (const int R = slab_rows(P); R > 0) {
+        const dim3 grid((unsigned)((P.NY + R - 1) / R));
+        if (P.thermal)
+            hipLaunchKernelGGL((k_step2y_fp64<true, true>), grid, dim3(SLAB), 0, s, P, fin, gin, fout, gout, tl_in,
+                               tl_out, R);
+        else
+            hipLaunchKernelGGL((k_step2y_fp64<true, false>), grid, dim3(SLAB), 0, s, P, fin, gin, fout, gout, tl_in,
+                               tl_out, R);
         return;
     }
     if (P.thermal)

@@ -72,13 +72,16 @@ def test_small_3d_two_step_launches(shape, channel):
 
 # FP64 two-step launches.  2-D: one tile that is narrower and one that is
 # shorter than 32 x 4, exact tiles, partial tiles in x and y, a streamed lattice
-# with non-temporal stores, a channel.  3-D: whole tiles with non-temporal stores; partial
+# with non-temporal stores, a channel.  3-D of few columns (slabs of rows): one
+# row more than the last slab, fewer rows than a slab, exact slabs, two rows a
+# slab.  3-D: whole tiles with non-temporal stores; partial
 # tiles in x and y and a shorter last z range; a channel in cache (61: one
 # narrow tile) and one streamed with rows that are no whole lines.  Random
 # populations, so that every direction differs; equal, bit for bit, to the same
 # lattice advanced one step per launch.
 @pytest.mark.parametrize("shape,channel", [((20, 3, 1), False), ((64, 32, 1), False), ((45, 27, 1), False),
-                                           ((1040, 630, 1), False), ((130, 61, 1), True),
+                                           ((1040, 630, 1), False), ((130, 61, 1), True), ((4, 15, 4), True),
+                                           ((1, 3, 2), False), ((5, 10, 7), False), ((8, 64, 8), False),
                                            ((96, 80, 112), False), ((93, 79, 110), False), ((125, 113, 101), False),
                                            ((61, 61, 240), True), ((113, 113, 113), True)], ids=str)
 def test_fp64_two_step_launches(shape, channel):
