@@ -253,3 +253,34 @@ def test_hit_tables_ahead(shape, draws):
     assert np.array_equal(a.get_populations()[0], b.get_populations()[0])
     a.close()
     b.close()
+
+
+# The interpolation with gradients, eight lanes a particle: counts around a wave
+# (8) and a block (32), particles on and beside the walls and the periodic faces,
+# fluid and temperature together, fluid alone, and walls of the fluid only (the
+# two fields read apart).  FP64: every field as the oracle's, bit for bit.
+@pytest.mark.parametrize("n", [1, 7, 33])
+@pytest.mark.parametrize("kind", ["both", "fluid", "apart"])
+def test_gradient_interpolation_counts(kind, n):
+    cfg = configs.rb2d(12, 10, 7, Ra=1e4, seed=5, noise=0.05)
+    if kind == "fluid":
+        cfg = configs.poiseuille(12, 10, 7, tau=0.8, g=1e-4)
+    if kind == "apart":
+        cfg.flags &= ~abi.TEMPERATURE_BC_Y
+    flags = abi.LAGRANGE_WRAP | abi.LAGRANGE_GRADIENT | abi.LAGRANGE_ADDEDMASS
+    rng = np.random.default_rng(n)
+    a = np.zeros(n, dtype=abi.particle_dtype())
+    a["name"], a["tau_drag"], a["beta_coeff"] = np.arange(n), 5.0, 0.8
+    for axis, m in (("x", 12.0), ("y", 10.0), ("z", 7.0)):
+        a[axis] = rng.uniform(0.0, m, n)
+    a["y"][:2], a["x"][2:4], a["z"][4:6] = (0.2, 9.9)[:min(n, 2)], (0.1, 11.9)[:max(0, min(n - 2, 2))], \
+        (0.1, 6.9)[:max(0, min(n - 4, 2))]
+    got = []
+    for x in (Oracle(cfg), Lattice(cfg)):
+        x.initial_conditions()
+        x.particles_init(abi.make_particle_config(flags, 1, tau_drag=(1, 5.0, 5.0), beta_coeff=(1, 0.8, 0.8)))
+        x.set_particles(a)
+        x.step(6)
+        got.append(x.particles())
+    for f in abi.PARTICLE_FIELDS:
+        assert np.array_equal(got[0][f], got[1][f], equal_nan=True), f
