@@ -1406,10 +1406,19 @@ __device__ __forceinline__ uint32_t fb_cell(const PartParams &P, int im, int jm,
     return (uint32_t)((((int64_t)km + 1) * (P.NY + 1) + (jm + 1)) * (P.NX + 1) + (im + 1));
 }
 
+// Also takes back the heads of the previous call's cells (head[cell] = -1).
+// This and the setting of the heads (k_fb_deps) were launches of their own: a
+// step of 149 particles in 40x72x45 57.1 us with them, 55.1 without; 9000 in
+// 96^3 163 and 158.
 __global__ void __launch_bounds__(PB) k_fb_cells(PartParams P, uint32_t sent, uint32_t *kin, uint32_t *vin,
-                                                 double *rec, double g0, double g1, double g2)
+                                                 double *rec, double g0, double g1, double g2,
+                                                 const uint32_t *__restrict__ old_keys, int64_t old_n, int *head)
 {
     const int64_t p = (int64_t)blockIdx.x * PB + threadIdx.x;
+    if (p < old_n) {
+        const uint32_t old = old_keys[p];
+        if (old != sent) head[old] = -1;
+    }
     if (p >= P.np) return;
     const uint32_t o = (uint32_t)P.orig[p];
     uint32_t key = sent;
@@ -1449,30 +1458,21 @@ __global__ void __launch_bounds__(PB) k_fb_cells(PartParams P, uint32_t sent, ui
     vin[o] = (uint32_t)p;
 }
 
-// head[cell] = first sorted position of the cell (set), or -1 (clear)
-__global__ void __launch_bounds__(PB) k_fb_heads(const uint32_t *keys, int64_t M, uint32_t sent, int *head, int set)
+// The deposits of every sorted particle, corner-major: dep[c][t][3] =
+// (fac f_p) * w_c with the stencil's weights (lagrange.c:1271-1292), w_c =
+// (X * Y) * Z, X = x - (im + 1/2) on the +x corners and (im + 3/2) - x on the
+// -x corners, likewise Y and Z; ord[t] the particle's reference index.  And
+// head[cell] = the cell's first sorted position.
+__global__ void __launch_bounds__(PB) k_fb_deps(PartParams P, const uint32_t *__restrict__ keys,
+                                                const uint32_t *__restrict__ vals, const double *__restrict__ rec,
+                                                uint32_t sent, int64_t M, double *__restrict__ dep,
+                                                uint32_t *__restrict__ ord, int *__restrict__ head)
 {
     const int64_t t = (int64_t)blockIdx.x * PB + threadIdx.x;
     if (t >= M) return;
     const uint32_t key = keys[t];
     if (key == sent) return;
-    if (!set)
-        head[key] = -1;
-    else if (t == 0 || keys[t - 1] != key)
-        head[key] = (int)t;
-}
-
-// The deposits of every sorted particle, corner-major: dep[c][t][3] =
-// (fac f_p) * w_c with the stencil's weights (lagrange.c:1271-1292), w_c =
-// (X * Y) * Z, X = x - (im + 1/2) on the +x corners and (im + 3/2) - x on the
-// -x corners, likewise Y and Z; ord[t] the particle's reference index.
-__global__ void __launch_bounds__(PB) k_fb_deps(PartParams P, const uint32_t *__restrict__ keys,
-                                                const uint32_t *__restrict__ vals, const double *__restrict__ rec,
-                                                uint32_t sent, int64_t M, double *__restrict__ dep,
-                                                uint32_t *__restrict__ ord)
-{
-    const int64_t t = (int64_t)blockIdx.x * PB + threadIdx.x;
-    if (t >= M || keys[t] == sent) return;
+    if (t == 0 || keys[t - 1] != key) head[key] = (int)t;
     const double *q = rec + 8 * (int64_t)vals[t];
     const double px = q[3], py = q[4], pz = q[5];
     const double im = floor(px - 0.5), jm = floor(py - 0.5), km = floor(pz - 0.5);
@@ -1752,21 +1752,18 @@ size_t feedback_sort_bytes(int64_t nitems, int key_bits)
 int launch_feedback(const PartParams &P, const FeedbackBufs &B, hipStream_t s)
 {
     const uint32_t sent = B.key_bits >= 32 ? 0xFFFFFFFFu : (uint32_t)((1ull << B.key_bits) - 1);
-    if (B.old_n > 0)
-        hipLaunchKernelGGL(k_fb_heads, dim3(blocks_of(B.old_n, PB)), dim3(PB), 0, s, B.old_keys, B.old_n, sent, B.head,
-                           0);
     const int64_t M = P.np;
+    const int64_t most = M > B.old_n ? M : B.old_n;
+    if (most > 0)
+        hipLaunchKernelGGL(k_fb_cells, dim3(blocks_of(most, PB)), dim3(PB), 0, s, P, sent, B.kin, B.vin, B.rec, B.gv[0],
+                           B.gv[1], B.gv[2], B.old_keys, B.old_n, B.head);
     if (M > 0) {
-        hipLaunchKernelGGL(k_fb_cells, dim3(blocks_of(M, PB)), dim3(PB), 0, s, P, sent, B.kin, B.vin, B.rec, B.gv[0],
-                           B.gv[1], B.gv[2]);
         size_t bytes = B.tmp_bytes;
         if (hipcub::DeviceRadixSort::SortPairs(B.tmp, bytes, B.kin, B.kout, B.vin, B.vout, (int)M, 0, B.key_bits,
                                                s) != hipSuccess)
             return -2;
-        hipLaunchKernelGGL(k_fb_heads, dim3(blocks_of(M, PB)), dim3(PB), 0, s, (const uint32_t *)B.kout, M, sent,
-                           B.head, 1);
         hipLaunchKernelGGL(k_fb_deps, dim3(blocks_of(M, PB)), dim3(PB), 0, s, P, (const uint32_t *)B.kout,
-                           (const uint32_t *)B.vout, (const double *)B.rec, sent, M, B.dep, B.ord);
+                           (const uint32_t *)B.vout, (const double *)B.rec, sent, M, B.dep, B.ord, B.head);
     }
     const dim3 grid(blocks_of(P.NX, FBX), blocks_of(P.NY, FBY), P.NZ), block(FBX, FBY);
     if (B.fb_float)
