@@ -465,6 +465,7 @@ void launch_fields_f32(const KParams &P, const float *fin, const float *gin, con
 // (f, g out; lag tl_out, a different array).
 bool two_step_ok(const KParams &P);    // float storage
 bool two_step_ok64(const KParams &P);  // FP64
+bool two_step_slab64(const KParams &P);  // FP64, 3-D of few columns (launches of a few blocks)
 void launch_two_steps_fp32(const KParams &P, const float *fin, const float *gin, float *fout, float *gout,
                            const float *tl_in, float *tl_out, hipStream_t s);
 void launch_two_steps_fp64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,

@@ -60,9 +60,10 @@ struct Batch {
     std::vector<int> steps;   // steps of each lattice per chunk
     std::vector<char> two;    // lattice i goes two steps per launch
     std::vector<char> flips;  // a chunk changes lattice i's buffer or lag parity
-    // 3-D lattices large enough for two steps per launch alone run their own
-    // launches (k_step2z_fp32, k_step2z_fp64) as a branch of the chunk on a stream of their
-    // own instead of joining a batched group
+    // 3-D lattices large enough for two steps per launch alone (the z march:
+    // k_step2z_fp32, k_step2z_fp64), and a single slab lattice, run their own
+    // launches as a branch of the chunk on a stream of their own instead of
+    // joining a batched group
     std::vector<int> solo;    // lattice indices
     std::vector<hipStream_t> sstream;
     std::vector<hipEvent_t> sdone;
@@ -131,6 +132,13 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
     B.flips.assign(lats.size(), 0);
     B.solo.clear();
     std::vector<char> solo(lats.size(), 0);
+    // Two or more slab lattices, whose own launches would be a few blocks each,
+    // share the batched single steps; one takes its two steps per launch as a
+    // branch.  us per step of 1, 2, 8, 32 FP64 channels 4x64x4, a branch each
+    // and together: 3.3 4.9, 6.3 5.5, 15.5 6.7, 52.6 10.6.
+    auto slab_of = [](const ch4g_lattice *L) { return !L->dev32 && two_step_slab64(L->base); };
+    int nslab = 0;
+    for (const ch4g_lattice *L : lats) nslab += L && slab_of(L);
     for (size_t i = 0; i < lats.size(); i++) {
         int rc = check_member(lats[i]);
         if (rc) return rc;
@@ -139,7 +147,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         ch4g_lattice *L = lats[i];
         // two steps per launch: 2-D lattices in the batched two-step kernels,
         // large 3-D lattices on their own branch
-        B.two[i] = two_step_ready(L);
+        B.two[i] = (nslab < 2 || !slab_of(L)) && two_step_ready(L);
         solo[i] = B.two[i] && L->cfg.NZ > 1;
         if (solo[i]) B.solo.push_back((int)i);
         // two-step lattices: the population buffer flips with every launch,

@@ -1091,6 +1091,8 @@ bool two_step_ok64(const KParams &P)
     return (double)z_iterations(columns, P.NZ, z_range(columns, P.NZ)) * t_iter < 2.0 * (double)P.N * t_node;
 }
 
+bool two_step_slab64(const KParams &P) { return P.NZ > 1 && slab_rows(P) > 0; }
+
 template <class TZ>
 static void launch_z2_64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,
                          const double *tl_in, double *tl_out, hipStream_t s)

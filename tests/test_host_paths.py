@@ -1,0 +1,67 @@
+"""The host side of libch4g.so with the HIP runtime replaced by hip_stub.cpp
+(host memory, no kernel runs, launches counted by name): what is launched,
+allocated and given back, and what happens when an allocation fails.  Each case
+is a program of its own, so that the stub stays out of this process."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = f"""
+import ctypes as C, sys
+sys.path[:0] = [{os.path.join(ROOT, 'ch4-project_amd')!r}, {HERE!r}]
+S = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+S.stub_launches.restype = S.stub_streams_made.restype = S.stub_captures.restype = C.c_long
+S.stub_live_bytes.restype = C.c_size_t
+S.stub_fail.argtypes = [C.c_size_t, C.c_long, C.c_long]
+import numpy as np
+from ch4g import abi, footprint_bytes, Lattice, serve, step_batch, workloads
+import configs
+
+def started(cfg, n=1):
+    lat = Lattice(cfg)
+    lat.initial_conditions()
+    lat.step(n)
+    return lat
+
+def launches(part=b"k_"):
+    return S.stub_launches(part)
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = tmp_path_factory.mktemp("stub") / "hip_stub.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "hip_stub.cpp"), "-o", str(so)], check=True)
+    return str(so)
+
+
+@pytest.fixture
+def run(stub):
+    def go(code):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + code, stub], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return go
+
+
+# Ensembles of FP64 3-D lattices of few columns: one batched launch per step for
+# all of them on the batch's stream, whatever their number; one alone keeps its
+# two steps per launch.
+@pytest.mark.parametrize("n", [2, 3, 32])
+def test_few_column_ensembles_share_their_launches(run, n):
+    run(f"""
+lats = [started(workloads.channel3d(*s, tau=1.0, precision=abi.FP64)) for s in
+        [(4, 64, 4), (8, 24, 6), (8, 64, 8)] * 11][:{n}]
+S.stub_reset()
+step_batch(lats, 7)
+assert launches(b"k_step_batch64") == launches() == 7, launches()
+assert S.stub_streams_made() == 1, S.stub_streams_made()
+S.stub_reset()
+step_batch(lats[:1], 7)
+assert launches(b"k_step2y_fp64") == 3 and launches() == 4, launches()
+""")
