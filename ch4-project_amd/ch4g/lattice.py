@@ -108,7 +108,8 @@ def step_batch(lattices, nsteps):
 
 def serve(jobs, mode=0, hbm_budget=0, chunk_steps=0, max_active=0, use_graphs=True, schedule=0):
     """Run a request stream (list of abi.Job, modified in place with the
-    admission/finish times, averages and status); returns the list."""
+    admission/finish times, averages and status); returns the list.
+    use_graphs has no effect."""
     arr = (Job * len(jobs))(*jobs)
     sp = ServeParams()
     sp.hbm_budget, sp.mode, sp.chunk_steps, sp.max_active = int(hbm_budget), int(mode), int(chunk_steps), int(max_active)

@@ -1,7 +1,7 @@
 // Serving of many lattices on one GPU (include/ch4g.h ch4g_step_batch,
 // ch4g_serve): batched steps over a tile -> lattice table, and the
 // continuous-batching request loop (admission by device footprint, chunks of
-// steps replayed from captured graphs, retirement with the final averages).
+// steps, retirement with the final averages).
 //
 // Compiled with -ffp-contract=off (host arithmetic included).
 #include <hip/hip_runtime.h>
@@ -68,18 +68,11 @@ struct Batch {
     std::vector<hipStream_t> sstream;
     std::vector<hipEvent_t> sdone;
     int chunk = 0;            // launches per chunk = max steps
-    hipGraphExec_t graph = nullptr;
     hipEvent_t ev = nullptr;
 
     ~Batch() { release(); }
-    void drop_graph()
-    {
-        if (graph) (void)hipGraphExecDestroy(graph);
-        graph = nullptr;
-    }
     void release()
     {
-        drop_graph();
         if (dev) (void)hipFree(dev);
         dev = nullptr;
         dev_cap = 0;
@@ -121,7 +114,6 @@ int kind_of(const ch4g_lattice *L) { return (L->base.fluid ? BATCH_FLUID : 0) | 
 // population sets (one kernel instance per group).
 int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<int> &steps)
 {
-    B.drop_graph();
     B.lats = lats;
     B.steps = steps;
     B.host.clear();
@@ -294,8 +286,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
 }
 
 // The chunk's launches: group 0 on the batch stream, group g > 0 on its own
-// stream forked from and joined back into the batch stream (under capture
-// this makes parallel branches of one graph).
+// stream forked from and joined back into the batch stream.
 int launch_steps(Batch &B)
 {
     const size_t ng = B.groups.size(), ns = B.solo.size();
@@ -357,37 +348,19 @@ int launch_steps(Batch &B)
 
 // Advance every lattice of the table by its steps of one chunk (ordered
 // after each lattice's own queued work, and before any work queued on it
-// later); the launches are replayed from a captured graph when asked.
-int advance(Batch &B, bool use_graph)
+// later).  The launches are enqueued one by one: a served chunk captured as
+// one graph, with a branch for each group, was replayed instead until two
+// served streams ended their process with a host segmentation fault whose
+// cause is not known.
+int advance(Batch &B)
 {
     if (B.lats.empty() || B.chunk <= 0) return 0;
     for (ch4g_lattice *L : B.lats) {
         HIPCHK(hipEventRecord(B.ev, L->stream));
         HIPCHK(hipStreamWaitEvent(B.stream, B.ev, 0));
     }
-    if (use_graph) {
-        if (!B.graph) {
-            hipGraph_t g = nullptr;
-            HIPCHK(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
-            int lrc = launch_steps(B);
-            hipError_t e = hipStreamEndCapture(B.stream, &g);
-            if (lrc) {
-                if (g) (void)hipGraphDestroy(g);
-                return lrc;
-            }
-            if (e != hipSuccess) return fail(-2, "hipStreamEndCapture failed: %s", hipGetErrorString(e));
-            e = hipGraphInstantiate(&B.graph, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
-            if (e != hipSuccess) {
-                B.graph = nullptr;
-                return fail(-2, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
-            }
-        }
-        HIPCHK(hipGraphLaunch(B.graph, B.stream));
-    } else {
-        int lrc = launch_steps(B);
-        if (lrc) return lrc;
-    }
+    int lrc = launch_steps(B);
+    if (lrc) return lrc;
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(B.ev, B.stream));
     for (ch4g_lattice *L : B.lats) HIPCHK(hipStreamWaitEvent(L->stream, B.ev, 0));
@@ -444,7 +417,7 @@ int ch4g_step_batch(ch4g_lattice *const *lats, int n, int nsteps)
     thread_local Batch B;
     int rc = build(B, v, std::vector<int>((size_t)n, nsteps));
     if (rc) return rc;
-    rc = advance(B, false);
+    rc = advance(B);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(B.stream));
     commit(B);
@@ -559,8 +532,8 @@ int ch4g_serve(const ch4g_serve_params *sp, ch4g_job *jobs, int32_t njobs)
         // ---- one chunk.  Batched: every resident job takes part, with all
         // the chunk's steps (lock-step) or a share proportional to its
         // remaining steps, spread over the chunk's launches (even shares keep
-        // each lattice's buffer parity, so the tables and their captured
-        // graph stay valid until the set changes; a job that can finish
+        // each lattice's buffer parity, so the tables stay valid until the
+        // set changes; a job that can finish
         // does); shares are refreshed every 16 chunks.  Jobs that arrived
         // while the chunk ran are set up after it and join the next one.
         // Plain: the single job runs to its end in one call.
@@ -584,9 +557,9 @@ int ch4g_serve(const ch4g_serve_params *sp, ch4g_job *jobs, int32_t njobs)
                 table_dirty = false;
                 chunks_since_share = 0;
             }
-            if ((rc = advance(B, sp->use_graphs != 0))) break;
+            if ((rc = advance(B))) break;
             const size_t in_chunk = B.lats.size(); // active[0 .. in_chunk) take part
-            // The chunk (a graph whose branches run on several streams)
+            // The chunk, whose branches run on several streams,
             // completes before any other runtime call: admission allocates,
             // frees and launches, and doing that while a chunk was in flight
             // ended the process in the runtime now and then.

@@ -65,3 +65,22 @@ S.stub_reset()
 step_batch(lats[:1], 7)
 assert launches(b"k_step2y_fp64") == 3 and launches() == 4, launches()
 """)
+
+
+# A served stream (arrivals, odd shares, a rebuilt table, jobs of every group)
+# captures no graph while jobs run together.
+def test_served_chunks_are_launched_not_captured(run):
+    run("""
+cfgs = [workloads.rb2d(48, 24, 1, Ra=2e5, precision=abi.FP64), workloads.channel3d(8, 24, 6, precision=abi.FP64),
+        workloads.rb2d(96, 48, 1, Ra=1e6), workloads.channel3d(40, 24, 20)]
+jobs = []
+for i, cfg in enumerate(cfgs):
+    j = abi.Job()
+    j.cfg, j.nsteps, j.arrival_s = cfg, 60 - 7 * i, 0.001 * i
+    jobs.append(j)
+for schedule in (abi.SCHEDULE_LOCKSTEP, abi.SCHEDULE_PROPORTIONAL):
+    done = serve([abi.Job.from_buffer_copy(j) for j in jobs], mode=abi.SERVE_BATCHED, chunk_steps=7,
+                 use_graphs=True, schedule=schedule)
+    assert all(d.status == 0 for d in done)
+    assert S.stub_captures() == 0 and launches(b"k_step_batch32") > 0 and launches(b"k_step2_batch64") > 0
+""")
