@@ -284,3 +284,52 @@ def test_gradient_interpolation_counts(kind, n):
         got.append(x.particles())
     for f in abi.PARTICLE_FIELDS:
         assert np.array_equal(got[0][f], got[1][f], equal_nan=True), f
+
+
+# FP64 members of a batch that take one step per launch there (k_step_batch64:
+# linear and row grids, with and without temperature, temperature alone, the
+# local-strain closure; lattices of few columns, two of them; streamed in groups
+# of blocks with non-temporal stores) and a z-marching lattice on its own branch
+# beside them.  Random populations; equal, bit for bit, to each alone in single
+# steps, for odd and even counts.
+@pytest.mark.parametrize("kind", ["small", "les", "branch", "streamed"])
+def test_fp64_batched_single_steps(kind):
+    from ch4g import step_batch, workloads
+    rb, ch = configs.rb2d, workloads.channel3d
+
+    def les(cfg):
+        cfg.flags |= abi.FLUID_LES | abi.FLUID_LES_LOCAL_STRAIN
+        if cfg.has(abi.LB_TEMPERATURE):
+            cfg.flags |= abi.TEMPERATURE_LES
+        cfg.les_cs = 0.1
+        return cfg
+
+    conduction = rb(40, 12, 9, Ra=1e4)
+    conduction.flags &= ~(abi.LB_FLUID | abi.TEMPERATURE_BUOYANCY | abi.FLUID_BC_Y)
+    cfgs = {"small": [rb(48, 40, 30, Ra=1e5), rb(64, 24, 20, Ra=1e5), ch(40, 24, 20, precision=abi.FP64),
+                      ch(128, 20, 12, precision=abi.FP64), conduction, ch(4, 16, 4, precision=abi.FP64),
+                      rb(5, 10, 7, Ra=1e4)],
+            "les": [les(rb(20, 14, 9, Ra=1e5)), les(rb(64, 9, 5, Ra=1e5)), les(ch(61, 17, 8, precision=abi.FP64))],
+            "branch": [rb(96, 80, 112, Ra=1e6), ch(24, 20, 16, precision=abi.FP64), ch(8, 24, 6, precision=abi.FP64)],
+            "streamed": [les(rb(128, 160, 130, Ra=1e6))]}[kind]
+    many, one = [Lattice(c) for c in cfgs], [Lattice(c) for c in cfgs]
+    two = [lat.steps_per_launch() == 2 for lat in many]
+    assert two == {"small": [False] * 5 + [True] * 2, "les": [False] * 3, "branch": [True, False, True],
+                   "streamed": [False]}[kind]
+    rng = np.random.default_rng(8)
+    for a, b in zip(many, one):
+        b.set_fusion(False)
+        a.initial_conditions()
+        p, g = (x * (1.0 + 1e-2 * rng.uniform(-1, 1, x.shape)) for x in a.get_populations())
+        for lat in (a, b):
+            lat.set_populations(p, g if a.cfg.has(abi.LB_TEMPERATURE) else None)
+            lat.step(1)
+    for n in (1, 7, 10) if kind != "streamed" else (3,):
+        step_batch(many, n)
+        for a, b in zip(many, one):
+            b.step(n)
+            for x, y in zip(a.get_populations(), b.get_populations()):
+                assert np.array_equal(x, y), (n, a.cfg.NX, a.cfg.NY, a.cfg.NZ)
+            assert np.isfinite(a.get_populations()[0]).all()
+    for lat in many + one:
+        lat.close()
