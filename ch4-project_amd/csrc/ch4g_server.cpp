@@ -62,9 +62,11 @@ struct Batch {
     std::vector<char> flips;  // a chunk changes lattice i's buffer or lag parity
     // 3-D lattices large enough for two steps per launch alone (the z march:
     // k_step2z_fp32, k_step2z_fp64), and a single slab lattice, run their own
-    // launches as a branch of the chunk on a stream of their own instead of
-    // joining a batched group
+    // launches as branches of the chunk instead of joining a batched group, on
+    // up to SOLO_STREAMS streams (more than there are hardware queues)
+    static constexpr size_t SOLO_STREAMS = 8;
     std::vector<int> solo;    // lattice indices
+    size_t solo_streams() const { return std::min(solo.size(), SOLO_STREAMS); }
     std::vector<hipStream_t> sstream;
     std::vector<hipEvent_t> sdone;
     int chunk = 0;            // launches per chunk = max steps
@@ -251,7 +253,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         B.gdone.push_back(e);
     }
-    while (B.sstream.size() < B.solo.size()) {
+    while (B.sstream.size() < B.solo_streams()) {
         hipStream_t t = nullptr;
         hipEvent_t e = nullptr;
         HIPCHK(hipStreamCreateWithFlags(&t, hipStreamNonBlocking));
@@ -289,7 +291,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
 // stream forked from and joined back into the batch stream.
 int launch_steps(Batch &B)
 {
-    const size_t ng = B.groups.size(), ns = B.solo.size();
+    const size_t ng = B.groups.size(), ns = B.solo_streams();
     if (ng > 1 || ns > 0) {
         HIPCHK(hipEventRecord(B.fork, B.stream));
         for (size_t g = 1; g < ng; g++) HIPCHK(hipStreamWaitEvent(B.gstream[g - 1], B.fork, 0));
@@ -298,10 +300,10 @@ int launch_steps(Batch &B)
     // solo 3-D lattices: their share as two-step launches (plus one single
     // step for an odd share) from the buffers and lag arrays of the chunk's
     // start, exactly as ch4g_step advances them
-    for (size_t k = 0; k < ns; k++) {
+    for (size_t k = 0; k < B.solo.size(); k++) {
         ch4g_lattice *L = B.lats[(size_t)B.solo[k]];
         const int st = B.steps[(size_t)B.solo[k]];
-        hipStream_t t = B.sstream[k];
+        hipStream_t t = B.sstream[k % ns];
         const KParams P = params_for(L, 0, (int)L->itime + 1);
         int cur = L->cur;
         void *tl = L->tlag, *ta = L->tlag_alt;
@@ -316,8 +318,8 @@ int launch_steps(Batch &B)
         else if (st & 1)
             launch_step_fp64(P, (const double *)L->f[cur], (const double *)L->g[cur], (double *)L->f[cur ^ 1],
                              (double *)L->g[cur ^ 1], (double *)tl, (double *)L->taules, t);
-        HIPCHK(hipEventRecord(B.sdone[k], t));
     }
+    for (size_t k = 0; k < ns; k++) HIPCHK(hipEventRecord(B.sdone[k], B.sstream[k]));
     for (size_t g = 0; g < ng; g++) {
         const Batch::Group &G = B.groups[g];
         hipStream_t st = g == 0 ? B.stream : B.gstream[g - 1];

@@ -84,3 +84,15 @@ for schedule in (abi.SCHEDULE_LOCKSTEP, abi.SCHEDULE_PROPORTIONAL):
     assert all(d.status == 0 for d in done)
     assert S.stub_captures() == 0 and launches(b"k_step_batch32") > 0 and launches(b"k_step2_batch64") > 0
 """)
+
+
+# Lattices on branches of their own share a bounded number of streams.
+def test_branches_share_streams(run):
+    run("""
+lats = [started(workloads.channel3d(64, 64, 256)) for _ in range(20)]
+assert lats[0].steps_per_launch() == 2
+S.stub_reset()
+step_batch(lats, 4)
+assert launches(b"k_step2z_fp32") == launches() == 40
+assert S.stub_streams_made() <= 1 + 8, S.stub_streams_made()
+""")
