@@ -394,12 +394,23 @@ double seconds_since(std::chrono::steady_clock::time_point t0)
     return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
-// device bytes a job holds: populations and lags, the FP64 fields and
-// partial sums of its final dump_averages, the per-row base tables
+// device bytes a job holds: populations and lag, the FP64 fields and
+// partial sums of its final dump_averages, the per-row base tables, the HIT
+// tables
 int64_t job_bytes(const ch4g_config &c)
 {
     const int64_t N = (int64_t)c.NX * c.NY * c.NZ;
-    return ch4g_footprint_bytes(&c) + N * 40 + ((int64_t)1 << 20);
+    const int64_t hit = (c.flags & CH4G_FLUID_FORCING_HIT)
+                            ? (int64_t)2 * HIT_AHEAD * CH4G_HIT_NK * ((int64_t)c.NX + c.NY + c.NZ) * 8
+                            : 0;
+    return ch4g_footprint_bytes(&c) + N * 40 + ((int64_t)1 << 20) + hit;
+}
+
+// ... and, with a temperature, the second lag array of two steps per launch
+int64_t second_lag_bytes(const ch4g_config &c)
+{
+    if (!(c.flags & CH4G_LB_TEMPERATURE)) return 0;
+    return (int64_t)c.NX * c.NY * c.NZ * (c.precision == CH4G_FP64 ? 8 : 4);
 }
 
 }  // namespace
@@ -485,7 +496,7 @@ int ch4g_serve(const ch4g_serve_params *sp, ch4g_job *jobs, int32_t njobs)
         const double now = seconds_since(t0);
         while (next < order.size() && jobs[order[next]].arrival_s <= now) {
             ch4g_job &J = jobs[order[next]];
-            const int64_t nb = job_bytes(J.cfg);
+            int64_t nb = job_bytes(J.cfg);
             if (nb > budget) { // can never fit
                 J.status = fail(-3, "job needs %lld bytes, budget %lld", (long long)nb, (long long)budget);
                 next++;
@@ -493,6 +504,10 @@ int ch4g_serve(const ch4g_serve_params *sp, ch4g_job *jobs, int32_t njobs)
                 continue;
             }
             if (!batched && !active.empty()) break;
+            // a budget without room for the second lag array: single steps
+            const int64_t lag = second_lag_bytes(J.cfg);
+            const bool two = nb + lag <= budget;
+            if (two) nb += lag;
             if (used + nb > budget || (sp->max_active > 0 && (int)active.size() >= sp->max_active)) break;
             ch4g_lattice *L = nullptr;
             int r = ch4g_create(&J.cfg, &L);
@@ -500,6 +515,7 @@ int ch4g_serve(const ch4g_serve_params *sp, ch4g_job *jobs, int32_t njobs)
             if (!r && batched && (L->base.hit || L->base.les_fd || L->d_f0))
                 r = fail(-1, "HIT-forced, finite-difference LES and NOZEROMODE jobs are not batched (serve them "
                              "with CH4G_SERVE_SEQUENTIAL)");
+            if (!r && !two) r = ch4g_set_fusion(L, 0);
             if (!r && J.nsteps > 0) r = ch4g_step(L, 1); // first step: reads the initial populations
             if (r) {
                 if (L) ch4g_destroy(L);

@@ -448,7 +448,10 @@ typedef struct ch4g_serve_params {
  * they finish.  Returns when every job is done or rejected.                */
 int ch4g_serve(const ch4g_serve_params *sp, ch4g_job *jobs, int32_t njobs);
 
-/* Device bytes a lattice with this configuration would hold (admission). */
+/* Device bytes ch4g_create allocates for the populations and per-node arrays
+ * of this configuration (admission).  Calls that need more allocate it at their
+ * first use: a lattice with temperature that takes two steps per launch one
+ * more real per node, the field outputs their FP64 fields.                  */
 int64_t ch4g_footprint_bytes(const ch4g_config *cfg);
 
 #ifdef __cplusplus

@@ -20,7 +20,7 @@ std::map<std::string, long> launched;
 std::map<void *, size_t> device;  // live allocations
 std::set<void *> streams, events;
 long mallocs = 0, fail_from = -1, fail_to = -1, streams_made = 0, captures = 0;
-size_t fail_bytes = 0;
+size_t fail_bytes = 0, live_bytes = 0, peak_bytes = 0;
 hipError_t last = hipSuccess;
 
 struct Config {
@@ -48,12 +48,8 @@ long stub_launches(const char *part)
         if (k.first.find(part) != std::string::npos) n += k.second;
     return n;
 }
-size_t stub_live_bytes()
-{
-    size_t n = 0;
-    for (auto &d : device) n += d.second;
-    return n;
-}
+size_t stub_live_bytes() { return live_bytes; }
+size_t stub_peak_bytes() { return peak_bytes; }  // since stub_reset
 long stub_streams_made() { return streams_made; }
 long stub_captures() { return captures; }
 // device allocations fail: those of at least `bytes`, from the `first` such
@@ -69,6 +65,7 @@ void stub_reset()
 {
     launched.clear();
     streams_made = captures = 0;
+    peak_bytes = live_bytes;
 }
 
 // ---- the runtime
@@ -111,11 +108,16 @@ hipError_t hipMalloc(void **p, size_t n)
     *p = calloc(1, n ? n : 1);
     if (!*p) return ret(hipErrorOutOfMemory);
     device[*p] = n;
+    live_bytes += n;
+    if (live_bytes > peak_bytes) peak_bytes = live_bytes;
     return hipSuccess;
 }
 hipError_t hipFree(void *p)
 {
-    if (!device.erase(p)) return ret(hipErrorInvalidValue);
+    auto d = device.find(p);
+    if (d == device.end()) return ret(hipErrorInvalidValue);
+    live_bytes -= d->second;
+    device.erase(d);
     free(p);
     return hipSuccess;
 }

@@ -16,7 +16,7 @@ import ctypes as C, sys
 sys.path[:0] = [{os.path.join(ROOT, 'ch4-project_amd')!r}, {HERE!r}]
 S = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 S.stub_launches.restype = S.stub_streams_made.restype = S.stub_captures.restype = C.c_long
-S.stub_live_bytes.restype = C.c_size_t
+S.stub_live_bytes.restype = S.stub_peak_bytes.restype = C.c_size_t
 S.stub_fail.argtypes = [C.c_size_t, C.c_long, C.c_long]
 import numpy as np
 from ch4g import abi, footprint_bytes, Lattice, serve, step_batch, workloads
@@ -95,4 +95,28 @@ S.stub_reset()
 step_batch(lats, 4)
 assert launches(b"k_step2z_fp32") == launches() == 40
 assert S.stub_streams_made() <= 1 + 8, S.stub_streams_made()
+""")
+
+
+# A served job never holds more than the budget, the second lag array of two
+# steps per launch included; where only that does not fit, it takes single steps.
+@pytest.mark.parametrize("mode", ["SERVE_BATCHED", "SERVE_SEQUENTIAL"])
+@pytest.mark.parametrize("precision", ["FP64", "FP32_DEV"])
+def test_served_job_stays_in_its_budget(run, mode, precision):
+    run(f"""
+cfg = workloads.rb2d(1024, 512, 1, Ra=1e6, precision=abi.{precision})
+real = 8 if cfg.precision == abi.FP64 else 4
+tables = 1 << 18  # of the batch
+need = footprint_bytes(cfg) + 40 * cfg.nodes() + (1 << 20)
+for extra, two in ((0, False), (real * cfg.nodes() + tables, True)):
+    job = abi.Job()
+    job.cfg, job.nsteps = cfg, 9
+    S.stub_reset()
+    done = serve([job], mode=abi.{mode}, hbm_budget=need + extra)
+    assert done[0].status == 0
+    assert S.stub_peak_bytes() <= need + extra, (S.stub_peak_bytes(), need + extra)
+    assert (launches(b"k_step2") > 0) == two
+job = abi.Job()
+job.cfg, job.nsteps = cfg, 9
+assert serve([job], mode=abi.{mode}, hbm_budget=need - 1)[0].status < 0
 """)
