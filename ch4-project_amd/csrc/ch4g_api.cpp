@@ -355,15 +355,20 @@ int ensure_tlag_alt(ch4g_lattice *L)
     return 0;
 }
 
-// ... with the second lag array in place; single steps where no memory is left
+// ... with the second lag array in place.  Where no memory is left the call
+// takes single steps; the next one asks again.
 bool two_step_ready(ch4g_lattice *L)
 {
     if (!two_step_eligible(L)) return false;
-    if (!ensure_tlag_alt(L)) return true;
-    (void)hipGetLastError();
-    g_err[0] = 0;
-    L->use_fusion = false;
-    return false;
+    if (!L->base.thermal || L->tlag_alt) return true;
+    if (ensure_tlag_alt(L)) {
+        (void)hipGetLastError();
+        g_err[0] = 0;
+        return false;
+    }
+    // graphs captured meanwhile hold single steps
+    if (hipStreamSynchronize(L->stream) == hipSuccess) destroy_graphs(L);
+    return true;
 }
 
 }  // namespace ch4g
@@ -388,9 +393,8 @@ int launch_two_steps(ch4g_lattice *L)
 // Capture (once per starting buffer pair) and replay GRAPH_STEPS
 // steady-state steps.  Kernel arguments of these steps depend only on the
 // buffer parities.
-int replay_graph(ch4g_lattice *L)
+int replay_graph(ch4g_lattice *L, bool two)
 {
-    const bool two = two_step_ready(L); // allocates before any capture
     const int start = L->cur | (L->tpar << 1);
     if (!L->graph[start]) {
         hipGraph_t g = nullptr;
@@ -805,17 +809,21 @@ int ch4g_step(ch4g_lattice *L, int nsteps)
     // HIT tables ahead: 1, 2, 4, ... steps, so that the first kernel does not
     // wait for all of them
     int ahead = 1;
+    // two steps per launch: asked once, past the first step (it may allocate,
+    // which a capture may not)
+    int two = -1;
     while (s < nsteps) {
+        if (two < 0 && !L->first && nsteps - s >= 2) two = two_step_ready(L);
         // Steady-state steps (not the first, no per-step host forcing tables,
         // no particles) depend only on the buffer parities: replay a captured
         // GRAPH_STEPS-step graph instead of launching.
         if (L->use_graphs && !L->first && L->itime >= 1 && !L->base.hit && !L->part && nsteps - s >= GRAPH_STEPS) {
-            int rc = replay_graph(L);
+            int rc = replay_graph(L, two > 0);
             if (rc) return rc;
             s += GRAPH_STEPS;
             continue;
         }
-        if (nsteps - s >= 2 && two_step_ready(L)) {
+        if (nsteps - s >= 2 && two > 0) {
             int rc = launch_two_steps(L);
             if (rc) return rc;
             s += 2;

@@ -200,8 +200,9 @@ int ch4g_set_fusion(ch4g_lattice *lat, int enable);
  * steps through an LDS tile), 3-D and large enough (k_step2z_fp32,
  * k_step2z_fp64: x-y tiles marching along z through an LDS ring of planes;
  * from about 96^3 where rows fill their tiles) or, FP64, 3-D of few columns
- * (k_step2y_fp64), else 1.  Odd remainders run
- * as single steps; results are identical either way.  No reference
+ * (k_step2y_fp64), else 1.  Odd remainders run as single steps, and so does
+ * a call that finds no memory for a thermal lattice's second lag array (one
+ * real per node); results are identical either way.  No reference
  * counterpart (launch mechanics of this library).                          */
 int ch4g_steps_per_launch(const ch4g_lattice *lat, int *steps);
 

@@ -120,3 +120,26 @@ job = abi.Job()
 job.cfg, job.nsteps = cfg, 9
 assert serve([job], mode=abi.{mode}, hbm_budget=need - 1)[0].status < 0
 """)
+
+
+# No memory for the second lag array: single steps in that call, two per launch
+# again once there is room; ch4g_set_fusion's setting is the caller's alone.
+def test_two_steps_return_when_memory_does(run):
+    run("""
+for cfg in (workloads.rb2d(512, 128, 1, precision=abi.FP64), workloads.rb2d(512, 128, 1, precision=abi.FP32_DEV)):
+    lat = started(cfg)
+    S.stub_fail(4 * cfg.nodes(), 0, 1000)
+    S.stub_reset()
+    lat.step(70)
+    assert launches(b"k_step2") == 0 and launches(b"k_step_fp") > 0 and lat.itime == 71
+    step_batch([lat], 5)
+    assert launches(b"k_step2") == 0 and launches(b"k_step_batch") == 5
+    S.stub_fail(0, 0, 0)
+    S.stub_reset()
+    lat.step(70)
+    assert launches(b"k_step_fp") == 0 and launches(b"k_step2_fp") == 16 + 3 and lat.itime == 146
+    S.stub_reset()
+    step_batch([lat], 4)
+    assert launches(b"k_step2_batch") == launches() == 2
+    lat.close()
+""")
