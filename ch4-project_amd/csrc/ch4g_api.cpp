@@ -35,6 +35,12 @@ int fail(int code, const char *fmt, ...)
     return code;
 }
 
+void forget_error()
+{
+    (void)hipGetLastError();
+    g_err[0] = 0;
+}
+
 }  // namespace ch4g
 
 namespace ch4g {
@@ -362,8 +368,7 @@ bool two_step_ready(ch4g_lattice *L)
     if (!two_step_eligible(L)) return false;
     if (!L->base.thermal || L->tlag_alt) return true;
     if (ensure_tlag_alt(L)) {
-        (void)hipGetLastError();
-        g_err[0] = 0;
+        forget_error();
         return false;
     }
     // graphs captured meanwhile hold single steps

@@ -351,6 +351,22 @@ struct RecordBufs {
     void *tmp;
     size_t tmp_bytes;
 };
+// Row of each member of ch4g_particle, in the struct's order.
+constexpr int NREC = (int)(sizeof(ch4g_particle) / sizeof(double));
+struct RecordRows {
+    uint8_t row[NREC];
+    int n;
+    constexpr RecordRows() : row(), n(0)
+    {
+        // runs of consecutive rows: {first row, count}
+        constexpr int run[][2] = {{PNAME, 1}, {PX, 3}, {PVX, 3}, {PVXO, 3}, {PAX, 3}, {PAXO, 3}, {PUX, 3}, {PUXO, 3},
+                                  {PG, 9}, {PDTU, 3}, {PT, 3}, {PTAU, 2}, {PGT, 3}, {PPO, 6}, {PASP, 3}, {PNO, 6},
+                                  {PTP, 2}, {PGC, 1}, {PSED, 1}, {PCT, 12}, {PCSR, 7}};
+        for (auto &r : run)
+            for (int k = 0; k < r[1]; k++) row[n++] = (uint8_t)(r[0] + k);
+    }
+};
+static_assert(RecordRows().n == NREC, "the runs cover the record");
 size_t live_scan_bytes(int64_t np);
 int launch_live_rows(const PartParams &P, const RecordBufs &B, hipStream_t s);
 int launch_records(const PartParams &P, const int *src, int64_t m, double *out, hipStream_t s);

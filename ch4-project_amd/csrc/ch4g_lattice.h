@@ -55,8 +55,8 @@ struct Particles {
     size_t ro_tmp_bytes = 0;
     int cell_bits = 32;
     int64_t last_reorder = 0;
-    // reading the records back: [4][cap] flags, ranks and rows by reference
-    // index and live rows, scan scratch, one chunk of records
+    // reading the records back, one allocation: [4][cap] flags, ranks and rows
+    // by reference index and live rows, scan scratch, one chunk of records
     int *d_live = nullptr;
     void *d_scan_tmp = nullptr;
     size_t scan_tmp_bytes = 0;
@@ -130,6 +130,7 @@ namespace ch4g {
 
 // error reporting shared by the C-ABI units (message via ch4g_last_error)
 int fail(int code, const char *fmt, ...);
+void forget_error();  // of a call that went on without what failed
 int dalloc(ch4g_lattice *L, void **p, size_t bytes);
 int ensure_scratch(ch4g_lattice *L);
 KParams params_for(const ch4g_lattice *L, int first, int itime);

@@ -274,7 +274,7 @@ void free_state(Particles *P)
 {
     void *ptrs[] = {P->d_state, P->d_alive, P->d_ndraw, P->d_bsum, P->d_kin, P->d_vin, P->d_vout, P->d_sort_tmp,
                     P->d_keys[0], P->d_keys[1], P->d_rec, P->d_dep, P->d_ord, P->d_head, P->d_orig, P->d_orig2, P->d_alive2,
-                    P->d_state2, P->d_ck, P->d_ck2, P->d_cv, P->d_cv2, P->d_ro_tmp, P->d_live, P->d_scan_tmp, P->d_records};
+                    P->d_state2, P->d_ck, P->d_ck2, P->d_cv, P->d_cv2, P->d_ro_tmp, P->d_records};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     P->d_state = nullptr;
@@ -1008,6 +1008,39 @@ int ch4g_particles_count(ch4g_lattice *L, int64_t *n)
     return 0;
 }
 
+namespace {
+
+// ch4g_get_particles without device memory of its own: the state read back a
+// row at a time.
+int records_by_row(ch4g_lattice *L, ch4g_particle *out, int64_t cap, int64_t *n)
+{
+    Particles *Q = L->part;
+    const size_t np = (size_t)Q->np;
+    std::vector<int> alive(np), orig(np);
+    HIPCHK(hipMemcpyAsync(alive.data(), Q->d_alive, np * sizeof(int), hipMemcpyDeviceToHost, L->stream));
+    HIPCHK(hipMemcpyAsync(orig.data(), Q->d_orig, np * sizeof(int), hipMemcpyDeviceToHost, L->stream));
+    HIPCHK(hipStreamSynchronize(L->stream));
+    // place of each row's record: its rank among the live ones in reference order
+    std::vector<int64_t> row_of(np), place(np, -1);
+    for (size_t p = 0; p < np; p++) row_of[(size_t)orig[p]] = (int64_t)p;
+    int64_t live = 0;
+    for (int64_t p : row_of)
+        if (alive[(size_t)p]) place[(size_t)p] = live++;
+    constexpr RecordRows rows;
+    std::vector<double> v(np);
+    for (int f = 0; f < NREC; f++) {
+        HIPCHK(hipMemcpyAsync(v.data(), Q->d_state + (int64_t)rows.row[f] * Q->cap, np * sizeof(double),
+                              hipMemcpyDeviceToHost, L->stream));
+        HIPCHK(hipStreamSynchronize(L->stream));
+        for (size_t p = 0; p < np; p++)
+            if (place[p] >= 0 && place[p] < cap) (&out[place[p]].name)[f] = v[p];
+    }
+    *n = live;
+    return 0;
+}
+
+}  // namespace
+
 int ch4g_get_particles(ch4g_lattice *L, ch4g_particle *out, int64_t cap, int64_t *n)
 {
     if (!L || !n || (cap > 0 && !out)) return fail(-1, "null argument");
@@ -1018,13 +1051,17 @@ int ch4g_get_particles(ch4g_lattice *L, ch4g_particle *out, int64_t cap, int64_t
     // be in cell order) and copied straight to the caller: reading all rows
     // back and forming them on the host took 220 ms for 500,000 particles
     const int64_t np = Q->np, c = Q->cap;
-    int rc;
-    if (!Q->d_live) {
-        const size_t chunk = (size_t)(c < RECORD_CHUNK ? c : RECORD_CHUNK);
+    if (!Q->d_records) {
+        auto lines = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
         Q->scan_tmp_bytes = live_scan_bytes(c);
-        if ((rc = dalloc(L, (void **)&Q->d_records, chunk * sizeof(ch4g_particle)))) return rc;
-        if ((rc = dalloc(L, &Q->d_scan_tmp, Q->scan_tmp_bytes > 0 ? Q->scan_tmp_bytes : 1))) return rc;
-        if ((rc = dalloc(L, (void **)&Q->d_live, (size_t)4 * c * sizeof(int)))) return rc;
+        const size_t rec = lines((size_t)(c < RECORD_CHUNK ? c : RECORD_CHUNK) * sizeof(ch4g_particle)),
+                     scan = lines(Q->scan_tmp_bytes);
+        if (dalloc(L, (void **)&Q->d_records, rec + scan + (size_t)4 * c * sizeof(int))) {
+            forget_error();
+            return records_by_row(L, out, cap, n);
+        }
+        Q->d_scan_tmp = (char *)Q->d_records + rec;
+        Q->d_live = (int *)((char *)Q->d_records + rec + scan);
     }
     const PartParams P = part_params(L);
     RecordBufs B;

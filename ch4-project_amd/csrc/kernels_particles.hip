@@ -1595,23 +1595,7 @@ __global__ void __launch_bounds__(PB) k_permute(PartParams P, const uint32_t *sr
     }
 }
 
-// Row of each member of ch4g_particle, in the struct's order.
-constexpr int NREC = (int)(sizeof(ch4g_particle) / sizeof(double));
-struct RecordRows {
-    uint8_t row[NREC];
-    int n;
-    constexpr RecordRows() : row(), n(0)
-    {
-        // runs of consecutive rows: {first row, count}
-        constexpr int run[][2] = {{PNAME, 1}, {PX, 3}, {PVX, 3}, {PVXO, 3}, {PAX, 3}, {PAXO, 3}, {PUX, 3}, {PUXO, 3},
-                                  {PG, 9}, {PDTU, 3}, {PT, 3}, {PTAU, 2}, {PGT, 3}, {PPO, 6}, {PASP, 3}, {PNO, 6},
-                                  {PTP, 2}, {PGC, 1}, {PSED, 1}, {PCT, 12}, {PCSR, 7}};
-        for (auto &r : run)
-            for (int k = 0; k < r[1]; k++) row[n++] = (uint8_t)(r[0] + k);
-    }
-};
 __constant__ constexpr RecordRows record_rows;
-static_assert(record_rows.n == NREC, "the runs cover the record");
 
 // alive flag and row of each particle by reference index
 __global__ void __launch_bounds__(PB) k_by_reference(PartParams P, int *flag, int *row)
@@ -1632,7 +1616,7 @@ __global__ void __launch_bounds__(PB) k_live_rows(int64_t np, const int *flag, c
 
 // Records of m particles: a thread per member, so that records are written as
 // one stream; the rows are read a value at a time.  Bound by the copy to the
-// host that follows (624 B a record over the host link).
+// host that follows (640 B a record over the host link).
 __global__ void __launch_bounds__(PB) k_records(PartParams P, const int *__restrict__ src, uint32_t m,
                                                 double *__restrict__ out)
 {

@@ -143,3 +143,36 @@ for cfg in (workloads.rb2d(512, 128, 1, precision=abi.FP64), workloads.rb2d(512,
     assert launches(b"k_step2_batch") == launches() == 2
     lat.close()
 """)
+
+
+# Particle records where the device has no room for the read-back buffers: the
+# same records, rows read one at a time; nothing is left over from the failed
+# allocation, and the buffers come once there is room.
+def test_particle_records_without_device_memory(run):
+    run("""
+lat = started(configs.poiseuille(8, 8, 8, tau=0.8, g=0.0), 0)
+lat.particles_init(abi.make_particle_config(abi.LAGRANGE_WRAP, 1))
+rng = np.random.default_rng(5)
+a = np.zeros(70001, dtype=abi.particle_dtype())
+for k in a.dtype.names:
+    a[k] = rng.uniform(1.0, 7.0, len(a))
+lat.set_particles(a)
+before = S.stub_live_bytes()
+for first in (0, 1, 2):
+    S.stub_fail(0, first, 1)
+    back = lat.particles()
+    if first == 0:
+        assert np.array_equal(back, a)
+        short = np.zeros(11, dtype=a.dtype)
+        n = C.c_int64()
+        S.stub_fail(0, 0, 1)
+        assert lat._L.ch4g_get_particles(lat.handle, short.ctypes.data, 10, C.byref(n)) == 0
+        assert n.value == len(a) and np.array_equal(short[:10], a[:10]) and not short[10:].view(np.float64).any()
+        assert S.stub_live_bytes() == before
+        assert launches(b"k_records") == 0
+kept = S.stub_live_bytes() - before
+assert a.dtype.itemsize * 65536 + 16 * len(a) <= kept <= a.dtype.itemsize * 65536 + 16 * len(a) + (1 << 20), kept
+S.stub_fail(0, 0, 0)
+lat.particles()
+assert S.stub_live_bytes() - before == kept
+""")
