@@ -13,6 +13,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <initializer_list>
 #include <mutex>
 #include <new>
 #include <utility>
@@ -35,11 +36,7 @@ int fail(int code, const char *fmt, ...)
     return code;
 }
 
-void forget_error()
-{
-    (void)hipGetLastError();
-    g_err[0] = 0;
-}
+void forget_error() { g_err[0] = 0; }
 
 }  // namespace ch4g
 
@@ -50,6 +47,7 @@ int dalloc(ch4g_lattice *L, void **p, size_t bytes)
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError();  // reported here, not by the next call's check
         return fail(-3, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     }
     L->bytes += (int64_t)bytes;
@@ -200,29 +198,42 @@ KParams params_for(const ch4g_lattice *L, int first, int itime)
     return P;
 }
 
+// Buffers that are used together: all of them or, where one fails, none (a
+// retry then starts over).
+struct Buffer {
+    double **p;
+    size_t doubles;
+};
+static int ensure(ch4g_lattice *L, std::initializer_list<Buffer> bufs)
+{
+    if (*bufs.begin()->p) return 0;
+    for (const Buffer &b : bufs) {
+        const int rc = dalloc(L, (void **)b.p, b.doubles * sizeof(double));
+        if (!rc) continue;
+        for (const Buffer *d = bufs.begin(); d != &b; d++) {
+            (void)hipFree(*d->p);
+            *d->p = nullptr;
+            L->bytes -= (int64_t)(d->doubles * sizeof(double));
+        }
+        return rc;
+    }
+    return 0;
+}
+
 int ensure_scratch(ch4g_lattice *L)
 {
     const size_t N = (size_t)L->N;
-    int rc;
-    if (!L->d_dens) {
-        if ((rc = dalloc(L, (void **)&L->d_dens, N * sizeof(double)))) return rc;
-        if ((rc = dalloc(L, (void **)&L->d_u, 3 * N * sizeof(double)))) return rc;
-        if ((rc = dalloc(L, (void **)&L->d_t, N * sizeof(double)))) return rc;
-        if ((rc = dalloc(L, (void **)&L->d_part, (size_t)reduce_blocks(L->base) * NOUT * sizeof(double)))) return rc;
-        if ((rc = dalloc(L, (void **)&L->d_res, NOUT * sizeof(double)))) return rc;
-    }
-    return 0;
+    return ensure(L, {{&L->d_dens, N},
+                      {&L->d_u, 3 * N},
+                      {&L->d_t, N},
+                      {&L->d_part, (size_t)reduce_blocks(L->base) * NOUT},
+                      {&L->d_res, NOUT}});
 }
 
 int ensure_stage(ch4g_lattice *L)
 {
     const size_t N = (size_t)L->N;
-    int rc;
-    if (!L->d_fs) {
-        if ((rc = dalloc(L, (void **)&L->d_fs, (size_t)Q * N * sizeof(double)))) return rc;
-        if ((rc = dalloc(L, (void **)&L->d_gs, (size_t)Q * N * sizeof(double)))) return rc;
-    }
-    return 0;
+    return ensure(L, {{&L->d_fs, (size_t)Q * N}, {&L->d_gs, (size_t)Q * N}});
 }
 
 // Gather of the current state into FP64 scratch (any output may be null).

@@ -1096,7 +1096,11 @@ int ch4g_set_particles(ch4g_lattice *L, const ch4g_particle *in, int64_t n)
     int rc;
     if (n > L->part->cap) {
         HIPCHK(hipStreamSynchronize(L->stream));
-        if ((rc = alloc_state(L, n))) return rc;
+        if ((rc = alloc_state(L, n))) {
+            // the old arrays are gone and the new ones are not there
+            particles_free(L);
+            return rc;
+        }
     }
     return upload(L, in, n);
 }

@@ -398,7 +398,8 @@ int ch4g_get_particles(ch4g_lattice *lat, ch4g_particle *out, int64_t cap, int64
 
 /* Replace the particle state (read_point_particle_h5 restart,
  * lagrange.c:128-131).  Requires ch4g_particles_init first; the count may
- * differ from particle_number.                                              */
+ * differ from particle_number.  Where the device has no room for a larger
+ * count, the lattice is left without particles.                             */
 int ch4g_set_particles(ch4g_lattice *lat, const ch4g_particle *in, int64_t n);
 
 /* ------------------------------------------------------------------------ */

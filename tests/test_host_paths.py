@@ -176,3 +176,43 @@ S.stub_fail(0, 0, 0)
 lat.particles()
 assert S.stub_live_bytes() - before == kept
 """)
+
+
+# An allocation that fails among several leaves nothing behind, and a retry gets
+# all of them (no call goes on with some of its buffers).
+@pytest.mark.parametrize("call,buffers", [("lat.hydro_fields()", 5), ("lat.dump_averages()", 5),
+                                          ("lat.get_populations()", 2)])
+def test_failed_allocations_are_taken_back(run, call, buffers):
+    run(f"""
+for k in range({buffers}):
+    lat = started(workloads.rb2d(64, 32, 1, precision=abi.FP64), 3)
+    live, own = S.stub_live_bytes(), lat.device_bytes
+    S.stub_fail(0, k, 1)
+    try:
+        {call}
+        raise SystemExit("call without its memory")
+    except Exception as e:
+        assert "hipMalloc" in str(e), e
+    assert (S.stub_live_bytes(), lat.device_bytes) == (live, own)
+    {call}
+    lat.close()
+""")
+
+
+def test_particles_without_memory_leave_the_lattice(run):
+    run("""
+flags = (abi.LAGRANGE_WRAP | abi.LAGRANGE_GRADIENT | abi.LAGRANGE_ADDEDMASS | abi.LAGRANGE_TWOWAY_MOMENTUM)
+for k in range(8):
+    lat = started(configs.poiseuille(8, 8, 8, tau=0.8, g=0.0), 0)
+    lat.particles_init(abi.make_particle_config(flags, 3, tau_drag=(1, 5.0, 5.0), beta_coeff=(1, 0.8, 0.8)))
+    S.stub_fail(0, k, 1)
+    try:
+        lat.set_particles(np.ones(50, dtype=abi.particle_dtype()))
+        raise SystemExit("particles without their memory")
+    except Exception as e:
+        assert "hipMalloc" in str(e), e
+    S.stub_reset()
+    lat.step(3)
+    assert launches() == launches(b"k_step") > 0 and lat.particles_count() == 0
+    lat.close()
+""")
