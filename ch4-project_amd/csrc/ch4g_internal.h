@@ -482,6 +482,10 @@ void launch_fields_f32(const KParams &P, const float *fin, const float *gin, con
 bool two_step_ok(const KParams &P);    // float storage
 bool two_step_ok64(const KParams &P);  // FP64
 bool two_step_slab64(const KParams &P);  // FP64, 3-D of few columns (launches of a few blocks)
+// FP64, 2-D with tiles that are mostly idle: their number, else 0; and whether
+// two steps pay for launches of so many
+int64_t two_step_thin64(const KParams &P);
+bool two_step_thin_pays64(int64_t tiles);
 void launch_two_steps_fp32(const KParams &P, const float *fin, const float *gin, float *fout, float *gout,
                            const float *tl_in, float *tl_out, hipStream_t s);
 void launch_two_steps_fp64(const KParams &P, const double *fin, const double *gin, double *fout, double *gout,

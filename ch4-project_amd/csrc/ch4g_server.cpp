@@ -132,7 +132,13 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
     // and together: 3.3 4.9, 6.3 5.5, 15.5 6.7, 52.6 10.6.
     auto slab_of = [](const ch4g_lattice *L) { return !L->dev32 && two_step_slab64(L->base); };
     int nslab = 0;
-    for (const ch4g_lattice *L : lats) nslab += L && slab_of(L);
+    // 2-D ones with mostly idle tiles take two steps while these are few in all
+    auto thin_of = [](const ch4g_lattice *L) { return L->dev32 ? 0 : two_step_thin64(L->base); };
+    int64_t thin = 0;
+    for (const ch4g_lattice *L : lats) {
+        nslab += L && slab_of(L);
+        thin += L ? thin_of(L) : 0;
+    }
     for (size_t i = 0; i < lats.size(); i++) {
         int rc = check_member(lats[i]);
         if (rc) return rc;
@@ -141,7 +147,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
         ch4g_lattice *L = lats[i];
         // two steps per launch: 2-D lattices in the batched two-step kernels,
         // large 3-D lattices on their own branch
-        B.two[i] = (nslab < 2 || !slab_of(L)) && two_step_ready(L);
+        B.two[i] = (nslab < 2 || !slab_of(L)) && (!thin_of(L) || two_step_thin_pays64(thin)) && two_step_ready(L);
         solo[i] = B.two[i] && L->cfg.NZ > 1;
         if (solo[i]) B.solo.push_back((int)i);
         // two-step lattices: the population buffer flips with every launch,

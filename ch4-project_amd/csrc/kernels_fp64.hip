@@ -1061,9 +1061,35 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
         sets(std::false_type{}, std::true_type{});
 }
 
+// 2-D lattices whose rows leave much of their tiles idle: less than 60 % full,
+// or a last tile of fewer than four columns in rows less than 80 % full (its
+// lanes' loads and stores share no lines) while the launch is a few rounds of
+// blocks.  Two steps pay for them only while one block per CU covers the lattice.  us per step, single -> two:
+// Rayleigh-Benard 4x1000 5.1 -> 4.4, 16x1000 5.6 -> 3.8, 33x256 5.3 -> 5.4; with
+// more tiles 1x30000 7.6 -> 57, 4x16000 7.7 -> 28, 16x4000 8.0 -> 8.9, 33x4000
+// 14.5 -> 19.8, 97x1000 11.0 -> 12.9; channel 8x20000 11.7 -> 16.5; and full
+// enough: 20x16000 -> 0.92 of single, 32x16000 56 -> 39, 40x4000 16.5 -> 16.9,
+// 48x16000 99 -> 71, 65x16000 138 -> 109, 97x4000 36.7 -> 34.7, 100x1000 11.0 ->
+// 10.5, 129x4000 -> 0.79.  Rows of one or two
+// nodes take longer in two steps at any length (1x64 3.6 -> 5.3).
+constexpr int64_t THIN_TILES = 256;
+static bool thin2d(const KParams &P)
+{
+    const int64_t lanes = (P.NX + T2D_TX - 1) / T2D_TX * T2D_TX, last = P.NX - (lanes - T2D_TX);
+    return (int64_t)P.NX * 10 < lanes * 6 ||
+           (last < 4 && (int64_t)P.NX * 10 < lanes * 8 && batch2_tiles64(P.NX, P.NY) < 8 * THIN_TILES);
+}
+
+// tiles of a lattice that takes two steps only while its launch is that small
+int64_t two_step_thin64(const KParams &P)
+{
+    return P.NZ == 1 && thin2d(P) ? batch2_tiles64(P.NX, P.NY) : 0;
+}
+bool two_step_thin_pays64(int64_t tiles) { return tiles <= THIN_TILES; }
+
 // Two steps per launch (k_step2_fp64, k_step2y_fp64, k_step2z_fp64): lattices
 // with the fluid whose planes buffer resources reach, without the general force
-// paths.  2-D: always (faster at every size measured, see k_step2_fp64).
+// paths.  2-D: see thin2d.
 // Tiles: 32 x 8 with the temperature (141 KB of LDS), 64 x 8 without (135 KB).
 using Tile64 = TileZ<true, true, 32, 8, true>;
 using Tile64F = TileZ<true, false, 64, 8, true>;
@@ -1083,7 +1109,8 @@ static int64_t z_columns64(const KParams &P)
 bool two_step_ok64(const KParams &P)
 {
     if (!P.fluid || P.first || P.hit || P.les || P.twoway || P.nozero || !planes_ok(P, 8)) return false;
-    if (P.NZ == 1 || slab_rows(P) > 0) return true;
+    if (P.NZ == 1) return !thin2d(P) || (P.NX >= 3 && two_step_thin_pays64(two_step_thin64(P)));
+    if (slab_rows(P) > 0) return true;
     const bool cached = state_bytes(P, 8) <= CACHED_BYTES;
     const double t_iter = P.thermal ? (cached ? 9.1 : 11.6) : (cached ? 6.5 : 9.5);           // us
     const double t_node = P.thermal ? (cached ? 92e-6 : 119e-6) : (cached ? 49e-6 : 57e-6);  // us

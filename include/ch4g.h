@@ -197,7 +197,8 @@ int ch4g_set_fusion(ch4g_lattice *lat, int enable);
 
 /* Steps one steady-state launch advances: 2 for lattices without HIT forcing,
  * LES, NOZEROMODE or particles that are 2-D (k_step2_fp32, k_step2_fp64: two
- * steps through an LDS tile), 3-D and large enough (k_step2z_fp32,
+ * steps through an LDS tile; FP64 not where long narrow rows leave the tiles
+ * mostly idle), 3-D and large enough (k_step2z_fp32,
  * k_step2z_fp64: x-y tiles marching along z through an LDS ring of planes;
  * from about 96^3 where rows fill their tiles) or, FP64, 3-D of few columns
  * (k_step2y_fp64), else 1.  Odd remainders run as single steps, and so does

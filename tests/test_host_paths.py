@@ -216,3 +216,24 @@ for k in range(8):
     assert launches() == launches(b"k_step") > 0 and lat.particles_count() == 0
     lat.close()
 """)
+
+
+# FP64 2-D lattices whose rows leave their tiles mostly idle take two steps per
+# launch only while their launches are small, alone and in a batch.
+def test_thin_2d_lattices_take_single_steps(run):
+    run("""
+def steps(nx, ny):
+    return Lattice(workloads.rb2d(nx, ny, 1, precision=abi.FP64)).steps_per_launch()
+
+for nx, ny in ((1, 64), (2, 1000), (1, 30000), (4, 5000), (8, 20000), (16, 10000), (33, 4000), (36, 1000), (97, 1000)):
+    assert steps(nx, ny) == 1, (nx, ny)
+for nx, ny in ((3, 64), (16, 1000), (33, 256), (20, 16000), (32, 16000), (40, 4000), (65, 16000), (97, 4000), (100, 1000),
+               (129, 1000), (512, 256)):
+    assert steps(nx, ny) == 2, (nx, ny)
+for n, two in ((3, True), (16, False)):
+    lats = [started(workloads.rb2d(6, 300, 1, precision=abi.FP64)) for _ in range(n)]
+    wide = started(workloads.rb2d(64, 32, 1, precision=abi.FP64))
+    S.stub_reset()
+    step_batch(lats + [wide], 8)
+    assert launches(b"k_step2_batch64") == 4 and launches(b"k_step_batch64") == (0 if two else 8)
+""")
