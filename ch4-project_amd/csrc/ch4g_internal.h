@@ -220,8 +220,11 @@ __device__ __forceinline__ uint32_t block_linear()
 // all XCDs work on the same planes of memory (256^3 988 -> 949 us; in eight
 // ranges 1000).  2-D tiles keep the eight ranges up to 1 GiB (2047x1021 102
 // -> 84, 2048x1024 85 -> 83; 4096x2048: 310 round-robin, 325 ranges, 301
-// groups).  FP64 (one step per launch): ranges up to 1.5 GiB, 2048x1024 280
-// -> 251, 128^3 265 -> 248; beyond in groups, 200^3 962 -> 947.
+// groups).  FP64, one step per launch, in eight ranges with plain stores -> in
+// groups (bytes of state): Rayleigh-Benard 16x200x200 (0.4 GB) 79 -> 76, 65x16000
+// (0.6) 140 -> 124, 100^3 (0.6) 125 -> 116, 130x100x120 (0.95) 215 -> 179; with
+// LES 128x64x128 (0.6) 136 -> 124, 128^3 (1.3) 258 -> 252, 96^3 (0.5) 116 -> 123;
+// forced turbulence 128^3 (0.6) 137 -> 130, 150^3 (1.0) 248 -> 227; 200^3 962 -> 947.
 constexpr int64_t CACHED_BYTES = (int64_t)320 << 20;
 struct StepOrder {
     bool nts;  // non-temporal stores
@@ -235,7 +238,7 @@ inline int64_t state_bytes(const KParams &P, int64_t rsz)
 {
     return 2 * (int64_t)Q * P.N * rsz * ((P.fluid ? 1 : 0) + (P.thermal ? 1 : 0));
 }
-constexpr int64_t RANGE_BYTES_2D = (int64_t)1 << 30, RANGE_BYTES_64 = (int64_t)3 << 29;
+constexpr int64_t RANGE_BYTES_2D = (int64_t)1 << 30;
 
 // compile-time loop over q
 template <int q, int Q_, typename F>

@@ -245,7 +245,7 @@ int build(Batch &B, const std::vector<ch4g_lattice *> &lats, const std::vector<i
             G.nblk[(size_t)k] = t0;
             B.slots.push_back({0u, (uint32_t)t0}); // sentinel
         }
-        G.order = step_order(bytes, whole_lines, G.two ? RANGE_BYTES_2D : G.dev32 ? CACHED_BYTES : RANGE_BYTES_64);
+        G.order = step_order(bytes, whole_lines, G.two ? RANGE_BYTES_2D : CACHED_BYTES);
         B.groups.push_back(G);
     }
     if (!B.stream) HIPCHK(hipStreamCreateWithFlags(&B.stream, hipStreamNonBlocking));

@@ -1025,9 +1025,7 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
         grid = dim3((unsigned)((P.N + 255) / 256));
         block = dim3(256);
     }
-    const StepOrder o = step_order(state_bytes(P, 8), dense || P.NX % 16 == 0, RANGE_BYTES_64);
-    // ranges and plain stores go together (see step_order)
-    const bool nt = o.nts && o.run == RUN_GROUP;
+    const StepOrder o = step_order(state_bytes(P, 8), dense || P.NX % 16 == 0, CACHED_BYTES);
     // planes beyond the reach of buffer resources take the general instance
     const bool buf = planes_ok(P, 8), gen = P.hit || P.les || P.twoway || P.nozero || !buf;
     auto sets = [&](auto fl, auto th) {
@@ -1038,7 +1036,7 @@ void launch_step_fp64(const KParams &P, const double *fin, const double *gin, do
             return;
         }
         with_bool(dense, [&](auto d) {
-            with_bool(nt, [&](auto n) {
+            with_bool(o.nts, [&](auto n) {
                 constexpr bool D = decltype(d)::value, NT = decltype(n)::value;
                 auto go = [&](auto g, auto bf) {
                     hipLaunchKernelGGL((k_step_fp64<false, FL, TH, D, NT, decltype(g)::value, decltype(bf)::value>),
@@ -1188,11 +1186,10 @@ void launch_batch_fp64(const BatchEntry *tab, const BatchSlot *slots, int nslots
 {
     dim3 grid((unsigned)nblocks), block(256);
     gen = gen || !buf;
-    const bool nt = o.nts && o.run == RUN_GROUP;
     auto sets = [&](auto fl, auto th) {
         constexpr bool FL = decltype(fl)::value, TH = decltype(th)::value;
         with_bool(dense, [&](auto d) {
-            with_bool(nt, [&](auto n) {
+            with_bool(o.nts, [&](auto n) {
                 constexpr bool D = decltype(d)::value, NT = decltype(n)::value;
                 auto go = [&](auto g, auto bf) {
                     hipLaunchKernelGGL((k_step_batch64<FL, TH, D, NT, decltype(g)::value, decltype(bf)::value>), grid,

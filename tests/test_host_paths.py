@@ -237,3 +237,20 @@ for n, two in ((3, True), (16, False)):
     step_batch(lats + [wide], 8)
     assert launches(b"k_step2_batch64") == 4 and launches(b"k_step_batch64") == (0 if two else 8)
 """)
+
+
+# FP64 single steps beyond the cached sizes go in groups of blocks with
+# non-temporal stores (fifth template argument), below them with plain ones.
+def test_fp64_streamed_single_steps_use_streaming_stores(run):
+    run("""
+for n, streamed in ((64, 0), (100, 1), (112, 1)):
+    cfg = configs.hit(n, les=False) if n == 112 else workloads.rb2d(n, n, n, precision=abi.FP64)
+    lat = started(cfg)
+    lat.set_fusion(False)
+    S.stub_reset()
+    lat.step(2)
+    t = 0 if n == 112 else 1
+    dense = 1 if n % 64 else 0
+    assert launches(f"k_step_fp64ILb0ELb1ELb{t}ELb{dense}ELb{streamed}E".encode()) == launches() == 2
+    lat.close()
+""")
