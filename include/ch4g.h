@@ -392,9 +392,10 @@ int ch4g_particles_count(ch4g_lattice *lat, int64_t *n);
 
 /* Read back the particles in the reference's array order (output_particles,
  * lagrange.c:1598; write_point_particle_h5 payload).  At most `cap` records;
- * *n receives the live count.  Synchronous.  The first call allocates up to 42
- * MB and 16 bytes a particle on the device, which the lattice keeps; without
- * room for that the rows are read back one at a time.                       */
+ * *n receives the live count.  Synchronous.  For more than a few particles the
+ * first call allocates up to 42 MB and 16 bytes a particle on the device,
+ * which the lattice keeps; without room for that the records are formed on
+ * the host.                                                                 */
 int ch4g_get_particles(ch4g_lattice *lat, ch4g_particle *out, int64_t cap, int64_t *n);
 
 /* Replace the particle state (read_point_particle_h5 restart,

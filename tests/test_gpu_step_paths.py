@@ -333,3 +333,9 @@ def test_fp64_batched_single_steps(kind):
             assert np.isfinite(a.get_populations()[0]).all()
     for lat in many + one:
         lat.close()
+
+
+# Records of few particles (formed on the host), some dropped, rows in cell order.
+@pytest.mark.parametrize("n,dead", [(100, [0, 7, 99]), (128, []), (129, [128])], ids=str)
+def test_few_particle_records(n, dead):
+    test_particle_records_in_chunks(n, dead)

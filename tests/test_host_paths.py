@@ -254,3 +254,21 @@ for n, streamed in ((64, 0), (100, 1), (112, 1)):
     assert launches(f"k_step_fp64ILb0ELb1ELb{t}ELb{dense}ELb{streamed}E".encode()) == launches() == 2
     lat.close()
 """)
+
+
+# A few particles are read back without kernels or device buffers.
+@pytest.mark.parametrize("n,kernels", [(1, False), (128, False), (129, True)])
+def test_few_particle_records_are_formed_on_the_host(run, n, kernels):
+    run(f"""
+lat = started(configs.poiseuille(8, 8, 8, tau=0.8, g=0.0), 0)
+lat.particles_init(abi.make_particle_config(abi.LAGRANGE_WRAP, 1))
+a = np.zeros({n}, dtype=abi.particle_dtype())
+for i, k in enumerate(a.dtype.names):
+    a[k] = 1000.0 * i + np.arange({n})
+lat.set_particles(a)
+S.stub_reset()
+live = S.stub_live_bytes()
+back = lat.particles()
+assert (launches() > 0) == {kernels} and (S.stub_live_bytes() > live) == {kernels}
+assert {kernels} or np.array_equal(back, a)
+""")
