@@ -1010,7 +1010,7 @@ int ch4g_particles_count(ch4g_lattice *L, int64_t *n)
 
 namespace {
 
-constexpr int64_t RECORDS_ON_HOST = 128;
+constexpr int64_t RECORDS_ON_HOST = 600;
 
 // ch4g_get_particles without device memory of its own: the state read back, as
 // many rows at a time as 16 MB hold.
@@ -1018,7 +1018,16 @@ int records_on_host(ch4g_lattice *L, ch4g_particle *out, int64_t cap, int64_t *n
 {
     Particles *Q = L->part;
     const size_t np = (size_t)Q->np;
+    const int64_t ld = Q->cap, fit = ((int64_t)16 << 20) / (ld * (int64_t)sizeof(double));
+    const int most = (int)(fit < 1 ? 1 : (fit > PF_COUNT ? PF_COUNT : fit));
+    std::vector<double> v((size_t)(most * ld));
+    auto rows_from = [&](int r) {
+        const int k = r + most < PF_COUNT ? most : PF_COUNT - r;
+        return hipMemcpyAsync(v.data(), Q->d_state + r * ld, (size_t)(k * ld) * sizeof(double), hipMemcpyDeviceToHost,
+                              L->stream);
+    };
     std::vector<int> alive(np), orig(np);
+    HIPCHK(rows_from(0));
     HIPCHK(hipMemcpyAsync(alive.data(), Q->d_alive, np * sizeof(int), hipMemcpyDeviceToHost, L->stream));
     HIPCHK(hipMemcpyAsync(orig.data(), Q->d_orig, np * sizeof(int), hipMemcpyDeviceToHost, L->stream));
     HIPCHK(hipStreamSynchronize(L->stream));
@@ -1029,19 +1038,23 @@ int records_on_host(ch4g_lattice *L, ch4g_particle *out, int64_t cap, int64_t *n
     for (int64_t p : row_of)
         if (alive[(size_t)p]) place[(size_t)p] = live++;
     constexpr RecordRows rows;
-    const int64_t ld = Q->cap, fit = ((int64_t)16 << 20) / (ld * (int64_t)sizeof(double));
-    const int most = (int)(fit < 1 ? 1 : (fit > PF_COUNT ? PF_COUNT : fit));
-    std::vector<double> v((size_t)(most * ld));
     for (int r = 0; r < PF_COUNT; r += most) {
-        const int k = r + most < PF_COUNT ? most : PF_COUNT - r;
-        HIPCHK(hipMemcpyAsync(v.data(), Q->d_state + r * ld, (size_t)(k * ld) * sizeof(double), hipMemcpyDeviceToHost,
-                              L->stream));
-        HIPCHK(hipStreamSynchronize(L->stream));
+        if (r > 0) {
+            HIPCHK(rows_from(r));
+            HIPCHK(hipStreamSynchronize(L->stream));
+        }
+        // the members these rows hold
+        int member[NREC], n_member = 0;
+        int64_t at[NREC];
         for (int f = 0; f < NREC; f++) {
-            if (rows.row[f] < r || rows.row[f] >= r + k) continue;
-            const double *row = v.data() + (rows.row[f] - r) * ld;
-            for (size_t p = 0; p < np; p++)
-                if (place[p] >= 0 && place[p] < cap) (&out[place[p]].name)[f] = row[p];
+            if (rows.row[f] < r || rows.row[f] >= r + most) continue;
+            member[n_member] = f;
+            at[n_member++] = (rows.row[f] - r) * ld;
+        }
+        for (size_t p = 0; p < np; p++) {
+            if (place[p] < 0 || place[p] >= cap) continue;
+            double *record = &out[place[p]].name;
+            for (int m = 0; m < n_member; m++) record[member[m]] = v[(size_t)at[m] + p];
         }
     }
     *n = live;
@@ -1060,7 +1073,7 @@ int ch4g_get_particles(ch4g_lattice *L, ch4g_particle *out, int64_t cap, int64_t
     // be in cell order) and copied straight to the caller: reading all rows
     // back and forming them on the host took 220 ms for 500,000 particles.  For
     // few, the kernels' launches cost more than the rows (us a call, host and
-    // device: 1 particle 72 91, 100 104 117, 5000 612 299)
+    // device: 1 particle 72 91, 100 104 117; 1100 104 88, 5000 537 235)
     if (Q->np <= RECORDS_ON_HOST) return records_on_host(L, out, cap, n);
     const int64_t np = Q->np, c = Q->cap;
     if (!Q->d_records) {

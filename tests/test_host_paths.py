@@ -257,7 +257,7 @@ for n, streamed in ((64, 0), (100, 1), (112, 1)):
 
 
 # A few particles are read back without kernels or device buffers.
-@pytest.mark.parametrize("n,kernels", [(1, False), (128, False), (129, True)])
+@pytest.mark.parametrize("n,kernels", [(1, False), (600, False), (601, True)])
 def test_few_particle_records_are_formed_on_the_host(run, n, kernels):
     run(f"""
 lat = started(configs.poiseuille(8, 8, 8, tau=0.8, g=0.0), 0)
