@@ -111,22 +111,26 @@ constexpr int RED_THREADS = 256, RED_WAVES = RED_THREADS / 64;
 constexpr int NTERM = 25;  // ch4g_output without lb, which is formed from the sums
 
 // work of one block: unit = (z plane, part of it); a part is RED_WAVES waves,
-// each 64 x of `rows` consecutive rows
+// each lx x of 64 / lx groups of `rows` consecutive rows (lx: 64 or, for
+// narrower lattices, the power of two that holds a row)
 struct PlaneWork {
-    int nxt, rows, parts;
+    int lx, nxt, rows, parts;
     int64_t units;
 };
 
 static PlaneWork plane_work(const KParams &P)
 {
     PlaneWork w;
-    w.nxt = (P.NX + 63) / 64;
-    // rows per wave: up to 16 (the two rows next to a march are read again),
+    w.lx = 64;
+    while (w.lx / 2 >= P.NX) w.lx /= 2;
+    w.nxt = (P.NX + w.lx - 1) / w.lx;
+    const int groups = 64 / w.lx;
+    // rows per lane: up to 16 (the two rows next to a march are read again),
     // fewer where that would leave less than 4 waves per SIMD
-    const int64_t waves = (int64_t)w.nxt * P.NY * P.NZ;
+    const int64_t waves = (int64_t)w.nxt * ((P.NY + groups - 1) / groups) * P.NZ;
     const int64_t r = waves / 4096;
     w.rows = (int)(r < 1 ? 1 : (r > 16 ? 16 : r));
-    const int64_t tasks = (int64_t)w.nxt * ((P.NY + w.rows - 1) / w.rows);
+    const int64_t tasks = (int64_t)w.nxt * ((P.NY + groups * w.rows - 1) / (groups * w.rows));
     w.parts = (int)((tasks + RED_WAVES - 1) / RED_WAVES);
     w.units = (int64_t)w.parts * P.NZ;
     return w;
@@ -251,7 +255,8 @@ __global__ void __launch_bounds__(RED_THREADS) k_plane_sums(KParams P, Fields F,
     const uint32_t first = xcd_block(blockIdx.x, gridDim.x);
     for (int64_t unit = first; unit < w.units; unit += gridDim.x) {
         const int z = (int)(unit / w.parts), task = (int)(unit - (int64_t)z * w.parts) * RED_WAVES + wave;
-        const int x = task % w.nxt * 64 + lane, y0 = task / w.nxt * w.rows, y1 = min(y0 + w.rows, NY);
+        const int x = task % w.nxt * w.lx + lane % w.lx;
+        const int y0 = (task / w.nxt * (64 / w.lx) + lane / w.lx) * w.rows, y1 = min(y0 + w.rows, NY);
         if (x < NX && y0 < NY) {
             const int64_t plane = (int64_t)z * NY * NX;
             const int64_t dzp = (int64_t)(wrapc(z + 1, NZ) - z) * NY * NX, dzm = (int64_t)(wrapc(z - 1, NZ) - z) * NY * NX;

@@ -336,6 +336,14 @@ def test_fp64_batched_single_steps(kind):
 
 
 # Records of few particles (formed on the host), some dropped, rows in cell order.
-@pytest.mark.parametrize("n,dead", [(100, [0, 7, 99]), (128, []), (129, [128])], ids=str)
+@pytest.mark.parametrize("n,dead", [(100, [0, 7, 99]), (600, []), (601, [600])], ids=str)
 def test_few_particle_records(n, dead):
     test_particle_records_in_chunks(n, dead)
+
+
+# The same for lattices narrower than a wave, several groups of rows in one:
+# every power of two and its neighbours, with a partial last group.
+@pytest.mark.parametrize("shape", [(1, 3, 1), (1, 200, 130), (2, 131, 3), (5, 70, 33), (8, 67, 9), (17, 37, 5),
+                                   (32, 9, 4), (33, 10, 4)], ids=str)
+def test_diagnostics_of_narrow_lattices(shape):
+    test_diagnostics_at_partial_waves(shape)
