@@ -116,7 +116,7 @@ struct ch4g_lattice {
     // captured GRAPH_STEPS-step sequences, one per starting buffer and
     // temperature-lag buffer (index cur | tpar << 1)
     hipGraphExec_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
-    // two-step launches (2-D FP32 storage) write the lag into a second array;
+    // two-step launches write the lag into a second array;
     // tlag stays the current one, tpar counts the swaps mod 2
     void *tlag_alt = nullptr;
     int tpar = 0;

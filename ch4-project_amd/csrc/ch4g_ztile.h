@@ -7,23 +7,23 @@
 namespace ch4g {
 
 // Two steps per launch for 3-D lattices (NZ > 1), marching along z.  A block
-// owns a 64 x TY column of x-y tiles over a range of z planes and has one
+// owns a TX x TY column of x-y tiles over a range of zc planes and has one
 // thread per node of the tile with its one-node x-y halo.  Iteration j:
 //   A  step 1 at plane j for the tile + halo nodes (gather from the global
-//      state, collide into registers); the populations with c_z = -1 go to
-//      the LDS ring M;
+//      state, collision); the populations with c_z = -1 go to the LDS ring M;
 //   B  step 2 at plane j - 1 for the tile nodes, gathering from LDS: c_z = +1
 //      from plane j - 2 (ring P), c_z = 0 from plane j - 1 (ring Z), c_z = -1
-//      from plane j (ring M); collide into the global output;
-//   C  the registers of step A go to ring Z (c_z = 0 and the step-1
-//      temperature lag) and ring P (c_z = +1, two slots by plane parity);
-//      the tile nodes also keep their populations 16 and 18 (c_z = -1) in
-//      ring W, which the wall rules of step B read at the node itself one
-//      plane later (fluid bounce-back at y = 0 takes f_16, f_18 there, the
-//      fixed-T rule at y = NY - 1 takes g_16, g_18).
-// Planes just below and above the block's range are computed in step A
-// (z-halo) but not written.  Per two steps the state is read (1 + 2/ZC)
-// times over the tile + halo area (x-y halo: 396 / 256 nodes for TY = 4) and
+//      from plane j (ring M); collision into the global output;
+//   C  (HOLD) the registers of step A go to ring Z (c_z = 0 and the step-1
+//      temperature, the lag of step 2) and ring P (c_z = +1, two slots by
+//      plane parity); without HOLD step A writes them at once into the slots
+//      step B does not read.
+// The tile nodes also keep their populations 16 and 18 (c_z = -1) in ring W,
+// which the wall rules of step B read at the node itself one plane later
+// (fluid bounce-back at y = 0 takes f_16, f_18 there, the fixed-T rule at
+// y = NY - 1 takes g_16, g_18).  Planes just below and above the block's range
+// are computed in step A (z halo) but not written.  Per two steps the state is
+// read (1 + 2/zc) times over the tile + halo area (M/T of the tile) and
 // written once; the temperature lag is read from tl_in and written to tl_out
 // (halo nodes of one block are tile nodes of another).
 namespace z2 {

@@ -843,24 +843,7 @@ __device__ __forceinline__ void finish_raw(const KParams &P, const Row &R, const
     }
 }
 
-// Two steps per launch for 3-D lattices (NZ > 1), marching along z.  A block
-// owns a TX x TY column of x-y tiles over a range of zc planes and has one
-// thread per node of the tile with its one-node x-y halo.  Iteration j:
-//   A  step 1 at plane j for the tile + halo nodes (gather from the global
-//      state, collision);
-//   B  step 2 at plane j - 1 for the tile nodes, gathering from LDS: c_z = +1
-//      from plane j - 2 (ring P), c_z = 0 from plane j - 1 (ring Z), c_z = -1
-//      from plane j (ring M); collision into the global output.
-// Ring Z also holds the step-1 temperature (the lag of step 2); ring W keeps
-// the tile nodes' populations 16 and 18 (c_z = -1), which the wall rules of
-// step B read at the node itself one plane later (fluid bounce-back at y = 0
-// takes f_16, f_18 there... see ring_src).  With HOLD the c_z >= 0 results of
-// step A wait in registers and go to the rings after step B (C); without it
-// step A writes them at once into the slots step B does not read.  The planes
-// just below and above the block's range are computed in step A (z halo) but
-// not written.  Per two steps the state is read (1 + 2/zc) x M/T times and
-// written once; the temperature lag is read from tl_in and written to tl_out
-// (halo nodes of one block are tile nodes of another).
+// Two steps per launch for 3-D lattices, marching along z (ch4g_ztile.h).
 template <bool FLUID, bool THERMAL, typename A, bool NTS, class TZ>
 __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp32(KParams P, const float *__restrict__ fin,
                                                              const float *__restrict__ gin, float *__restrict__ fout,
@@ -1291,7 +1274,12 @@ static int64_t z_columns(const KParams &P)
 // against 37) and 100^3 (58.6 against 61.4) single.  Channel 113^3 34.1 -> 31.7,
 // 125^3 49 -> 45, 185^3 176 -> 150; 96^3 (21.9 against 22.7) single; channels
 // whose rows fill less than 85 % of their tiles stay single (160^3 117 against
-// 105).
+// 105).  The first line holds for float arithmetic but in channels of two planes,
+// and not for thin lattices in double arithmetic, whose launches are mostly z halo:
+// single -> marching, float Rayleigh-Benard 1024x1024x2 125 -> 115, 1024x512x4 118
+// -> 99, channel 1024x1024x2 57 -> 62, x3 89 -> 82; double Rayleigh-Benard
+// 1024x1024x2 126 -> 164, x8 489 -> 511, 256x256x32 123 -> 117, channel
+// 1024x1024x2 56 -> 70, x4 119 -> 113.
 static bool z_marching_pays(const KParams &P)
 {
     const int64_t tiles_x = (P.NX + 63) / 64, fill = (int64_t)P.NX * 100 / (64 * tiles_x);

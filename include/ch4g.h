@@ -409,10 +409,10 @@ int ch4g_set_particles(ch4g_lattice *lat, const ch4g_particle *in, int64_t n);
  * (the reference runs one job per MPI launch, main.c); these entry points
  * are for hosts that run ensembles of the reference's jobs.                 */
 
-/* Advance n lattices by nsteps steps together: one kernel launch per step
- * (per storage/population variant) covers every lattice through a table of
- * 256-node tiles.  Each lattice's fields are bit-identical to ch4g_step on
- * it alone.  Lattices must be past their first step (ch4g_step(lat, 1)),
+/* Advance n lattices by nsteps steps together: one kernel launch per step or
+ * two steps (per storage/population variant) covers every lattice through a
+ * table of tiles, large 3-D lattices run their own launches beside them.
+ * Each lattice's fields are bit-identical to ch4g_step on it alone.  Lattices must be past their first step (ch4g_step(lat, 1)),
  * without HIT forcing or particles, on the current device.                  */
 int ch4g_step_batch(ch4g_lattice *const *lats, int n, int nsteps);
 
