@@ -520,7 +520,8 @@ struct RegOut64 {
 // steps.
 //
 // A single step moves the state at 5 TB/s and is bound by that; here it is
-// read (with the tile's halo, 1.33 times) and written once per two steps.  us
+// read (with the tile's halo 1.33 times, 1.07 from memory as the L2s share halo
+// lines) and written once per two steps.  us
 // per step, single -> this: Rayleigh-Benard 96^3 112 -> 81, 128^3 249 -> 186,
 // 185^3 752 -> 589, 256^3 1996 -> 1492, 96x80x112 111 -> 83; channel 113^3
 // 91 -> 72, 128^3 120 -> 86, 192^3 413 -> 280.  An iteration (11.6 us at 256^3)
@@ -650,7 +651,7 @@ __global__ void __launch_bounds__(TZ::THREADS) k_step2z_fp64(KParams P, const do
 // into LDS, one node per thread, the second from there into the global state.
 //
 // Small lattices pay one launch's ramp and drain, large ones one read (1.6
-// times, with the halo) and write of the state, for two steps.  32 x 4 tiles:
+// times, with the halo; 1.1 from memory) and write of the state, for two steps.  32 x 4 tiles:
 // two blocks of 64 KB of LDS on a CU, so one's loads overlap the other's
 // collisions.  us per step, single -> this: Rayleigh-Benard 64x32 3.92 -> 3.56,
 // 256x128 6.1 -> 4.2, 512x256 12.5 -> 10.6, 969x487 58.7 -> 39.2, 1024x512 67
