@@ -105,7 +105,9 @@ void launch_load(const KParams &P, const double *fs, const double *gs, void *f, 
 // whole march.  256^3, us, one node per thread and one LDS tree per term ->
 // this: averages 630 -> 280 (0.67 GB of fields), final sum 616 -> 8; rulers,
 // one block per plane before, x 3480, y 744, z 660 -> 670 together.  Small
-// lattices: 32 -> 10 for the averages.
+// lattices: 32 -> 10 for the averages.  Lattices narrower than a wave put several
+// rows into one for the plane sums (us an averages call, one row a wave -> this:
+// 1x1000x1000 1950 -> 1330, 8x256x256 170 -> 137, 3x300x21 74 -> 48).
 
 constexpr int RED_THREADS = 256, RED_WAVES = RED_THREADS / 64;
 constexpr int NTERM = 25;  // ch4g_output without lb, which is formed from the sums
